@@ -44,6 +44,60 @@ def test_accumulator_bitwise(N, M, K):
     assert torch.equal(got, ref)
 
 
+def _fast(a8, w):
+    """(N, M) accumulator from the kernel; w (M, K) float."""
+    return fast_accum_mm(a8.to(DEV), w.t().contiguous().to(torch.bfloat16).to(DEV)).cpu()
+
+
+@pytest.mark.parametrize("N,M", [(4, 63), (15, 64), (16, 65), (17, 127), (63, 1), (65, 129)])
+def test_accumulator_tile_edges(N, M):
+    """Rows and columns around the kernel's tiles (4 and 16 rows a wave, 64 a
+    workgroup, 64 columns), operands over E4M3's whole range in one group,
+    rows and columns of zeros, activation rows off 8-byte alignment."""
+    K = 160
+    g = torch.Generator().manual_seed(N * M)
+    bits = torch.randint(0, 256, (N + M, K + 3), generator=g, dtype=torch.uint8)
+    bits[(bits & 0x7f) == 0x7f] = 3                        # no NaN
+    x = bits.view(E4M3)
+    a8 = x[:N, 3:]                                         # row stride 163, base off by 3
+    w = x[N:, :K].float()
+    w[M // 2] = 0.0
+    w[0] = torch.where(torch.rand(K, generator=g) < 0.9, 0.0, 2.0 ** -9)  # products far below a
+    print(f"fast accum edges N={N} M={M}", flush=True)
+    ad = bits.to(DEV).view(E4M3)[:N, 3:]
+    ad[N // 2] = 0.0
+    ref_a = a8.float()
+    ref_a[N // 2] = 0.0
+    got = fast_accum_mm(ad, w.t().contiguous().to(torch.bfloat16).to(DEV)).cpu()
+    assert torch.equal(got, oracle.fast_accum_mm(ref_a, w))
+
+
+@pytest.mark.parametrize("what", ["deep", "nan", "weight"])
+def test_accumulator_general_arithmetic(what):
+    """Groups that the packed arithmetic does not take: products 14 and more
+    exponents below the row's largest activation, NaN activations, weights
+    that are no E4M3 values (more mantissa bits, larger exponents)."""
+    N, M, K = 20, 70, 128
+    a8 = _e4m3((N, K), 100.0, seed=5, specials=False)
+    w = _e4m3((M, K), 0.05, seed=6).float()
+    if what == "deep":
+        a = a8.float()
+        a[:, ::2] = 2.0 ** -9                              # the only ones with a weight
+        a8 = a.to(E4M3)
+        w[:, 1::2] = 0.0
+        w[:, ::2] = w[:, ::2].sign() * 2.0 ** -9
+    elif what == "nan":
+        a8.view(torch.uint8)[3, 70] = 0x7f
+    else:
+        w[7] *= 1.0 + 2.0 ** -7
+        w[9, 40] = 3.0e4
+    w = w.to(torch.bfloat16).float()
+    print(f"fast accum general {what}", flush=True)
+    got, ref = _fast(a8, w), oracle.fast_accum_mm(a8.float(), w)
+    assert torch.equal(got.isnan(), ref.isnan())
+    assert torch.equal(got.nan_to_num(), ref.nan_to_num())
+
+
 def test_linear_bitwise_and_strided_weight():
     N, M, K = 33, 200, 256
     g = torch.Generator().manual_seed(1)
