@@ -154,6 +154,27 @@ SIGNATURES = {
         _c_p, _c_p, _c_p, _c_p,                   # q, k, vt, out
         _c_i64, _c_i64, _c_i64, _c_i64, _c_f, _c_p,  # N, heads, L, head_dim, scale, stream
     ],
+    "evo2_prefill_attention_rows": [
+        _c_p, _c_p, _c_p, _c_p,                   # q, k, vt, out
+        _c_i64, _c_i64, _c_i64,                   # out strides (n, h, row)
+        _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_f, _c_p,  # N, heads, L, Lv, head_dim, scale, stream
+    ],
+    "evo2_rotary_prefill": [
+        _c_p, _c_i64, _c_p, _c_f,                 # qkv, sqkv, inv_freq, factor
+        _c_p, _c_p, _c_p, _c_i64,                 # q, k, vt, Lv
+        _c_p, _c_i64, _c_i64, _c_i64,             # key pages + strides (page, h, d)
+        _c_p, _c_i64, _c_i64, _c_i64,             # value pages + strides (page, h, l)
+        _c_i64, _c_p, _c_i64, _c_i64,             # num_pages, table, row stride, columns
+        _c_i64, _c_i64, _c_i64, _c_i64, _c_p,     # N, heads, head_dim, L, stream
+    ],
+    "evo2_rotary_decode": [
+        _c_p, _c_i64, _c_p, _c_f,                 # qkv, sqkv, inv_freq, factor
+        _c_p,                                     # q
+        _c_p, _c_i64, _c_i64, _c_i64,             # key pages + strides (page, h, d)
+        _c_p, _c_i64, _c_i64, _c_i64,             # value pages + strides (page, h, l)
+        _c_i64, _c_p, _c_i64, _c_i64,             # num_pages, table, row stride, columns
+        _c_p, _c_i64, _c_i64, _c_i64, _c_p,       # positions, B, heads, head_dim, stream
+    ],
     "evo2_fp8_quantize": [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_p],
     "evo2_rms_norm": [
         _c_p, _c_i64, _c_p, _c_i64,               # x, sx, residual, sr

@@ -9,9 +9,12 @@ past each sequence's own masked.  Keys and values are each read once (the
 context is split into 2048-position chunks whose partial softmax sums are
 merged by a second launch); the arithmetic is fp32 up to the bf16 output.
 
+Rotary and the page writes are one launch between the qkv projection and the
+attention (csrc/rotary.hip: rotary_prefill, rotary_decode).
+
 Prefill attention (a prompt against itself, causal) runs on the HIP kernel
-in csrc/attention_prefill.hip at head_dim 128 (the values transposed once
-per call; fp32 scores and softmax, bf16 softmax weights in the value
+in csrc/attention_prefill.hip at head_dim 128 (the values transposed, by
+rotary_prefill or once per call; fp32 scores and softmax, bf16 softmax weights in the value
 product); other head dims on torch's fused attention kernels where the
 platform has them for the inputs, else a chunked product with contiguous
 operands and an fp32 softmax.
@@ -184,6 +187,56 @@ class PagedKVCache:
         return kd[..., :L], vd[:, :, :L]
 
 
+def rotary_prefill(qkv, cache, block_table, inv_freq, factor, nseq, L):
+    """Rotary and cache write of nseq prompts of L tokens in one launch: qkv
+    (nseq * L, 3 * heads * 128) bf16 rows (q | k | v).  Writes k and v into
+    `cache`'s pages (block_table (>= nseq, pages) int32) and returns the
+    operands of prefill attention: q, k (nseq, heads, L, 128) rotated, and the
+    values transposed, (nseq, heads, 128, L rounded up to 8), zeros from L on."""
+    _lib.require_device(qkv, cache.k, cache.v, block_table, inv_freq)
+    nh, hd = cache.k.shape[1], cache.k.shape[2]
+    if qkv.shape != (nseq * L, 3 * nh * hd) or qkv.dtype != torch.bfloat16 or qkv.stride(1) != 1:
+        raise ValueError(f"qkv must be ({nseq * L}, {3 * nh * hd}) bf16 rows, got "
+                         f"{tuple(qkv.shape)} {qkv.dtype}")
+    if (block_table.dtype != torch.int32 or block_table.stride(1) != 1
+            or block_table.shape[0] < nseq):
+        raise ValueError("block_table must be (>= nseq, pages) int32 with unit column stride")
+    Lv = -(-L // 8) * 8
+    q = torch.empty(nseq, nh, L, hd, dtype=qkv.dtype, device=qkv.device)
+    k = torch.empty_like(q)
+    vt = torch.empty(nseq, nh, hd, Lv, dtype=qkv.dtype, device=qkv.device)
+    _lib.call("evo2_rotary_prefill", _lib.ptr(qkv), qkv.stride(0), _lib.ptr(inv_freq),
+              float(factor), _lib.ptr(q), _lib.ptr(k), _lib.ptr(vt), Lv,
+              _lib.ptr(cache.k), *cache.k.stride()[:3], _lib.ptr(cache.v), *cache.v.stride()[:3],
+              cache.k.shape[0], _lib.ptr(block_table), block_table.stride(0),
+              block_table.shape[1], nseq, nh, hd, L, _lib.stream_of(qkv))
+    return q, k, vt
+
+
+def rotary_decode(qkv, cache, block_table, positions, inv_freq, factor):
+    """Rotary and cache write of one token per sequence in one launch: qkv
+    (B, 3 * heads * head_dim) bf16 rows (q | k | v) at positions (B,) int64.
+    Writes k and v into `cache`'s pages and returns q (B, heads, head_dim)."""
+    _lib.require_device(qkv, cache.k, cache.v, block_table, positions, inv_freq)
+    nh, hd = cache.k.shape[1], cache.k.shape[2]
+    B = qkv.shape[0]
+    if qkv.shape[1] != 3 * nh * hd or qkv.dtype != torch.bfloat16 or qkv.stride(1) != 1:
+        raise ValueError(f"qkv must be (B, {3 * nh * hd}) bf16 rows, got {tuple(qkv.shape)} "
+                         f"{qkv.dtype}")
+    if block_table.dtype != torch.int32 or block_table.stride(1) != 1 or block_table.shape[0] < B:
+        raise ValueError("block_table must be (>= B, pages) int32 with unit column stride")
+    if positions.shape != (B,):
+        raise ValueError(f"positions must be ({B},), got {tuple(positions.shape)}")
+    positions = positions.to(torch.int64).contiguous()
+    q = torch.empty(B, nh, hd, dtype=qkv.dtype, device=qkv.device)
+    _lib.call("evo2_rotary_decode", _lib.ptr(qkv), qkv.stride(0), _lib.ptr(inv_freq),
+              float(factor), _lib.ptr(q),
+              _lib.ptr(cache.k), *cache.k.stride()[:3], _lib.ptr(cache.v), *cache.v.stride()[:3],
+              cache.k.shape[0], _lib.ptr(block_table), block_table.stride(0),
+              block_table.shape[1], _lib.ptr(positions), B, nh, hd, _lib.stream_of(qkv))
+    return q
+
+
 _FUSED_SDPA = None  # whether torch's fused attention kernels take these inputs here
 
 
@@ -218,13 +271,22 @@ def prefill_attention(q, k, v, scale):
         raise ValueError(f"prefill_attention takes head_dim 128 and L a multiple of 8, got {hd}, {L}")
     if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
         raise ValueError("prefill_attention takes bf16 q, k, v")
-    q = q.contiguous()
-    k = k.contiguous()
-    vt = v.transpose(-1, -2).contiguous()
-    out = torch.empty_like(q)
-    _lib.call("evo2_prefill_attention", _lib.ptr(q), _lib.ptr(k), _lib.ptr(vt), _lib.ptr(out),
-              N, nh, L, hd, float(scale), _lib.stream_of(q))
+    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    prefill_attention_rows(q.contiguous(), k.contiguous(), v.transpose(-1, -2).contiguous(), scale,
+                           out)
     return out
+
+
+def prefill_attention_rows(q, k, vt, scale, out):
+    """The kernel of prefill_attention for any L: q, k (N, heads, L, 128)
+    contiguous, vt (N, heads, 128, Lv) contiguous with Lv >= L a multiple of 8
+    and finite from L on; the result goes to `out` (N, heads, L, 128), a view
+    of any strides with unit last one."""
+    _lib.require_device(q, k, vt, out)
+    N, nh, L, hd = q.shape
+    _lib.call("evo2_prefill_attention_rows", _lib.ptr(q), _lib.ptr(k), _lib.ptr(vt), _lib.ptr(out),
+              out.stride(0), out.stride(1), out.stride(2), N, nh, L, vt.shape[3], hd, float(scale),
+              _lib.stream_of(q))
 
 
 def causal_prefill_attention(q, k, v, scale):
@@ -251,4 +313,5 @@ def causal_prefill_attention(q, k, v, scale):
 
 
 __all__ = ["decode_attention", "workspace", "paged_decode_attention", "check_block_table",
-           "PagedKVCache", "causal_prefill_attention", "prefill_attention", "PAGE"]
+           "PagedKVCache", "causal_prefill_attention", "prefill_attention",
+           "prefill_attention_rows", "rotary_prefill", "rotary_decode", "PAGE"]

@@ -2,10 +2,11 @@
 // cores (head_dim 128): out[i] = sum_{j <= i} softmax_j(scale q_i . k_j) v_j
 // per (sequence, head), as Evo2Attention computes it at prefill
 // (model.py:104-153; the reference leaves the kernel to vLLM's flash
-// attention).  Inputs in the harness's layouts: q, k and out (N, heads, L,
-// 128) and the values transposed, vt (N, heads, 128, L), so that both
-// products read 16 contiguous bytes per lane and no operand is transposed in
-// registers.
+// attention).  Inputs in the harness's layouts: q and k (N, heads, L, 128) and
+// the values transposed, vt (N, heads, 128, Lv), Lv >= L a multiple of 8 with
+// finite padding, so that both products read 16 contiguous bytes per lane and
+// no operand is transposed in registers.  The output's rows go to any strides:
+// token-major (N, L, heads, 128) is what the output projection reads.
 //
 // A workgroup takes 256 queries of one (sequence, head): eight waves of 32
 // (two 16-query tiles, two waves a SIMD; the workgroups of one XCD take whole
@@ -48,8 +49,10 @@ constexpr float AP_SLACK = 8.0f;           // log2 headroom of the reference max
 struct PrefillArgs {
   const bf16_t *q, *k, *vt;
   bf16_t *out;
-  int64_t plane;   // elements per (sequence, head) plane: L * 128
+  int64_t on, oh, ol;  // output strides: sequence, head, query
+  int64_t plane;   // elements per (sequence, head) plane of q and k: L * 128
   int L;
+  int Lv;          // row stride of the transposed values
   int heads;
   int nqb;         // query blocks per plane
   float c2;        // scale * log2(e)
@@ -73,8 +76,9 @@ __global__ __launch_bounds__(AP_NW * 64, 1) void attn_prefill_kernel(PrefillArgs
     h = static_cast<int>(blockIdx.y);
   }
   const int64_t pl = static_cast<int64_t>(blockIdx.z) * p.heads + h;
-  const bf16_t *q = p.q + pl * p.plane, *k = p.k + pl * p.plane, *vt = p.vt + pl * p.plane;
-  bf16_t *out = p.out + pl * p.plane;
+  const bf16_t *q = p.q + pl * p.plane, *k = p.k + pl * p.plane;
+  const bf16_t *vt = p.vt + pl * AP_HD * p.Lv;
+  bf16_t *out = p.out + static_cast<int64_t>(blockIdx.z) * p.on + h * p.oh;
   const int L = p.L;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -91,22 +95,23 @@ __global__ __launch_bounds__(AP_NW * 64, 1) void attn_prefill_kernel(PrefillArgs
   // (i % 16) ^ ((r >> 3) & 15), keys kb0 + 8 c .., of dim row r (values).
   // Buffer loads over the (sequence, head) plane: a lane's offset within the
   // block is fixed, the block's in an SGPR; key rows past the prompt read
-  // zeros (past the plane), value chunks past it the next row's first keys
-  // or zeros, finite values whose probabilities are 0.
+  // zeros (past the plane), value chunks past it the padding, the next row's
+  // first keys or zeros, finite values whose probabilities are 0.
   const uint32_t pbytes = static_cast<uint32_t>(p.plane * 2);
+  const uint32_t vbytes = static_cast<uint32_t>(p.Lv) * (AP_HD * 2u);
   const __amdgpu_buffer_rsrc_t krs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(k), 0, pbytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t vrs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(vt), 0, pbytes, 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(vt), 0, vbytes, 0x00020000);
   uint32_t koff[32 / AP_NW], voff[32 / AP_NW];
 #pragma unroll
   for (int jj = 0; jj < 32 / AP_NW; ++jj) {
     const int j = (32 / AP_NW) * wave + jj;
     const int r = 4 * j + (lane >> 4);
-    // byte offsets below 256 L < 2^32 (checked on the host), in 32 bits unsigned
+    // byte offsets below 256 Lv < 2^32 (checked on the host), in 32 bits unsigned
     koff[jj] = (static_cast<uint32_t>(r) * AP_HD + 8u * ((lane & 15) ^ ((r >> 2) & 15))) * 2u;
     voff[jj] =
-        (static_cast<uint32_t>(r) * static_cast<uint32_t>(L) + 8u * ((lane & 15) ^ ((r >> 3) & 15))) * 2u;
+        (static_cast<uint32_t>(r) * static_cast<uint32_t>(p.Lv) + 8u * ((lane & 15) ^ ((r >> 3) & 15))) * 2u;
   }
   auto issue = [&](int b) __attribute__((always_inline)) {
     const int kb0 = b * AP_KB;
@@ -270,7 +275,7 @@ __global__ __launch_bounds__(AP_NW * 64, 1) void attn_prefill_kernel(PrefillArgs
     const int qi = wq0 + 16 * nt + n;
     if (qi >= L) continue;
     const float inv = 1.0f / l;  // every query attends to itself: l >= 1
-    bf16_t *orow = out + static_cast<int64_t>(qi) * AP_HD + 32 * g;
+    bf16_t *orow = out + qi * p.ol + 32 * g;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       uint4 w;
@@ -287,27 +292,29 @@ __global__ __launch_bounds__(AP_NW * 64, 1) void attn_prefill_kernel(PrefillArgs
 
 using namespace evo2;
 
-extern "C" int evo2_prefill_attention(const void *q, const void *k, const void *vt, void *out, int64_t N,
-                                      int64_t heads, int64_t L, int64_t head_dim, float scale,
-                                      void *stream) {
-  // a (sequence, head) plane of 256 L bytes is addressed by 32-bit buffer offsets
-  if (N < 0 || heads <= 0 || L < 0 || N > 65535 || heads > 65535 || L * 256 > int64_t(0xffffffff))
-    return fail(EVO2_ERR_INVALID, "prefill_attention: bad sizes N=%lld heads=%lld L=%lld", (long long)N,
-                (long long)heads, (long long)L);
+extern "C" int evo2_prefill_attention_rows(const void *q, const void *k, const void *vt, void *out,
+                                           int64_t on, int64_t oh, int64_t ol, int64_t N,
+                                           int64_t heads, int64_t L, int64_t Lv, int64_t head_dim,
+                                           float scale, void *stream) {
+  // a (sequence, head) plane of 256 Lv bytes is addressed by 32-bit buffer offsets
+  if (N < 0 || heads <= 0 || L < 0 || Lv < L || N > 65535 || heads > 65535 || Lv * 256 > int64_t(0xffffffff))
+    return fail(EVO2_ERR_INVALID, "prefill_attention: bad sizes N=%lld heads=%lld L=%lld Lv=%lld",
+                (long long)N, (long long)heads, (long long)L, (long long)Lv);
   if (head_dim != AP_HD)
     return fail(EVO2_ERR_UNSUPPORTED, "prefill_attention: head_dim %lld (128 only)", (long long)head_dim);
   if (!(scale > 0.0f))
     return fail(EVO2_ERR_INVALID, "prefill_attention: scale %g (must be positive)", (double)scale);
   if (N == 0 || L == 0) return EVO2_OK;
   if (!q || !k || !vt || !out) return fail(EVO2_ERR_INVALID, "prefill_attention: null pointer argument");
-  // 16-byte loads of eight values along L in the transposed values
-  if (L % 8 || reinterpret_cast<uintptr_t>(q) % 16 || reinterpret_cast<uintptr_t>(k) % 16 ||
-      reinterpret_cast<uintptr_t>(vt) % 16 || reinterpret_cast<uintptr_t>(out) % 16)
+  // 16-byte loads of eight values along Lv in the transposed values, 16-byte stores
+  if (Lv % 8 || on % 8 || oh % 8 || ol % 8 || reinterpret_cast<uintptr_t>(q) % 16 ||
+      reinterpret_cast<uintptr_t>(k) % 16 || reinterpret_cast<uintptr_t>(vt) % 16 ||
+      reinterpret_cast<uintptr_t>(out) % 16)
     return fail(EVO2_ERR_UNSUPPORTED, "prefill_attention: L %% 8 or 16-byte alignment not met (L=%lld)",
-                (long long)L);
+                (long long)Lv);
   PrefillArgs a{static_cast<const bf16_t *>(q), static_cast<const bf16_t *>(k), static_cast<const bf16_t *>(vt),
-                static_cast<bf16_t *>(out), L * AP_HD, static_cast<int>(L), static_cast<int>(heads),
-                static_cast<int>(cdiv(L, AP_QB)), scale * 1.4426950408889634f, 0};
+                static_cast<bf16_t *>(out), on, oh, ol, L * AP_HD, static_cast<int>(L), static_cast<int>(Lv),
+                static_cast<int>(heads), static_cast<int>(cdiv(L, AP_QB)), scale * 1.4426950408889634f, 0};
   // whole heads per XCD where the heads split evenly over the eight (32
   // heads x 32768: 9.96 -> 8.34 ms, 8192: 1.05 -> 0.70 ms, the same bits)
   a.xcd_heads = heads % 8 == 0 && static_cast<int64_t>(a.nqb) * heads <= 0x7fffffff;
@@ -319,4 +326,11 @@ extern "C" int evo2_prefill_attention(const void *q, const void *k, const void *
                        dim3(static_cast<unsigned>(a.nqb), static_cast<unsigned>(heads), static_cast<unsigned>(N)),
                        dim3(AP_NW * 64), 0, static_cast<hipStream_t>(stream), a);
   return check_launch("prefill_attention");
+}
+
+extern "C" int evo2_prefill_attention(const void *q, const void *k, const void *vt, void *out, int64_t N,
+                                      int64_t heads, int64_t L, int64_t head_dim, float scale,
+                                      void *stream) {
+  return evo2_prefill_attention_rows(q, k, vt, out, heads * L * AP_HD, L * AP_HD, AP_HD, N, heads, L, L,
+                                     head_dim, scale, stream);
 }

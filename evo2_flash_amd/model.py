@@ -29,8 +29,8 @@ import torch
 from torch import nn
 
 from .attention import (PAGE, PagedKVCache, causal_prefill_attention, check_block_table,
-                        paged_decode_attention, shared_prefix_pages,
-                        workspace as attention_workspace)
+                        paged_decode_attention, prefill_attention_rows, rotary_decode,
+                        rotary_prefill, shared_prefix_pages, workspace as attention_workspace)
 from .metadata import build_metadata
 from .mixers import Linear, load_mixer_params, make_mixer, set_forward_context
 from .norm import Evo2RMSNorm
@@ -98,9 +98,10 @@ class Evo2Attention(nn.Module):
     def forward_decode(self, x, positions, block_table):
         """x (B, H): one token per sequence at `positions` (B,)."""
         B = x.shape[0]
-        q, k, v = self._qkv(x, positions)
-        self.cache.append(k, v.contiguous(), block_table, positions)
-        out = paged_decode_attention(q.contiguous(), self.cache.k, self.cache.v, block_table,
+        qkv, _ = self.qkv_proj(x)
+        q = rotary_decode(qkv, self.cache, block_table, positions, self.inv_freq,
+                          self.rope_factor)
+        out = paged_decode_attention(q, self.cache.k, self.cache.v, block_table,
                                      positions, self.hd ** -0.5, self._attn_ws,
                                      shared_pages=self.shared_pages)  # (B, nh, hd)
         o, _ = self.o_proj(out.reshape(B, self.heads * self.hd))
@@ -109,6 +110,15 @@ class Evo2Attention(nn.Module):
     def forward_prefill(self, x, nseq, L, block_table):
         """x (nseq * L, H): prompts of L tokens (positions 0..L-1) of sequences
         0..nseq-1 of `block_table`, packed in order."""
+        if x.is_cuda and self.hd == 128 and not (torch.is_grad_enabled() and x.requires_grad):
+            qkv, _ = self.qkv_proj(x)
+            q, k, vt = rotary_prefill(qkv, self.cache, block_table, self.inv_freq,
+                                      self.rope_factor, nseq, L)
+            out = torch.empty(nseq, L, self.heads, self.hd, dtype=x.dtype, device=x.device)
+            prefill_attention_rows(q, k, vt, self.hd ** -0.5, out.transpose(1, 2))
+            o, _ = self.o_proj(out.view(nseq * L, self.heads * self.hd))
+            return o
+        # other head dims, the CPU, and a differentiated input
         pos = torch.arange(L, device=x.device).repeat(nseq)
         q, k, v = self._qkv(x, pos)
         shape = (nseq, L, self.heads, self.hd)

@@ -373,6 +373,48 @@ int evo2_prefill_attention(const void *q, const void *k, const void *vt, void *o
                            int64_t heads, int64_t L, int64_t head_dim, float scale, void *stream);
 
 /*
+ * evo2_prefill_attention with padded values and any output strides:
+ *   vt  (N, heads, head_dim, Lv) bf16, Lv >= L a multiple of 8 with
+ *       256 Lv < 2^32, finite from L on;
+ *   out at out + n on + h oh + i ol (elements, multiples of 8), any L.
+ */
+int evo2_prefill_attention_rows(const void *q, const void *k, const void *vt, void *out, int64_t on,
+                                int64_t oh, int64_t ol, int64_t N, int64_t heads, int64_t L, int64_t Lv,
+                                int64_t head_dim, float scale, void *stream);
+
+/*
+ * Neox rotary of q and k with linear position scaling, and the write of k and
+ * v into 16-position KV pages, from rows of a qkv projection (q | k | v, each
+ * heads * head_dim bf16; row stride sqkv):
+ *   angle(t, i) = (t / factor) * inv_freq[i], i < head_dim / 2 (fp32)
+ *   key pages   (pages, heads, head_dim, 16), strides kp0, kp1, kp2
+ *   value pages (pages, heads, 16, head_dim), strides vp0, vp1, vp2
+ *   table       block table, row stride st, max_pages columns: position t of
+ *               sequence n is in page table[n, t / 16]; entries outside
+ *               [0, num_pages) are not written through.
+ * _prefill: rows n L + t, positions t = 0 .. L-1 of N sequences; also writes
+ *   q, k (N, heads, L, head_dim) and vt (N, heads, head_dim, Lv), zeros from L
+ *   on (Lv a multiple of 8, at most the next multiple of 64), the operands of
+ *   evo2_prefill_attention_rows; the last page's tail is zero.  head_dim 128,
+ *   16-byte aligned rows.
+ * _decode: one row a sequence at positions[b]; writes q (B, heads, head_dim).
+ *   Any even head_dim.
+ *
+ * Replaces the rotary embedding and cache writes of Evo2Attention
+ * (evo2_flash/model.py:104-153; vLLM's operators there).
+ */
+int evo2_rotary_prefill(const void *qkv, int64_t sqkv, const float *inv_freq, float factor, void *q,
+                        void *k, void *vt, int64_t Lv, void *k_pages, int64_t kp0, int64_t kp1,
+                        int64_t kp2, void *v_pages, int64_t vp0, int64_t vp1, int64_t vp2,
+                        int64_t num_pages, const int32_t *table, int64_t st, int64_t max_pages,
+                        int64_t N, int64_t heads, int64_t head_dim, int64_t L, void *stream);
+int evo2_rotary_decode(const void *qkv, int64_t sqkv, const float *inv_freq, float factor, void *q,
+                       void *k_pages, int64_t kp0, int64_t kp1, int64_t kp2, void *v_pages,
+                       int64_t vp0, int64_t vp1, int64_t vp2, int64_t num_pages,
+                       const int32_t *table, int64_t st, int64_t max_pages, const int64_t *positions,
+                       int64_t B, int64_t heads, int64_t head_dim, void *stream);
+
+/*
  * Static per-tensor activation quantisation for the fp8 projections:
  * q = e4m3fn(clamp(x / scale[0], -448, 448)), round to nearest even.
  *   x (rows, K) bf16, row stride sx; q (rows, K) e4m3 bytes, row stride sq.

@@ -236,3 +236,94 @@ def test_prefill_attention_peaked_scores():
     print("prefill_attention peaked scores", flush=True)
     out = prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5).cpu()
     assert max_rel_err(out, ref) <= 1e-2
+
+
+def _rotary64(x, pos, inv_freq, factor):
+    """Neox rotary in fp64: x (n, heads, hd) at positions pos (n,)."""
+    ang = (pos.double() / factor)[:, None] * inv_freq.double()
+    c, s = ang.cos()[:, None], ang.sin()[:, None]
+    a, b = x.double().chunk(2, -1)
+    return torch.cat([a * c - b * s, b * c + a * s], -1)
+
+
+def _near(got, ref):
+    """One bf16 rounding (2^-9 of the value) of an fp32 rotation whose angles
+    (below 100 rad here) carry 2^-23 relative errors: 2^-16 of |x| <= 8."""
+    assert ((got.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + 8 * 2.0 ** -16).all()
+
+
+def _qkv_case(rows, nh, hd, seed):
+    g = torch.Generator().manual_seed(seed)
+    wide = torch.randn(rows, 3 * nh * hd + 8, generator=g).to(bf)   # rows of a wider matrix
+    inv_freq = 1.0 / 10000.0 ** (torch.arange(0, hd, 2, dtype=torch.float32) / hd)
+    return g, wide, inv_freq
+
+
+@pytest.mark.parametrize("nseq,nh,L", [(1, 1, 1), (2, 3, 15), (1, 4, 64), (3, 5, 65), (2, 4, 79),
+                                       (1, 8, 200)])
+def test_rotary_prefill_vs_fp64(nseq, nh, L):
+    """Rotary, page writes and the transposed values of prompts around the
+    kernel's 64 positions, 16-position pages and four heads; one block-table
+    entry outside the cache.  Then attention over them at any L."""
+    from evo2_flash_amd.attention import prefill_attention_rows, rotary_prefill
+    hd = 128
+    g, wide, inv_freq = _qkv_case(nseq * L, nh, hd, nseq + L)
+    npg = -(-L // PAGE)
+    num_pages = nseq * npg + 2
+    table = (torch.randperm(num_pages - 1, generator=g)[:nseq * npg] + 1).int().view(nseq, npg)
+    bad = table[0, -1].item()
+    table[0, -1] = num_pages                       # not written through
+    cache = PagedKVCache(num_pages, nh, hd, DEV)
+    cache.k.fill_(7.0)
+    cache.v.fill_(7.0)
+    wd = wide.to(DEV)
+    print(f"rotary_prefill nseq={nseq} heads={nh} L={L}", flush=True)
+    q, k, vt = rotary_prefill(wd[:, :3 * nh * hd], cache, table.to(DEV), inv_freq.to(DEV), 4.0,
+                              nseq, L)
+    pos = torch.arange(L).repeat(nseq)
+    qr, kr, vr = wide[:, :3 * nh * hd].reshape(nseq * L, 3, nh, hd).unbind(1)
+    qr, kr = (_rotary64(t, pos, inv_freq, 4.0) for t in (qr, kr))
+    qr, kr, vr = (t.view(nseq, L, nh, hd).transpose(1, 2) for t in (qr, kr, vr))
+    _near(q.cpu(), qr)
+    _near(k.cpu(), kr)
+    assert torch.equal(vt.cpu()[..., :L], vr.transpose(-1, -2))
+    assert (vt.cpu()[..., L:] == 0).all()
+    # the pages hold the same k and v, a zero tail, and nothing else
+    want = PagedKVCache(num_pages, nh, hd, "cpu")
+    want.k.fill_(7.0)
+    want.v.fill_(7.0)
+    table[0, -1] = bad
+    want.write_prompt(k.cpu(), vr, table)
+    want.k[bad] = want.v[bad] = 7.0
+    assert torch.equal(cache.k.cpu(), want.k) and torch.equal(cache.v.cpu(), want.v)
+    out = torch.empty(nseq, L, nh, hd, dtype=bf, device=DEV)
+    prefill_attention_rows(q, k, vt, hd ** -0.5, out.transpose(1, 2))
+    ref = _causal_ref(q.cpu(), k.cpu(), vr, hd ** -0.5)
+    assert max_rel_err(out.cpu().transpose(1, 2), ref) <= 1e-2
+
+
+@pytest.mark.parametrize("B,nh,hd", [(1, 1, 64), (3, 9, 128), (5, 8, 32)])
+def test_rotary_decode_vs_fp64(B, nh, hd):
+    """One token per sequence, positions at both ends of pages, one sequence
+    whose page lies outside the cache, heads around the kernel's eight."""
+    from evo2_flash_amd.attention import rotary_decode
+    g, wide, inv_freq = _qkv_case(B, nh, hd, B + nh)
+    table = (torch.randperm(B * 3, generator=g) + 1).int().view(B, 3)
+    pos = torch.tensor([15, 16, 47, 0, 31][:B])
+    if B > 2:
+        table[2, 2] = -1
+    cache = PagedKVCache(B * 3 + 1, nh, hd, DEV)
+    wd = wide.to(DEV)
+    print(f"rotary_decode B={B} heads={nh} hd={hd}", flush=True)
+    q = rotary_decode(wd[:, :3 * nh * hd], cache, table.to(DEV), pos.to(DEV), inv_freq.to(DEV), 4.0)
+    qr, kr, vr = wide[:, :3 * nh * hd].reshape(B, 3, nh, hd).unbind(1)
+    _near(q.cpu(), _rotary64(qr, pos, inv_freq, 4.0))
+    kr = _rotary64(kr, pos, inv_freq, 4.0)
+    kc, vc = cache.k.cpu(), cache.v.cpu()
+    for b in range(B):
+        pg, off = int(table[b, pos[b] // PAGE]), int(pos[b] % PAGE)
+        if pg >= 0:
+            _near(kc[pg, :, :, off], kr[b])
+            assert torch.equal(vc[pg, :, off], vr[b])
+            kc[pg, :, :, off] = vc[pg, :, off] = 0
+    assert (kc == 0).all() and (vc == 0).all()      # and nowhere else
