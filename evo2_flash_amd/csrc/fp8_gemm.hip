@@ -7,7 +7,9 @@
 // (mixers.py:741-757, 1076-1092; scales in the dequantisation convention,
 // convert.py:195-201), and the same GEMM for out_proj when it is quantised.
 //
-// Kernel: a 256 x 256 output tile per workgroup (W rows x X rows).  Four
+// General kernel (shapes the persistent one below does not take: K off 128,
+// N off 8, unaligned outputs, operands past 2 GB): a 256 x 256 output tile per
+// workgroup (W rows x X rows).  Four
 // waves each own a 128 x 128 quadrant as 4 x 4 tiles of
 // v_mfma_f32_32x32x64_f8f6f4 (the weight is MFMA operand A, so each lane
 // ends up with four consecutive output columns of one row, stored as one
@@ -23,7 +25,9 @@
 // lanes (16 consecutive rows) at a time over 64 banks, and the swizzle puts
 // those 16 rows' chunks in 16 different bank groups.
 #include <algorithm>
+#include <climits>
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 
@@ -32,7 +36,17 @@ namespace evo2 {
 typedef __attribute__((ext_vector_type(8))) int i32x8;
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 typedef __attribute__((address_space(3))) void lds_void;
+
+template <int... I, class F>
+__device__ __forceinline__ void static_for_seq(std::integer_sequence<int, I...>, F &&f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+  static_for_seq(std::make_integer_sequence<int, N>{}, f);
+}
 
 constexpr int G_BM = 256;       // X rows per workgroup
 constexpr int G_BN = 256;       // W rows per workgroup
@@ -225,17 +239,21 @@ __global__ __launch_bounds__(256) void fp8_gemm_kernel(GemmArgs p) {
 }
 
 // ---------------------------------------------------------------------------
-// Persistent form of the same tile.  One workgroup per CU walks the output
-// tiles t = blockIdx.x, blockIdx.x + gridDim.x, ..., and its global -> LDS
-// pipeline runs straight across tile boundaries: the first slice of the next
-// tile is already loading while the current one finishes and writes its
-// epilogue, so a tile's start-up latency is paid once per workgroup rather
-// than once per tile.
+// Persistent form, with 64 to 256 X rows a tile (64 TM).  One workgroup per CU
+// walks the output tiles t = blockIdx.x, blockIdx.x + gridDim.x, ..., and its
+// global -> LDS pipeline runs straight across tile boundaries: the first slice
+// of the next tile is already loading while the current one finishes and
+// writes its epilogue, so a tile's start-up latency is paid once per workgroup
+// rather than once per tile.  Rows past M or N read zeros and store nothing,
+// so any M takes it, and the tile height is chosen by how many rounds over the
+// CUs a launch needs (persist_rows): a 256 x 256 grid leaves up to half of
+// them idle at M between 65 and ~6000.
 //
 // K moves in slices of 128 bytes: each row's slice is one whole 128-byte
 // line, so a direct-to-LDS instruction (64 lanes x 16 bytes = 8 rows) asks
-// for 8 full lines.  Two stages of 32 KB of W and 32 KB of X; slice k + 2 is
-// loaded into the stage of slice k as soon as every wave has read slice k,
+// for 8 full lines.  Two stages of 32 KB of W and 8 TM KB of X (three at TM <= 2,
+// whose short slices are bound by the loads' latency; more stages gained nothing
+// at TM 3 and do not fit at 4); slice k + 2 is loaded into the stage of slice k as soon as every wave has read slice k,
 // and a slice takes two v_mfma_f32_32x32x64_f8f6f4 sub-steps (64 bytes of K
 // each), so a load has a whole slice of matrix work (~1.1 us) to land and
 // the workgroup meets at one barrier per slice.  LDS rows are 128 bytes;
@@ -260,7 +278,6 @@ __device__ __forceinline__ int lane_now() {
 
 constexpr int Q_BK = 128;               // bytes of K per slice
 constexpr int Q_STAGE = G_BN * Q_BK;    // bytes per operand per stage
-constexpr int Q_KALIGN = 2 * Q_BK;      // K granularity: whole slice pairs per tile
 
 // The grouped order needs a grid of 256 and whole 4 x 8 blocks.
 __host__ __device__ inline bool persist_grouped(int ncu, int tiles_n, int tiles_m) {
@@ -268,9 +285,13 @@ __host__ __device__ inline bool persist_grouped(int ncu, int tiles_n, int tiles_
 }
 
 // Output tile (bn, bm) of the t-th tile in the persistent order, for
-// 0 <= t < tiles_n * tiles_m; a bijection onto the tile grid.
-__host__ __device__ inline void persist_tile(int t, int tiles_n, int tiles_m, bool grouped, int &bn,
-                                             int &bm) {
+// 0 <= t < tiles_n * tiles_m, with `grid` workgroups; a bijection onto the
+// tile grid.  Where the grid does not split into whole 4 x 8 blocks, the tiles
+// are numbered down panels of four W tiles (row by row inside a panel), and
+// each round hands every XCD one contiguous run of them: 32 tiles of a panel
+// are a 4 x 8 block again.
+__host__ __device__ inline void persist_tile(int t, int tiles_n, int tiles_m, int grid, bool grouped,
+                                             int &bn, int &bm) {
   if (grouped) {
     const int nbn = tiles_n >> 2;
     const int whole = ((nbn * (tiles_m >> 3)) >> 3) << 8;  // tiles in whole rounds
@@ -285,37 +306,50 @@ __host__ __device__ inline void persist_tile(int t, int tiles_n, int tiles_m, bo
     bn = (blk % nbn) * 4 + (i & 3);
     bm = (blk / nbn) * 8 + (i >> 2);
   } else {
-    bn = t % tiles_n;
-    bm = t / tiles_n;
+    const int r0 = t / grid * grid, pos = t - r0;
+    const int left = tiles_n * tiles_m - r0, cnt = left < grid ? left : grid;  // this round's tiles
+    const int x = pos & 7, rest = cnt & 7;
+    const int u = r0 + x * (cnt >> 3) + (x < rest ? x : rest) + (pos >> 3);
+    const int panel = u / (4 * tiles_m), v = u - panel * 4 * tiles_m;
+    const int w = tiles_n - 4 * panel < 4 ? tiles_n - 4 * panel : 4;
+    bm = v / w;
+    bn = 4 * panel + v - bm * w;
   }
 }
 
+// TM: the tile is 64 TM X rows (a wave 32 TM of them); ODD: an odd number of
+// slices per tile, so that every other tile starts in stage 1.
+template <int TM, bool ODD>
 __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int tiles_n, int tiles_m,
                                                                int grouped) {
-  __shared__ __align__(16) uint8_t w0[Q_STAGE], w1[Q_STAGE];
-  __shared__ __align__(16) uint8_t x0[Q_STAGE], x1[Q_STAGE];
+  constexpr int BM = 64 * TM;
+  constexpr int NST = TM <= 2 ? 3 : 2;  // stages
+  __shared__ __align__(16) uint8_t w0[Q_STAGE], w1[Q_STAGE], w2[NST > 2 ? Q_STAGE : 16];
+  __shared__ __align__(16) uint8_t x0[BM * Q_BK], x1[BM * Q_BK], x2[NST > 2 ? BM * Q_BK : 16];
   // The bias of even and odd tiles, loaded direct-to-LDS a whole tile ahead
   // of the epilogue that adds it (64 lanes x 16 bytes: the tile's 256
   // columns and the next 256, unused).  Reading it then never waits on the
   // memory pipe, where a load would also wait for the next tile's operand
   // loads and the stores before it.
   __shared__ __align__(16) bf16_t bias0[512], bias1[512];
-  constexpr int DB = Q_STAGE / 4 / 1024;  // 1 KB DMA blocks per operand, wave and slice (8)
+  constexpr int DB = Q_STAGE / 4 / 1024;  // 1 KB DMA blocks of W per wave and slice (8)
+  constexpr int DX = BM * Q_BK / 4 / 1024;  // and of X (2 TM)
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = (wave & 1) * 128;   // wave's W rows
-  const int wm = (wave >> 1) * 128;  // wave's X rows
+  const int wm = (wave >> 1) * (32 * TM);  // wave's X rows
   const int total = tiles_n * tiles_m;
-  const int KT = p.K / Q_BK;  // slices per tile, even
+  const int KT = p.K / Q_BK;  // slices per tile (even unless ODD)
   int grid = static_cast<int>(gridDim.x);
   asm volatile("" : "+s"(grid));  // kept in an SGPR, not reloaded from the dispatch packet
   const int ntile = (total - static_cast<int>(blockIdx.x) + grid - 1) / grid;
   const int nsteps = ntile * KT;
+  if (ntile <= 0) return;  // uniform; (the host launches no such workgroup)
 
   // Operands through buffer descriptors over the whole matrices (their byte
-  // extents fit 32 bits, checked on the host).
+  // extents fit 32 bits, checked on the host): rows past the last read zeros.
   const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t *>(p.w), 0, static_cast<int>((int64_t)(p.N - 1) * p.sw + p.K), 0x00020000);
   const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
@@ -327,9 +361,11 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
   // DMA: one wave instruction fills 1 KB = 8 rows of 128 bytes; lane i writes
   // row i / 8, physical chunk i % 8, which holds logical chunk
   // (i % 8) ^ ((row >> 1) & 7).  Block j of a wave covers rows
-  // 8 (DB wave + j) + i / 8, whose swizzle is ((i / 16) + 4 (j & 1)) & 7: two
-  // lane offsets per operand (even and odd blocks, row within the block and
-  // chunk), the block's row offset and the K offset in SGPRs.
+  // 8 (DB wave + j) + i / 8 (X: DX), whose swizzle is ((i / 16) + 4 (j & 1)) & 7:
+  // two lane offsets per operand (even and odd blocks, row within the block
+  // and chunk), the block's row offset and the K offset in SGPRs.  A block
+  // past the last row starts at the last row instead (the offset of a buffer
+  // access in its SGPR has to lie inside the buffer).
   int lw[2], lx[2];
   {
     const int r = lane >> 3;
@@ -340,18 +376,21 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
       lx[par] = r * static_cast<int>(p.sx) + chunk;
     }
   }
+  const int wlast = (p.N - 1) * static_cast<int>(p.sw), xlast = (p.M - 1) * static_cast<int>(p.sx);
   int tw = 0, tx = 0;  // byte offsets of the wave's first DMA row in the tile being loaded
   auto dma_tile = [&](int j) __attribute__((always_inline)) {
     int bn, bm;
-    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grouped != 0, bn, bm);
+    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grid, grouped != 0, bn, bm);
     tw = (bn * G_BN + DB * 8 * wave) * static_cast<int>(p.sw);
-    tx = (bm * G_BM + DB * 8 * wave) * static_cast<int>(p.sx);
+    tx = (bm * BM + DX * 8 * wave) * static_cast<int>(p.sx);
   };
   auto stage_w = [&](auto stage) __attribute__((always_inline)) -> uint8_t * {
-    return decltype(stage)::value ? w1 : w0;
+    constexpr int S = decltype(stage)::value;
+    return S == 0 ? w0 : S == 1 ? w1 : w2;
   };
   auto stage_x = [&](auto stage) __attribute__((always_inline)) -> uint8_t * {
-    return decltype(stage)::value ? x1 : x0;
+    constexpr int S = decltype(stage)::value;
+    return S == 0 ? x0 : S == 1 ? x1 : x2;
   };
   // Slice q of this workgroup's sequence (tile q / KT, K slice q % KT) into
   // a stage; slices past the end re-read the last one, so every step issues
@@ -369,11 +408,13 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
     uint8_t *lxp = stage_x(stage);
 #pragma unroll
     for (int j = 0; j < DB; ++j) {
-      const int blk = wave * DB + j;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (lds_void *)(lwp + blk * 1024), 16, lw[j & 1],
-                                               tw + 8 * j * static_cast<int>(p.sw) + koff, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_void *)(lxp + blk * 1024), 16, lx[j & 1],
-                                               tx + 8 * j * static_cast<int>(p.sx) + koff, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          wrs, (lds_void *)(lwp + (wave * DB + j) * 1024), 16, lw[j & 1],
+          min(tw + 8 * j * static_cast<int>(p.sw), wlast) + koff, 0, 0);
+      if (j < DX)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            xrs, (lds_void *)(lxp + (wave * DX + j) * 1024), 16, lx[j & 1],
+            min(tx + 8 * j * static_cast<int>(p.sx), xlast) + koff, 0, 0);
     }
   };
 
@@ -382,7 +423,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
   const int sw = (lr >> 1) & 7;  // swizzle of every row this lane reads
   // Fragments of sub-step h of a stage: row r = base + 32 t + lr, logical
   // chunks 4h + 2g and 4h + 2g + 1.
-  auto read_frags = [&](auto stage, auto sub, i32x8 fa[4], i32x8 fb[4]) __attribute__((always_inline)) {
+  auto read_frags = [&](auto stage, auto sub, i32x8 fa[4], i32x8 fb[TM]) __attribute__((always_inline)) {
     constexpr int H = decltype(sub)::value;
     const uint8_t *lwp = stage_w(stage);
     const uint8_t *lxp = stage_x(stage);
@@ -390,7 +431,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
     // in the order the MFMAs consume them (tn-major: every X fragment and W
     // fragment 0 first)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < TM; ++t) {
       const uint8_t *row = lxp + (wm + 32 * t + lr) * Q_BK;
       const uint4 b0 = *reinterpret_cast<const uint4 *>(row + c0);
       const uint4 b1 = *reinterpret_cast<const uint4 *>(row + c1);
@@ -407,13 +448,13 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
 
   // The accumulators of a tile start at its first MFMAs, which take C = 0
   // (no clearing between tiles), so they are not live across tiles.
-  f32x16 acc[4][4];
+  f32x16 acc[4][TM];
   const f32x16 zero16 = {};
-  auto mma = [&](const i32x8 fa[4], const i32x8 fb[4], auto first) __attribute__((always_inline)) {
+  auto mma = [&](const i32x8 fa[4], const i32x8 fb[TM], auto first) __attribute__((always_inline)) {
 #pragma unroll
     for (int tn = 0; tn < 4; ++tn)
 #pragma unroll
-      for (int tm = 0; tm < 4; ++tm)
+      for (int tm = 0; tm < TM; ++tm)
         acc[tn][tm] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
             fa[tn], fb[tm], decltype(first)::value ? zero16 : acc[tn][tm], 0, 0, 0, 0, 0, 0);
   };
@@ -422,37 +463,43 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
   auto load_bias = [&](auto par, int j) __attribute__((always_inline)) {
     if (!p.bias || wave != 0) return;  // uniform
     int bn, bm;
-    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grouped != 0, bn, bm);
+    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grid, grouped != 0, bn, bm);
     bf16_t *lb = decltype(par)::value ? bias1 : bias0;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(brs, (lds_void *)lb, 16, 16 * lane_now(), 2 * bn * G_BN,
                                              0, 0);
   };
   // Epilogue of tile j: lane holds, for X row m = m0 + wm + 32 tm + lr, the
   // W rows n = n0 + wn + 32 tn + 8 q + 4 g + i (i < 4) in acc[tn][tm][4 q + i].
-  // Every store address is one of four row pointers plus a constant; a lane
-  // issues EPI_STORES 16-byte stores (4 tm x 4 tn x 2 pairs).
-  constexpr int EPI_STORES = 4 * 4 * 2;
-  auto epilogue = [&](auto par, int j) __attribute__((always_inline)) {
+  // The stores go through a buffer descriptor over the tile's rows: a lane
+  // issues EPI_STORES 16-byte stores (TM tm x 4 tn x 2 pairs) whatever the
+  // tile, those past the last row or column falling outside it.
+  constexpr int EPI_STORES = TM * 4 * 2;
+  auto epilogue = [&](int j) __attribute__((always_inline)) {
     int bn, bm;
-    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grouped != 0, bn, bm);
+    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grid, grouped != 0, bn, bm);
     // The order is a bijection onto the grid (checked on the host for every
     // grid up to 64 x 40 tiles); a tile outside it stores nothing rather than
     // past the output (the operand loads are bounded by their descriptors).
     if (bn < 0 || bn >= tiles_n || bm < 0 || bm >= tiles_m) return;  // wave-uniform
-    // whole tiles only (the host checks M and N are multiples of 256 and the
-    // output rows 16-byte aligned)
+    // (N is a multiple of 8 and the output rows 16-byte aligned, checked on
+    // the host)
+    const int rows = min(BM, p.M - bm * BM), cols = min(G_BN, p.N - bn * G_BN);
+    const int so = static_cast<int>(p.so);
+    const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(
+        p.out + (int64_t)(bm * BM) * p.so + bn * G_BN, 0, 2 * ((rows - 1) * so + cols), 0x00020000);
     // Lanes l and l + 32 hold the same row: for each pair of column groups
     // (q, q + 1) they swap halves (v_permlane32_swap) so that lane l ends up
     // with columns 16 p .. 16 p + 7 and lane l + 32 with 16 p + 8 .. 16 p + 15,
     // and each stores 16 contiguous bytes: half as many store requests.
     const int ln = lane_now();
     const int elr = ln & 31, eg = ln >> 5;
-    bf16_t *obase = p.out + (int64_t)(bm * G_BM + wm + elr) * p.so + bn * G_BN + wn + 8 * eg;
-    const bf16_t *lb = (decltype(par)::value ? bias1 : bias0) + wn + 4 * eg;
+    const int left = cols - wn - 8 * eg;  // columns from the lane's first
+    const int voff = 2 * ((wm + elr) * so + wn + 8 * eg);
+    const bf16_t *lb = (j & 1 ? bias1 : bias0) + wn + 4 * eg;
     const bool has_bias = p.bias != nullptr;
 #pragma unroll
-    for (int tm = 0; tm < 4; ++tm) {
-      bf16_t *orow = obase + (int64_t)(32 * tm) * p.so;
+    for (int tm = 0; tm < TM; ++tm) {
+      const int vrow = voff + 64 * tm * so;
 #pragma unroll
       for (int tn = 0; tn < 4; ++tn) {
         uint32_t pk[4][2];  // column group q, packed pairs
@@ -477,7 +524,9 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
           // get y of lane - 32 and keep y
           const auto s0 = __builtin_amdgcn_permlane32_swap(pk[2 * pq][0], pk[2 * pq + 1][0], false, false);
           const auto s1 = __builtin_amdgcn_permlane32_swap(pk[2 * pq][1], pk[2 * pq + 1][1], false, false);
-          *reinterpret_cast<uint4 *>(orow + 32 * tn + 16 * pq) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+          const int c = 32 * tn + 16 * pq;
+          __builtin_amdgcn_raw_buffer_store_b128(u32x4{s0[0], s1[0], s0[1], s1[1]}, ors,
+                                                 c < left ? vrow + 2 * c : INT_MIN, 0, 0);
         }
       }
     }
@@ -495,33 +544,39 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
   // stores outstanding (and, in wave 0, the next bias load after them), all
   // issued after the loads of slice k + 1: loads and stores retire in order,
   // so waiting until at most EPI_STORES remain covers the loads.
-  i32x8 fa[2][4], fb[2][4];
-  auto interleave = [&](bool dma) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
+  i32x8 fa[2][4], fb[2][TM];
+  // every MFMA of a sub-step is followed by its share of the fragment reads
+  // and of the refill loads
+  auto interleave = [&](auto dma) __attribute__((always_inline)) {
+    static_for<4 * TM>([&](auto i) __attribute__((always_inline)) {
+      constexpr int I = decltype(i)::value, NM = 4 * TM, ND = 2 * (4 + TM), NV = DB + DX;
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
-      if (dma) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // VMEM read
-    }
+      __builtin_amdgcn_sched_group_barrier(0x100, (I + 1) * ND / NM - I * ND / NM, 0);  // DS read
+      if constexpr (decltype(dma)::value)
+        __builtin_amdgcn_sched_group_barrier(0x020, (I + 1) * NV / NM - I * NV / NM, 0);  // VMEM read
+    });
   };
   using std::integral_constant;
   using I0 = integral_constant<int, 0>;
   using I1 = integral_constant<int, 1>;
   using F0 = integral_constant<bool, false>;
   using F1 = integral_constant<bool, true>;
-  // first: slice 0 of a tile, whose sub-step 0 starts the accumulators
+  // first: slice 0 of a tile, whose sub-step 0 starts the accumulators.  With
+  // three stages slice k + 2 may still be in flight when slice k + 1 is
+  // waited for, and the freed stage takes slice k + 3.
   auto step = [&](auto stage, int k, bool after_epilogue, auto first) __attribute__((always_inline)) {
     constexpr int S = decltype(stage)::value;
+    constexpr int FLY = (NST - 2) * (DB + DX);
     read_frags(stage, I1{}, fa[1], fb[1]);
     mma(fa[0], fb[0], first);
-    interleave(false);
-    if (after_epilogue) vmcnt_wait<EPI_STORES>();
-    else vmcnt_wait<0>();
+    interleave(F0{});
+    if (after_epilogue) vmcnt_wait<FLY + EPI_STORES>();
+    else vmcnt_wait<FLY>();
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    issue(stage, k + 2);
-    read_frags(integral_constant<int, S ^ 1>{}, I0{}, fa[0], fb[0]);
+    issue(stage, k + NST);
+    read_frags(integral_constant<int, (S + 1) % NST>{}, I0{}, fa[0], fb[0]);
     mma(fa[1], fb[1], F0{});
-    interleave(true);
+    interleave(F1{});
   };
 
   using P0 = integral_constant<int, 0>;
@@ -530,30 +585,62 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
   dma_tile(0);
   issue(I0{}, 0);
   issue(I1{}, 1);
-  vmcnt_wait<2 * DB>();  // slice 0 (slice 1 in flight; the bias before them)
+  if constexpr (NST == 3) issue(integral_constant<int, 2>{}, 2);
+  vmcnt_wait<(NST - 1) * (DB + DX)>();  // slice 0 (the next in flight; the bias before them)
   __builtin_amdgcn_s_barrier();
   read_frags(I0{}, I0{}, fa[0], fb[0]);
-  int s = 0;
-  // Tile j of parity P: first the bias of tile j + 1 into the other buffer
-  // (its previous contents, tile j - 1's, were added before this tile
-  // began), then the slices in pairs (KT is even, so every tile starts in
-  // stage 0; the first pair starts the accumulators), then the epilogue
-  // with this buffer.
-  auto tile = [&](auto par, int j) __attribute__((always_inline)) {
-    constexpr int P = decltype(par)::value;
-    if (j + 1 < ntile) load_bias(integral_constant<int, P ^ 1>{}, j + 1);
-    step(I0{}, s, j > 0, F1{});
-    step(I1{}, s + 1, false, F0{});
-    s += 2;
-    for (int k = 2; k < KT; k += 2, s += 2) {
-      step(I0{}, s, false, F0{});
-      step(I1{}, s + 1, false, F0{});
+  if constexpr (NST == 3) {
+    // the slices of all tiles as one sequence, three stages in turn
+    int kk = 0, j = 0;  // slice within the tile, tile
+    bool after = false;
+    auto one = [&](auto stage, int k) __attribute__((always_inline)) {
+      if (kk == 0) {  // uniform: a tile begins (its accumulators at zero)
+        if (j + 1 < ntile) {
+          if (j & 1) load_bias(P0{}, j + 1);
+          else load_bias(P1{}, j + 1);
+        }
+#pragma unroll
+        for (int tn = 0; tn < 4; ++tn)
+#pragma unroll
+          for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = zero16;
+      }
+      step(stage, k, after, F0{});
+      after = ++kk == KT;
+      if (after) {
+        epilogue(j);
+        kk = 0;
+        ++j;
+      }
+    };
+    for (int k = 0; k < nsteps; k += 3) {
+      one(I0{}, k);
+      if (k + 1 < nsteps) one(I1{}, k + 1);
+      if (k + 2 < nsteps) one(integral_constant<int, 2>{}, k + 2);
     }
-    epilogue(par, j);
-  };
-  for (int j = 0; j < ntile; j += 2) {
-    tile(P0{}, j);
-    if (j + 1 < ntile) tile(P1{}, j + 1);
+  } else {
+    int s = 0;
+    // Tile j of parity P: first the bias of tile j + 1 into the other buffer
+    // (its previous contents, tile j - 1's, were added before this tile
+    // began), then the slices, the first starting the accumulators (an even
+    // count in pairs from stage 0; an odd one from stage P), then the epilogue
+    // with this buffer.
+    auto tile = [&](auto par, int j) __attribute__((always_inline)) {
+      constexpr int P = decltype(par)::value, S = ODD ? P : 0;
+      using A = integral_constant<int, S>;
+      using B = integral_constant<int, S ^ 1>;
+      if (j + 1 < ntile) load_bias(integral_constant<int, P ^ 1>{}, j + 1);
+      step(A{}, s++, j > 0, F1{});
+      if (!ODD) step(B{}, s++, false, F0{});
+      for (int k = ODD ? 1 : 2; k < KT; k += 2, s += 2) {
+        step(integral_constant<int, ODD ? S ^ 1 : 0>{}, s, false, F0{});
+        step(integral_constant<int, ODD ? S : 1>{}, s + 1, false, F0{});
+      }
+      epilogue(j);
+    };
+    for (int j = 0; j < ntile; j += 2) {
+      tile(P0{}, j);
+      if (j + 1 < ntile) tile(P1{}, j + 1);
+    }
   }
   // No direct-to-LDS write may still be landing when the workgroup's LDS is
   // handed to the next one.
@@ -791,11 +878,18 @@ __global__ __launch_bounds__(256) void fp8_pack_kernel(const uint8_t *w, int64_t
 }
 
 // The weight-streaming kernel reads the weight once per 64-row block, so its
-// cost grows with ceil(M / 64) x N x K, while up to one round of 256 x 256
-// tiles costs one tile's K loop.  Measured with the weights streaming from
-// HBM (K = 4096, us, stream / tiles): M=256, N=12288 42 / 62; M=512 75 / 62;
-// M=512, N=4096 25 / 41; M=1024 48 / 43; M=256, N=24576, K=8192 138 / 115.
-// Streaming takes ceil(M / 64) x N up to this; M <= 64 always streams.
+// cost grows with ceil(M / 64) x N x K, while one round of the persistent
+// kernel's smallest tiles costs one tile's K loop.  Measured with the weights
+// streaming from HBM (K = 4096, us, stream / tiles): M=65, N=4096 11.5 / 24.1;
+// M=300, N=4096 22.9 / 23.7; M=777, N=4096 53.7 / 24.9; N=12288: M=65 26.1 /
+// 31.6, M=128 28.2 / 33.8, M=200 44.1 / 31.7, M=300 51.3 / 32.9; K=1920,
+// N=5760: M=130 14.0 / 14.0, M=600 31.8 / 15.2.  Streaming takes
+// ceil(M / 64) x N up to TILE_MIN_WORK (the tiles are the faster from ~30000;
+// verify-sized steps, M <= 256 at N = 12288, keep the streaming kernels' sums,
+// the same bits with a packed weight and without), and up to STREAM_MAX_WORK where the
+// persistent kernel does not apply (against the 256 x 256 tile kernel: M=256,
+// N=12288 42 / 62; M=512, N=4096 25 / 41); M <= 64 always streams.
+#define TILE_MIN_WORK 50000
 #ifndef STREAM_MAX_WORK
 #define STREAM_MAX_WORK 60000
 #endif
@@ -881,6 +975,39 @@ static int cu_count() {
 // 75.8 us, the fastest of this kernel and of workgroups covering 2-4 row
 // blocks per weight load (which only won while the weights stayed
 // cache-resident).
+template <int TM>
+static void launch_persist(const GemmArgs &a, int ncu, hipStream_t st) {
+  const int tiles_n = static_cast<int>(cdiv(a.N, G_BN)), tiles_m = static_cast<int>(cdiv(a.M, 64 * TM));
+  const int grid = std::min(ncu, tiles_n * tiles_m);
+  const int grouped = persist_grouped(grid, tiles_n, tiles_m);
+  if (TM > 2 && a.K / Q_BK % 2)  // (three stages take any count of slices)
+    hipLaunchKernelGGL((fp8_gemm_persist_kernel<TM, (TM > 2)>), dim3(grid), dim3(256), 0, st, a, tiles_n, tiles_m, grouped);
+  else
+    hipLaunchKernelGGL((fp8_gemm_persist_kernel<TM, false>), dim3(grid), dim3(256), 0, st, a, tiles_n, tiles_m, grouped);
+}
+
+// X rows of a tile (in units of 64) of the persistent kernel: the fewest
+// rounds of tiles over the CUs, weighted by what a round costs, TM + 1.3
+// (rounds measured over 32768 x 12288 x 4096, us: 51.5, 39.5, 31.9, 22.3 for
+// TM 4 .. 1; a single round is bound by its loads' latency and costs a little
+// less).  The larger tile on a tie.  Measured at K = 4096 (1920 for N = 5760,
+// 1920), us for TM 4 / 3 / 2 / 1: 300 x 12288 52.0 / 46.6 / 37.5 / 33.2; 777 x
+// 12288 52.8 / 47.3 / 69.8 / 87.1; 3001 x 12288 163 / 147 / 182 / 265; 6001 x
+// 12288 262 / 265 / 304 / 409; 2047 x 5760 27.7 / 25.5 / 34.7 / 38.0; 2047 x
+// 1920 24.1 / 20.7 / 18.4 / 15.3.
+static int persist_rows(int64_t tiles_n, int64_t M, int ncu) {
+  int best = 4;
+  double least = 1e30;
+  for (int tm = 4; tm >= 1; --tm) {
+    const double cost = double(cdiv(tiles_n * cdiv(M, 64 * tm), ncu)) * (tm + 1.3);
+    if (cost < least - 1e-9) {
+      least = cost;
+      best = tm;
+    }
+  }
+  return best;
+}
+
 template <bool PACKED>
 static void launch_stream(const GemmArgs &a, hipStream_t st) {
   const int ncu = cu_count() > 0 ? cu_count() : 256;
@@ -954,23 +1081,30 @@ extern "C" int evo2_fp8_gemm(const void *x8, int64_t sx, const void *w8, int64_t
              w_scale, static_cast<const bf16_t *>(bias), static_cast<bf16_t *>(out), so,
              static_cast<int>(M), static_cast<int>(N), static_cast<int>(K)};
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t tiles_n = cdiv(N, G_BN), tiles_m = cdiv(M, G_BM);
+  const int ncu = cu_count();
+  // the persistent kernel: whole 128-byte slices of K, columns in eights,
+  // 16-byte aligned output rows, operands (rounded up to whole tiles) and a
+  // tile's output within 32-bit buffer offsets
+  const bool tiles = ncu > 0 && K % Q_BK == 0 && N % 8 == 0 && so % 8 == 0 &&
+                     reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
+                     (!bias || reinterpret_cast<uintptr_t>(bias) % 8 == 0) && so < (1 << 20) &&
+                     sx >= K && sw >= K && so >= N && tiles_n * tiles_m < (1 << 24) &&
+                     (tiles_n * G_BN) * sw + K < (int64_t(1) << 31) &&
+                     (tiles_m * G_BM) * sx + K < (int64_t(1) << 31);
+  const int64_t work = cdiv(M, S_ROWS) * N;
   if (K % S_BK == 0 && sx * S_ROWS < (int64_t(1) << 31) &&
-      (M <= S_ROWS || cdiv(M, S_ROWS) * N <= STREAM_MAX_WORK)) {
+      (M <= S_ROWS || work <= (tiles ? TILE_MIN_WORK : STREAM_MAX_WORK))) {
     // the weight-streaming kernel over ceil(M / 64) blocks of 64 rows
     launch_stream<false>(a, st);
     return check_launch("fp8_gemm");
   }
-  const int64_t tiles_n = cdiv(N, G_BN), tiles_m = cdiv(M, G_BM);
-  const int ncu = cu_count();
-  // the persistent form once every CU has a tile; its ring needs K to be a
-  // multiple of four K steps and the operands to fit 32-bit buffer offsets
-  if (ncu > 0 && tiles_n * tiles_m >= ncu && K % Q_KALIGN == 0 &&
-      M % G_BM == 0 && N % G_BN == 0 && so % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-      (!bias || reinterpret_cast<uintptr_t>(bias) % 8 == 0) &&
-      (N - 1) * sw + K < (int64_t(1) << 31) && (M - 1) * sx + K < (int64_t(1) << 31)) {
-    const int grouped = persist_grouped(ncu, static_cast<int>(tiles_n), static_cast<int>(tiles_m));
-    hipLaunchKernelGGL(fp8_gemm_persist_kernel, dim3(static_cast<unsigned>(ncu)), dim3(256), 0, st, a,
-                       static_cast<int>(tiles_n), static_cast<int>(tiles_m), grouped);
+  if (tiles) {
+    const int tm = persist_rows(tiles_n, M, ncu);
+    if (tm == 4) launch_persist<4>(a, ncu, st);
+    else if (tm == 3) launch_persist<3>(a, ncu, st);
+    else if (tm == 2) launch_persist<2>(a, ncu, st);
+    else launch_persist<1>(a, ncu, st);
     return check_launch("fp8_gemm");
   }
   dim3 grid(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m));
@@ -1031,7 +1165,7 @@ extern "C" int64_t evo2_fp8_gemm_persist_order(int64_t tiles_n, int64_t tiles_m,
   if (bn && bm) {
     for (int t = 0; t < total; ++t) {
       int n, m;
-      persist_tile(t, tn, tm, grouped, n, m);
+      persist_tile(t, tn, tm, ncu, grouped, n, m);
       bn[t] = n;
       bm[t] = m;
     }

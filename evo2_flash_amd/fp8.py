@@ -62,13 +62,15 @@ def fp8_gemm(x8, w8, x_scale, w_scale, bias=None, out=None):
     return out
 
 
-STREAM_MAX_WORK = 60000  # evo2_fp8_gemm streams the weight while ceil(M / 64) * N <= this
+STREAM_MAX_WORK = 60000  # evo2_fp8_gemm may stream the weight while ceil(M / 64) * N <= this
+TILE_MIN_WORK = 50000    # and above this prefers its persistent tile kernel (M > 64)
 
 
 def streams_weight(M, N):
-    """Whether evo2_fp8_gemm takes its weight-streaming kernel for M rows
+    """Whether evo2_fp8_gemm may take its weight-streaming kernel for M rows
     (always at M <= 64; over 64-row blocks while ceil(M / 64) * N is at most
-    STREAM_MAX_WORK): the shapes where a packed weight copy is read instead."""
+    STREAM_MAX_WORK): the shapes a packed weight copy is kept for.  Above
+    TILE_MIN_WORK the persistent tile kernel is the faster one."""
     return 0 < M and (M <= 64 or -(-M // 64) * N <= STREAM_MAX_WORK)
 
 
@@ -128,14 +130,16 @@ def fp8_gemm_packed(x8, wp, x_scale, w_scale, bias=None, out=None):
 def static_fp8_linear(x, weight, input_scale, weight_scale, bias=None, out=None, packed=None):
     """vLLM's static W8A8 linear: (..., K) bf16 -> (..., N) bf16; a 2-D x may
     write its result into `out` (M, N) bf16 with unit column stride.  With
-    `packed` (fp8_pack_weight(weight)), inputs of at most 64 rows take the
-    decode GEMM on it wherever the weight would be streamed (the same result
-    bits)."""
+    `packed` (fp8_pack_weight(weight)), inputs whose weight fp8_gemm would
+    stream take the decode GEMM on it (the same result bits): at most 64
+    rows, or ceil(M / 64) * N <= TILE_MIN_WORK."""
     K = x.shape[-1]
     x8 = quantize_input(x.reshape(-1, K), input_scale)
     gemm = fp8_gemm
     w = weight
-    if packed is not None and streams_weight(x8.shape[0], weight.shape[0]):
+    M, N = x8.shape[0], weight.shape[0]
+    if packed is not None and streams_weight(M, N) and (
+            M <= 64 or -(-M // 64) * N <= TILE_MIN_WORK):
         gemm, w = fp8_gemm_packed, packed
     if out is not None:
         if x.dim() != 2 or out.shape != (x.shape[0], weight.shape[0]) or out.stride(1) != 1:

@@ -475,11 +475,11 @@ int evo2_fp8_gemm_packed(const void *x8, int64_t sx, const void *wp,
 
 /*
  * The order in which evo2_fp8_gemm's persistent kernel (one workgroup per
- * compute unit, 256 x 256 output tiles) walks a grid of tiles_n x tiles_m
- * tiles on a device with ncu compute units: tile t, run by workgroup
+ * compute unit; 256 W rows x 64 to 256 X rows a tile) walks a grid of tiles_n x
+ * tiles_m tiles with ncu workgroups: tile t, run by workgroup
  * t mod ncu, is output tile (bn[t], bm[t]).  Fills bn / bm (tiles_n * tiles_m
  * entries each, both may be NULL) and returns 1 for the XCD-grouped order,
- * 0 for row-major, -1 for bad sizes.  Host only, no GPU needed.
+ * 0 for the panel order, -1 for bad sizes.  Host only, no GPU needed.
  *
  * No counterpart in the reference (its GEMM is a library call): a planning
  * query for callers and tests that check the tile order covers every tile.

@@ -100,6 +100,31 @@ def test_gemm_known_answer_persistent(M, N, K):
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 32768, 128), (257, 12288, 256), (300, 24584, 384),
+                                   (511, 12288, 640), (777, 12296, 256), (1537, 5768, 384),
+                                   (2047, 5760, 256), (3001, 8192, 128), (6001, 5000, 256)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_gemm_known_answer_ragged_tiles(M, N, K, bias):
+    """The persistent kernel off whole tiles, each of its four tile heights
+    (one and several rounds over the CUs, the last part-filled): rows and
+    columns past the output (columns in eights) and odd counts of 128-byte
+    slices.  Small-integer operands, exact sums: bit for bit, and nothing
+    written beside the output."""
+    g = torch.Generator().manual_seed(M + K)
+    x8 = _small_int_e4m3((M, K), g).to(DEV)
+    w8 = _small_int_e4m3((N, K), g).to(DEV)
+    b = torch.randint(-8, 9, (N,), generator=g).to(torch.bfloat16).to(DEV) if bias else None
+    wide = torch.full((M + 1, N + 8), 99.0, dtype=torch.bfloat16, device=DEV)
+    one = torch.ones(1, device=DEV)
+    print(f"ragged tiles M={M} N={N} K={K} bias={bias}", flush=True)
+    fp8_gemm(x8, w8, one, one, b, out=wide[:M, :N])
+    ref = x8.float() @ w8.float().t()               # |sums| <= 36 K: exact in fp32
+    if bias:
+        ref += b.float()
+    assert torch.equal(wide[:M, :N], ref.to(torch.bfloat16))
+    assert (wide[M] == 99).all() and (wide[:, N:] == 99).all()
+
+
 def test_static_linear_persistent_with_bias():
     M, N, K = 4096, 4096, 1024   # 16 x 16 tiles
     g = torch.Generator().manual_seed(11)
