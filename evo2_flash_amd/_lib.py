@@ -159,6 +159,16 @@ SIGNATURES = {
         _c_i64, _c_i64, _c_i64,                   # out strides (n, h, row)
         _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_f, _c_p,  # N, heads, L, Lv, head_dim, scale, stream
     ],
+    "evo2_bf16_stream_linear": [
+        _c_p, _c_i64, _c_p, _c_i64, _c_p,         # x, sx, w, sw, bias
+        _c_p, _c_i64, _c_p, _c_i64,               # residual, sr, out, so
+        _c_i64, _c_i64, _c_i64, _c_p,             # M, N, K, stream
+    ],
+    "evo2_bf16_stream_gated": [
+        _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i32,  # x, sx, w1, w2, sw, gelu
+        _c_p, _c_i64,                             # out, so
+        _c_i64, _c_i64, _c_i64, _c_p,             # M, N, K, stream
+    ],
     "evo2_rotary_prefill": [
         _c_p, _c_i64, _c_p, _c_f,                 # qkv, sqkv, inv_freq, factor
         _c_p, _c_p, _c_p, _c_i64,                 # q, k, vt, Lv

@@ -52,6 +52,7 @@ from .decode import channel_major_taps, hyena_decode
 from .fp8 import Fp8StaticLinear
 from .fp8_emul import static_fp8_linear_emulated
 from .hcl import hcl_block_t, hyena_hcl_prefill
+from .linear import linear
 from .metadata import decode_state_indices, longest_prefill_segment, prefill_tables
 from .prefill import fir_prefill_block_t, hyena_fir_prefill
 from .short_conv import PAD_SLOT_ID, causal_conv1d_update
@@ -76,7 +77,8 @@ ForwardContext = engine.ForwardContext
 # ---------------------------------------------------------------- projections
 class Linear(nn.Module):
     """Replicated bf16 linear with vLLM's `forward(x) -> (y, None)`; the GEMM
-    is the platform's library GEMM."""
+    is the weight-streaming kernel at decode batch sizes, else the platform's
+    library GEMM (linear.py)."""
 
     def __init__(self, in_features, out_features, bias=False, device=None, dtype=torch.bfloat16):
         super().__init__()
@@ -85,16 +87,10 @@ class Linear(nn.Module):
         self.bias = (nn.Parameter(torch.zeros(out_features, device=device, dtype=dtype),
                                   requires_grad=False) if bias else None)
 
-    def forward(self, x, out=None):
-        """x (..., in) -> ((..., out), None); a 2-D x may write its result into
-        `out` (the same GEMM F.linear runs: addmm with the bias)."""
-        if out is None:
-            return torch.nn.functional.linear(x, self.weight, self.bias), None
-        if self.bias is not None:
-            torch.addmm(self.bias, x, self.weight.t(), out=out)
-        else:
-            torch.mm(x, self.weight.t(), out=out)
-        return out, None
+    def forward(self, x, out=None, residual=None):
+        """x (..., in) -> ((..., out), None), plus `residual` when given; a 2-D x
+        may write its result into `out`."""
+        return linear(x, self.weight, self.bias, out, residual), None
 
 
 class ProjectionTap(nn.Module):

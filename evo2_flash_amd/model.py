@@ -31,6 +31,7 @@ from torch import nn
 from .attention import (PAGE, PagedKVCache, causal_prefill_attention, check_block_table,
                         paged_decode_attention, prefill_attention_rows, rotary_decode,
                         rotary_prefill, shared_prefix_pages, workspace as attention_workspace)
+from .linear import gated, linear
 from .metadata import build_metadata
 from .mixers import Linear, load_mixer_params, make_mixer, set_forward_context
 from .norm import Evo2RMSNorm
@@ -48,12 +49,10 @@ class Evo2MLP(nn.Module):
         self.l3 = Linear(inter, hidden, device=device)
         self.use_act = use_act
 
-    def forward(self, x):
-        z1, _ = self.l1(x)
-        z2, _ = self.l2(x)
-        if self.use_act:
-            z1 = nn.functional.gelu(z1)
-        out, _ = self.l3(z1 * z2)
+    def forward(self, x, residual=None):
+        """The MLP's output, plus `residual` (the layer's input) when given."""
+        z = gated(x, self.l1.weight, self.l2.weight, self.use_act)
+        out, _ = self.l3(z, residual=residual)
         return out
 
 
@@ -150,7 +149,7 @@ class Evo2DecoderLayer(nn.Module):
         else:
             m = self.mixer(pre, token_ids=token_ids)
         post, x = self.post_norm(m, x)
-        return self.mlp(post) + x
+        return self.mlp(post, residual=x)
 
     def forward_prefill(self, x, token_ids, nseq, L, block_table):
         """Prompts of L tokens of nseq sequences, packed (nseq * L, H); the
@@ -162,7 +161,7 @@ class Evo2DecoderLayer(nn.Module):
         else:
             m = self.mixer(pre, token_ids=token_ids)
         post, x = self.post_norm(m, x)
-        return self.mlp(post) + x
+        return self.mlp(post, residual=x)
 
 
 class Evo2DecodeModel(nn.Module):
@@ -284,7 +283,7 @@ class Evo2DecodeModel(nn.Module):
                     x = layer.forward_prefill(x, tok, n, L, self.block_table[b0:b0 + n])
             last.append(x.view(n, L, -1)[:, -1])
         h = self.norm(torch.cat(last))
-        return torch.nn.functional.linear(h, self.embed)
+        return linear(h, self.embed)
 
     def prefill_shared(self, prompt):
         """Prefill one prompt (L,) with L = shared_prefix into sequence 0 and
@@ -315,7 +314,7 @@ class Evo2DecodeModel(nn.Module):
             for layer in self.layers:
                 x = layer(positions, x, tokens, table)
         h = self.norm(x)
-        return torch.nn.functional.linear(h, self.embed)
+        return linear(h, self.embed)
 
     def hyena_params(self, i):
         """{parameter name: tensor} of Hyena layer i (checkpoint names)."""

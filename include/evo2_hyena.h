@@ -383,6 +383,26 @@ int evo2_prefill_attention_rows(const void *q, const void *k, const void *vt, vo
                                 int64_t head_dim, float scale, void *stream);
 
 /*
+ * bf16 projections of at most 16 rows (decode steps), fp32 sums:
+ *   _linear  out[m, n] = bf16(sum_k x[m, k] w[n, k] [+ bias[n]]), then with
+ *            residual (row stride sr) bf16(that + residual[m, n])
+ *   _gated   out = bf16(act(bf16(x w1^T)) * bf16(x w2^T)), act the exact GELU
+ *            (rounded to bf16) with gelu != 0, else the identity
+ *   x (M, K) row stride sx, w, w1, w2 (N, K) row stride sw, out (M, N) row
+ *   stride so, bias (N,), all bf16; K a multiple of 32, operand rows 16-byte
+ *   aligned.
+ *
+ * Serve out_proj (evo2_flash/mixers.py:801-803), the attention projections and
+ * the gated MLP (evo2_flash/model.py:77-153) at decode batch sizes.
+ */
+int evo2_bf16_stream_linear(const void *x, int64_t sx, const void *w, int64_t sw, const void *bias,
+                            const void *residual, int64_t sr, void *out, int64_t so, int64_t M,
+                            int64_t N, int64_t K, void *stream);
+int evo2_bf16_stream_gated(const void *x, int64_t sx, const void *w1, const void *w2, int64_t sw,
+                           int32_t gelu, void *out, int64_t so, int64_t M, int64_t N, int64_t K,
+                           void *stream);
+
+/*
  * Neox rotary of q and k with linear position scaling, and the write of k and
  * v into 16-position KV pages, from rows of a qkv projection (q | k | v, each
  * heads * head_dim bf16; row stride sqkv):

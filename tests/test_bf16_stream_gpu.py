@@ -1,0 +1,89 @@
+"""The weight-streaming bf16 projections of decode steps (csrc/bf16_stream.hip,
+linear.py) against 64-bit products: plain with bias and residual, and gated, at
+the edges of the kernel's tiles (1 to 16 rows, 16 weight rows a workgroup, eight
+parts of K in steps of 32), rows of wider matrices, and the calls that stay on
+the library (more rows, gradients, autocast).  Bound: one bf16 rounding per
+rounded step (2^-9 of its value) and fp32 sums of at most 11264 terms in any
+order (2^-16 of the sum of magnitudes)."""
+
+import pytest
+import torch
+
+from evo2_flash_amd import _lib
+from evo2_flash_amd.linear import gated, linear
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+bf = torch.bfloat16
+
+
+def _rand(*shape, seed, scale=1.0, pad=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    rows, cols = shape
+    return (torch.randn(rows, cols + pad, generator=g, device=DEV) * scale).to(bf)[:, :cols]
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (7, 37, 224), (8, 4096, 4096), (16, 513, 1920),
+                                   (3, 40, 288), (8, 48, 11264)])
+def test_linear_vs_fp64(M, N, K, monkeypatch):
+    x, w = _rand(M, K, seed=1, pad=8), _rand(N, K, seed=2, scale=0.05, pad=8)
+    b, r = _rand(1, N, seed=3)[0].contiguous(), _rand(M, N, seed=4, pad=(-N) % 8 + 8)
+    calls = []
+    call = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda n, *a: (calls.append(n), call(n, *a)))
+    print(f"bf16 stream M={M} N={N} K={K}", flush=True)
+    ref = x.double() @ w.double().t()
+    mag = x.double().abs() @ w.double().abs().t() * 2.0 ** -16
+    got = linear(x, w).double()
+    assert ((got - ref).abs() <= ref.abs() * 2.0 ** -8 + mag).all()
+    out = torch.full((M + 1, N), 7.0, dtype=bf, device=DEV)
+    assert linear(x, w, b, out=out[:M]).data_ptr() == out.data_ptr()
+    ref = ref + b.double()
+    assert ((out[:M].double() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag).all()
+    assert (out[M] == 7).all()
+    got = linear(x, w, b, residual=r).double()
+    sum_ = ref + r.double()
+    assert ((got - sum_).abs() <= (ref.abs() + sum_.abs()) * 2.0 ** -8 + mag).all()
+    assert calls == ["evo2_bf16_stream_linear"] * 3
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (16, 50, 1920), (8, 11264, 4096)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_gated_vs_fp64(M, N, K, gelu, monkeypatch):
+    x = _rand(M, K, seed=5)
+    w1, w2 = _rand(N, K, seed=6, scale=0.05), _rand(N, K, seed=7, scale=0.05)
+    calls = []
+    call = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda n, *a: (calls.append(n), call(n, *a)))
+    print(f"bf16 stream gated M={M} N={N} K={K} gelu={gelu}", flush=True)
+    got = gated(x, w1, w2, gelu).double()
+    z1, z2 = x.double() @ w1.double().t(), x.double() @ w2.double().t()
+    m1, m2 = ((x.double().abs() @ w.double().abs().t()) * 2.0 ** -16 + z.abs() * 2.0 ** -8
+              for w, z in ((w1, z1), (w2, z2)))
+    a = torch.nn.functional.gelu(z1) if gelu else z1
+    m1 = 1.13 * m1 + a.abs() * 2.0 ** -8               # |gelu'| <= 1.13, and its rounding
+    bound = m1 * (z2.abs() + m2) + a.abs() * m2 + (a * z2).abs() * 2.0 ** -8
+    assert ((got - a * z2).abs() <= bound).all()
+    assert calls == ["evo2_bf16_stream_gated"]
+
+
+def test_calls_that_stay_on_the_library(monkeypatch):
+    """More than 16 rows, a differentiated input, autocast, vmap and odd rows."""
+    w = _rand(64, 64, seed=8)
+    calls = []
+    monkeypatch.setattr(_lib, "call", lambda n, *a: calls.append(n))
+    F = torch.nn.functional.linear
+    x = _rand(17, 64, seed=9)
+    assert torch.equal(linear(x, w), F(x, w))
+    x = _rand(4, 64, seed=10).requires_grad_()
+    linear(x, w).float().sum().backward()
+    assert x.grad is not None
+    x = x.detach()
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert linear(x, w).dtype == torch.float16
+    xs = x.view(2, 2, 64)
+    assert torch.equal(torch.vmap(lambda t: linear(t, w))(xs), F(xs, w))
+    odd = _rand(4, 64, seed=11, pad=3)
+    assert torch.equal(linear(odd, w), F(odd, w))
+    assert linear(x.float(), w.float()).dtype == torch.float32
+    assert calls == []
