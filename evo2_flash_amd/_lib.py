@@ -236,6 +236,27 @@ SIGNATURES = {
         _c_p, _c_i64, _c_i64, _c_i64, _c_i64,     # y, ys0, nreq, T, H
         _c_i32, _c_i64, _c_p,                     # null_block, num_blocks, stream
     ],
+    "evo2_fir_verify_gated": [
+        _c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_i32, _c_p,  # zf, zs, w, w0, w1, K, D
+        _c_p, _c_i64, _c_i64, _c_i64,             # state + strides
+        _c_p, _c_i64, _c_i64,                     # ins + strides
+        _c_p, _c_i64, _c_i64, _c_i32,             # outs + strides, Q
+        _c_p, _c_p, _c_p,                         # starts, ends, accepted
+        _c_p, _c_i64,                             # g, gs
+        _c_i64, _c_i64, _c_i64,                   # nreq, T, H
+        _c_i32, _c_i64, _c_p,                     # null_block, num_blocks, stream
+    ],
+    "evo2_iir_verify_gated": [
+        _c_p, _c_i64, _c_p, _c_i64, _c_i64,       # zf, zs, log_poles + strides
+        _c_p, _c_i64, _c_i64, _c_p,               # residues + strides, D
+        _c_p, _c_i64, _c_i64, _c_i64,             # state + strides
+        _c_p, _c_i64, _c_i64,                     # ins + strides
+        _c_p, _c_i64, _c_i64, _c_i32,             # outs + strides, Q
+        _c_p, _c_p, _c_p,                         # starts, ends, accepted
+        _c_p, _c_i64,                             # g, gs
+        _c_i64, _c_i64, _c_i64,                   # nreq, T, H
+        _c_i32, _c_i64, _c_p,                     # null_block, num_blocks, stream
+    ],
     "evo2_spec_accepted": [
         _c_p, _c_i64, _c_i64,                     # stamps, stride, num_blocks
         _c_p, _c_i64, _c_p, _c_p,                 # slots, si0, computed, counts

@@ -200,18 +200,18 @@ __global__ __launch_bounds__(SC_CH) void conv_update_spec_kernel(SpecConvArgs p)
   const int c = blockIdx.x * SC_CH + threadIdx.x;
   const int r = blockIdx.y;
   if (c >= p.dim) return;
-  const int a = p.qsl[r], e = p.qsl[r + 1];
-  if (e <= a || a < 0 || e > p.T) return;
-  const int q = e - a;
+  const int a = p.qsl[r], e = min(p.qsl[r + 1], p.T);
+  if (e <= a || a < 0) return;
+  const int q = p.qsl[r + 1] - a;
   const int ic = p.in_col ? p.in_col[r] : 0, oc = p.out_col ? p.out_col[r] : 0;
   const int64_t in_slot = (ic >= 0 && ic < p.ncols) ? p.idx[(int64_t)r * p.si0 + (int64_t)ic * p.si1] : -1;
   const int64_t out_slot = (oc >= 0 && oc < p.ncols) ? p.idx[(int64_t)r * p.si0 + (int64_t)oc * p.si1] : -1;
   const int64_t acc_n = p.accepted[r];
   const int keep = p.state_len - p.max_q;
   // requests the convention cannot place: a padding or out-of-range slot,
-  // more rows than the verifier has positions, or an accepted count past the
-  // window; their rows are zero and no state is touched
-  const bool ok = q <= p.max_q && acc_n >= 1 && acc_n <= p.max_q &&
+  // rows past x, more rows than the verifier has positions, or an accepted
+  // count past the window; their rows are zero and no state is touched
+  const bool ok = q == e - a && q <= p.max_q && acc_n >= 1 && acc_n <= p.max_q &&
                   in_slot != p.pad_slot && in_slot >= 0 && in_slot < p.num_blocks &&
                   out_slot != p.pad_slot && out_slot >= 0 && out_slot < p.num_blocks;
   if (!ok) {

@@ -25,6 +25,14 @@
 // pieces of the same columns.  A destination equal to the null block, or outside the
 // pool, is not written (the reference skips block 0, line 80); a source
 // outside the pool reads as a zero state.
+//
+// Gated form (GATE): the whole inner half of a mixer's verify step.  x is the
+// short filter's output, rows of (x2, x1, v) triples; the operator's input is
+// u = bf16(x1 v), and what is stored is x2 * (y [+ D u]), rounded to bf16 after
+// every step as the separate operators round it (mixers.py:1264-1298,
+// 1366-1398).  As elementwise operators around the snapshots this was up to
+// five launches a layer of ~4.8 us each; the snapshot kernels are bound by their
+// stores and the rest is a few bytes a token beside them.
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -44,6 +52,9 @@ struct VerifyArgs {
   void *y; int64_t ys0;                   // (T, H) output, x's dtype
   int Q, H, null_block;
   int64_t num_blocks, T;
+  // gated form
+  const bf16_t *D;                        // (H,) or null
+  int poles_log;                          // poles holds log_poles
 };
 
 // Request r's token range, source block and whether it reads a real block.
@@ -78,15 +89,30 @@ __device__ __forceinline__ int64_t dest_of(const VerifyArgs &a, int64_t r, int p
   return (d == a.null_block || d < 0 || d >= a.num_blocks) ? -1 : d;
 }
 
+template <bool GATE>
 __device__ __forceinline__ float load_x(const VerifyArgs &a, int64_t t, int c) {
+  if constexpr (GATE) {  // u = x1 v
+    const bf16_t *z = static_cast<const bf16_t *>(a.x) + t * a.xs0 + 3 * (int64_t)c;
+    return rbf(bf2f(z[1]) * bf2f(z[2]));
+  }
   const int64_t off = t * a.xs0 + (int64_t)c * a.xs1;
   return a.x_f32 ? static_cast<const float *>(a.x)[off] : bf2f(static_cast<const bf16_t *>(a.x)[off]);
 }
 
-__device__ __forceinline__ void store_y(const VerifyArgs &a, int64_t t, int c, float v) {
+// u: the token's input (the gated form's skip term)
+template <bool GATE>
+__device__ __forceinline__ void store_y(const VerifyArgs &a, int64_t t, int c, float v, float u) {
   const int64_t off = t * a.ys0 + c;
-  if (a.x_f32) static_cast<float *>(a.y)[off] = v;
-  else static_cast<bf16_t *>(a.y)[off] = f2bf(v);
+  if constexpr (GATE) {
+    v = rbf(v);
+    if (a.D) v = rbf(v + rbf(bf2f(a.D[c]) * u));
+    const float x2 = bf2f(static_cast<const bf16_t *>(a.x)[t * a.xs0 + 3 * (int64_t)c]);
+    static_cast<bf16_t *>(a.y)[off] = f2bf(x2 * v);
+  } else if (a.x_f32) {
+    static_cast<float *>(a.y)[off] = v;
+  } else {
+    static_cast<bf16_t *>(a.y)[off] = f2bf(v);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -116,7 +142,7 @@ __device__ __forceinline__ void store_y(const VerifyArgs &a, int64_t t, int c, f
 // the stores and the taps first (one process; all bitwise equal).
 constexpr int VQ = 16;
 
-template <int CPW>
+template <int CPW, bool GATE>
 __global__ __launch_bounds__(4 * CPW, 4) void fir128_verify_kernel(VerifyArgs a) {
   static_assert(CPW == 64 || CPW == 128, "one channel or one channel pair per lane");
   constexpr int CPL = CPW / 64;  // channels per lane in the copies
@@ -165,7 +191,7 @@ __global__ __launch_bounds__(4 * CPW, 4) void fir128_verify_kernel(VerifyArgs a)
   }
   for (int p = m; p < n; p += NW)
 #pragma unroll
-    for (int i = 0; i < CPL; ++i) e[127 + p][CPL * lane + i] = cact ? load_x(a, q.first + p, cl + i) : 0.0f;
+    for (int i = 0; i < CPL; ++i) e[127 + p][CPL * lane + i] = cact ? load_x<GATE>(a, q.first + p, cl + i) : 0.0f;
   __syncthreads();
 
   if (p0 < n) {  // uniform
@@ -198,7 +224,7 @@ __global__ __launch_bounds__(4 * CPW, 4) void fir128_verify_kernel(VerifyArgs a)
 #pragma unroll
       for (int l = 0; l < 4; ++l) pl[l] = ((acc[0][l] + acc[1][l]) + acc[2][l]) + acc[3][l];
       const float yv = ((pl[0] + pl[2]) + (pl[1] + pl[3])) + last * e[127 + p][hc];
-      if (active) store_y(a, q.first + p, c, yv);
+      if (active) store_y<GATE>(a, q.first + p, c, yv, e[127 + p][hc]);
     }
   }
 
@@ -228,6 +254,7 @@ __global__ __launch_bounds__(4 * CPW, 4) void fir128_verify_kernel(VerifyArgs a)
 // their four partials to wave 0 through LDS, which combines them in the
 // reference's order.  After each token every wave writes a quarter of the
 // new window to the destination snapshot.
+template <bool GATE>
 __global__ __launch_bounds__(256) void fir128_verify_serial_kernel(VerifyArgs a) {
   __shared__ float ring[128][64];
   __shared__ float part[3][4][64];
@@ -256,7 +283,7 @@ __global__ __launch_bounds__(256) void fir128_verify_serial_kernel(VerifyArgs a)
   for (int pos = 0; pos < a.Q; ++pos) {
     if (q.first + pos >= q.end) break;  // uniform; positions are consecutive
     const int64_t t = q.first + pos;
-    const float x = active ? load_x(a, t, c) : 0.0f;
+    const float x = active ? load_x<GATE>(a, t, c) : 0.0f;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -277,7 +304,7 @@ __global__ __launch_bounds__(256) void fir128_verify_serial_kernel(VerifyArgs a)
       for (int l = 0; l < 4; ++l)
         p[l] = ((acc[l] + part[0][l][lane]) + part[1][l][lane]) + part[2][l][lane];
       const float yv = ((p[0] + p[2]) + (p[1] + p[3])) + last * x;
-      if (active) store_y(a, t, c, yv);
+      if (active) store_y<GATE>(a, t, c, yv, x);
       ring[(pos + 127) & 127][lane] = x;  // the dropped column's slot
     }
     __syncthreads();  // appended token visible; partials consumed
@@ -291,6 +318,7 @@ __global__ __launch_bounds__(256) void fir128_verify_serial_kernel(VerifyArgs a)
 
 // ---------------------------------------------------------------------------
 // K = 7: one channel per thread, the 6-column window in registers.
+template <bool GATE>
 __global__ __launch_bounds__(256) void fir7_verify_kernel(VerifyArgs a) {
   const int64_t r = blockIdx.y;
   const int c = blockIdx.x * 256 + threadIdx.x;
@@ -307,20 +335,20 @@ __global__ __launch_bounds__(256) void fir7_verify_kernel(VerifyArgs a) {
   const int n = static_cast<int>(max<int64_t>(0, min<int64_t>(a.Q, q.end - q.first)));
   float xs[VQ];
 #pragma unroll
-  for (int i = 0; i < VQ; ++i) xs[i] = i < n ? load_x(a, q.first + i, c) : 0.0f;
+  for (int i = 0; i < VQ; ++i) xs[i] = i < n ? load_x<GATE>(a, q.first + i, c) : 0.0f;
   for (int pos = 0; pos < n; ++pos) {
     const int64_t t = q.first + pos;
     float x = 0.0f;
 #pragma unroll
     for (int i = 0; i < VQ; ++i) x = i == pos ? xs[i] : x;
-    if (pos >= VQ) x = load_x(a, t, c);
+    if (pos >= VQ) x = load_x<GATE>(a, t, c);
     // ((p0 + p4) + (p1 + p5) + p2) + p3 (triton_verifier.py:35-43)
     float pa = s[0] * w[0], pb = s[1] * w[1];
     const float pc = s[2] * w[2], pd = s[3] * w[3];
     pa = pa + s[4] * w[4];
     pb = pb + s[5] * w[5];
     const float yv = (((pa + pb) + pc) + pd) + w[6] * x;
-    store_y(a, t, c, yv);
+    store_y<GATE>(a, t, c, yv, x);
 #pragma unroll
     for (int k = 0; k < 5; ++k) s[k] = s[k + 1];
     s[5] = x;
@@ -345,7 +373,7 @@ __device__ __forceinline__ float quad_move(float v) {
 // VEC: the state rows are 16 contiguous, 16-byte aligned fp32 (one float4 per
 // lane); otherwise each lane moves its four states one by one (a row of the
 // speculative layout is 17 fp32, its last column the position stamp).
-template <bool VEC>
+template <bool VEC, bool GATE>
 __global__ __launch_bounds__(256) void iir_verify_kernel(VerifyArgs a) {
   const int lane = threadIdx.x & 63;
   const int qd = lane & 3;
@@ -356,7 +384,11 @@ __global__ __launch_bounds__(256) void iir_verify_kernel(VerifyArgs a) {
   const Req q = request_of(a, r);
   const float4 p4 = *reinterpret_cast<const float4 *>(a.poles + (int64_t)cc * a.p0 + 4 * qd);
   const float4 r4 = *reinterpret_cast<const float4 *>(a.res + (int64_t)cc * a.r0 + 4 * qd);
-  const float pv[4] = {p4.x, p4.y, p4.z, p4.w};
+  float pv[4] = {p4.x, p4.y, p4.z, p4.w};
+  if (GATE && a.poles_log) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) pv[e] = expf(pv[e]);
+  }
   const float rv[4] = {r4.x, r4.y, r4.z, r4.w};
   float sv[4] = {0.f, 0.f, 0.f, 0.f};
   if (q.src_ok) {
@@ -373,13 +405,13 @@ __global__ __launch_bounds__(256) void iir_verify_kernel(VerifyArgs a) {
   const int n = static_cast<int>(max<int64_t>(0, min<int64_t>(a.Q, q.end - q.first)));
   float xs[VQ];
 #pragma unroll
-  for (int i = 0; i < VQ; ++i) xs[i] = i < n ? load_x(a, q.first + i, cc) : 0.0f;
+  for (int i = 0; i < VQ; ++i) xs[i] = i < n ? load_x<GATE>(a, q.first + i, cc) : 0.0f;
   for (int pos = 0; pos < n; ++pos) {  // uniform
     const int64_t t = q.first + pos;
     float x = 0.0f;
 #pragma unroll
     for (int i = 0; i < VQ; ++i) x = i == pos ? xs[i] : x;
-    if (pos >= VQ) x = load_x(a, t, cc);
+    if (pos >= VQ) x = load_x<GATE>(a, t, cc);
     float rr[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -403,7 +435,7 @@ __global__ __launch_bounds__(256) void iir_verify_kernel(VerifyArgs a) {
     rr[0] = rr[0] + rr[2];                                                   // += state + 2
     rr[1] = rr[1] + rr[3];
     const float yv = rr[0] + rr[1];                                          // += state + 1
-    if (qd == 0 && active) store_y(a, t, c, yv);
+    if (qd == 0 && active) store_y<GATE>(a, t, c, yv, x);
   }
 }
 
@@ -429,6 +461,40 @@ static int verify_common(const char *who, const void *x, int64_t nreq, int64_t T
   return EVO2_OK;
 }
 
+template <bool GATE>
+static int launch_fir(const VerifyArgs &a, int K, int64_t nreq, hipStream_t st) {
+  if (K == 128) {
+    // channel pairs move as 8-byte words when the state's channels are
+    // unit-stride and every pair starts 8-byte aligned
+    const bool pairs = a.ss1 == 1 && a.H % 2 == 0 && a.ss0 % 2 == 0 && a.ss2 % 2 == 0 &&
+                       (reinterpret_cast<uintptr_t>(a.st) & 7) == 0;
+    if (a.Q <= VQ && pairs) {
+      dim3 grid(static_cast<unsigned>(cdiv(a.H, 128)), static_cast<unsigned>(nreq));
+      hipLaunchKernelGGL((fir128_verify_kernel<128, GATE>), grid, dim3(512), 0, st, a);
+    } else {
+      dim3 grid(static_cast<unsigned>(cdiv(a.H, 64)), static_cast<unsigned>(nreq));
+      if (a.Q <= VQ)
+        hipLaunchKernelGGL((fir128_verify_kernel<64, GATE>), grid, dim3(256), 0, st, a);
+      else
+        hipLaunchKernelGGL(fir128_verify_serial_kernel<GATE>, grid, dim3(256), 0, st, a);
+    }
+  } else {
+    dim3 grid(static_cast<unsigned>(cdiv(a.H, 256)), static_cast<unsigned>(nreq));
+    hipLaunchKernelGGL(fir7_verify_kernel<GATE>, grid, dim3(256), 0, st, a);
+  }
+  return check_launch("fir_verify");
+}
+
+template <bool GATE>
+static int launch_iir(const VerifyArgs &a, int64_t nreq, hipStream_t st) {
+  const bool vec = a.ss2 == 1 && a.ss1 % 4 == 0 && a.ss0 % 4 == 0 &&
+                   reinterpret_cast<uintptr_t>(a.st) % 16 == 0;
+  dim3 grid(static_cast<unsigned>(cdiv(a.H, 64)), static_cast<unsigned>(nreq));
+  if (vec) hipLaunchKernelGGL((iir_verify_kernel<true, GATE>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((iir_verify_kernel<false, GATE>), grid, dim3(256), 0, st, a);
+  return check_launch("iir_verify");
+}
+
 extern "C" int evo2_fir_verify(const void *x, int64_t xs0, int64_t xs1, int32_t x_f32,
                                const void *w, int64_t w0, int64_t w1, int32_t K,
                                float *state, int64_t ss0, int64_t ss1, int64_t ss2,
@@ -448,27 +514,7 @@ extern "C" int evo2_fir_verify(const void *x, int64_t xs0, int64_t xs1, int32_t 
   VerifyArgs a{x, xs0, xs1, x_f32, static_cast<const bf16_t *>(w), w0, w1, nullptr, 0, 0,
                nullptr, 0, 0, state, ss0, ss1, ss2, ins, is0, is1, outs, os0, os1,
                starts, ends, accepted, y, ys0, Q, static_cast<int>(H), null_block, num_blocks, T};
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (K == 128) {
-    // channel pairs move as 8-byte words when the state's channels are
-    // unit-stride and every pair starts 8-byte aligned
-    const bool pairs = ss1 == 1 && H % 2 == 0 && ss0 % 2 == 0 && ss2 % 2 == 0 &&
-                       (reinterpret_cast<uintptr_t>(state) & 7) == 0;
-    if (Q <= VQ && pairs) {
-      dim3 grid(static_cast<unsigned>(cdiv(H, 128)), static_cast<unsigned>(nreq));
-      hipLaunchKernelGGL(fir128_verify_kernel<128>, grid, dim3(512), 0, st, a);
-    } else {
-      dim3 grid(static_cast<unsigned>(cdiv(H, 64)), static_cast<unsigned>(nreq));
-      if (Q <= VQ)
-        hipLaunchKernelGGL(fir128_verify_kernel<64>, grid, dim3(256), 0, st, a);
-      else
-        hipLaunchKernelGGL(fir128_verify_serial_kernel, grid, dim3(256), 0, st, a);
-    }
-  } else {
-    dim3 grid(static_cast<unsigned>(cdiv(H, 256)), static_cast<unsigned>(nreq));
-    hipLaunchKernelGGL(fir7_verify_kernel, grid, dim3(256), 0, st, a);
-  }
-  return check_launch("fir_verify");
+  return launch_fir<false>(a, K, nreq, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int evo2_iir_verify(const void *x, int64_t xs0, int64_t xs1, int32_t x_f32,
@@ -490,15 +536,57 @@ extern "C" int evo2_iir_verify(const void *x, int64_t xs0, int64_t xs1, int32_t 
     return fail(EVO2_ERR_UNSUPPORTED,
                 "iir_verify: poles and residues need 16 contiguous, 16-byte aligned fp32 per "
                 "channel");
-  const bool vec = ss2 == 1 && ss1 % 4 == 0 && ss0 % 4 == 0 &&
-                   reinterpret_cast<uintptr_t>(state) % 16 == 0;
   if (nreq == 0) return EVO2_OK;
   VerifyArgs a{x, xs0, xs1, x_f32, nullptr, 0, 0, poles, p0, p1, residues, r0, r1,
                state, ss0, ss1, ss2, ins, is0, is1, outs, os0, os1,
                starts, ends, accepted, y, ys0, Q, static_cast<int>(H), null_block, num_blocks, T};
-  dim3 grid(static_cast<unsigned>(cdiv(H, 64)), static_cast<unsigned>(nreq));
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (vec) hipLaunchKernelGGL(iir_verify_kernel<true>, grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(iir_verify_kernel<false>, grid, dim3(256), 0, st, a);
-  return check_launch("iir_verify");
+  return launch_iir<false>(a, nreq, static_cast<hipStream_t>(stream));
+}
+
+// The gated forms: as above with zf (T, 3H) bf16 in place of x.
+extern "C" int evo2_fir_verify_gated(const void *zf, int64_t zs, const void *w, int64_t w0, int64_t w1,
+                                     int32_t K, const void *D, float *state, int64_t ss0, int64_t ss1,
+                                     int64_t ss2, const int32_t *ins, int64_t is0, int64_t is1,
+                                     const int32_t *outs, int64_t os0, int64_t os1, int32_t Q,
+                                     const int64_t *starts, const int64_t *ends,
+                                     const int64_t *accepted, void *g, int64_t gs, int64_t nreq,
+                                     int64_t T, int64_t H, int32_t null_block, int64_t num_blocks,
+                                     void *stream) {
+  int rc = verify_common("fir_verify_gated", zf, nreq, T, H, Q, ins, outs, starts, ends, accepted, g, state,
+                         num_blocks);
+  if (rc) return rc;
+  if (K != 7 && K != 128)
+    return fail(EVO2_ERR_UNSUPPORTED, "fir_verify_gated: filter length %d (7 or 128 only)", K);
+  if (!w) return fail(EVO2_ERR_INVALID, "fir_verify_gated: null pointer argument");
+  if (nreq == 0) return EVO2_OK;
+  VerifyArgs a{zf, zs, 1, 0, static_cast<const bf16_t *>(w), w0, w1, nullptr, 0, 0,
+               nullptr, 0, 0, state, ss0, ss1, ss2, ins, is0, is1, outs, os0, os1,
+               starts, ends, accepted, g, gs, Q, static_cast<int>(H), null_block, num_blocks, T,
+               static_cast<const bf16_t *>(D), 0};
+  return launch_fir<true>(a, K, nreq, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int evo2_iir_verify_gated(const void *zf, int64_t zs, const float *log_poles, int64_t p0, int64_t p1,
+                                     const float *residues, int64_t r0, int64_t r1, const void *D,
+                                     float *state, int64_t ss0, int64_t ss1, int64_t ss2,
+                                     const int32_t *ins, int64_t is0, int64_t is1, const int32_t *outs,
+                                     int64_t os0, int64_t os1, int32_t Q, const int64_t *starts,
+                                     const int64_t *ends, const int64_t *accepted, void *g, int64_t gs,
+                                     int64_t nreq, int64_t T, int64_t H, int32_t null_block,
+                                     int64_t num_blocks, void *stream) {
+  int rc = verify_common("iir_verify_gated", zf, nreq, T, H, Q, ins, outs, starts, ends, accepted, g, state,
+                         num_blocks);
+  if (rc) return rc;
+  if (!log_poles || !residues) return fail(EVO2_ERR_INVALID, "iir_verify_gated: null pointer argument");
+  if (p1 != 1 || r1 != 1 || p0 % 4 || r0 % 4 || reinterpret_cast<uintptr_t>(log_poles) % 16 ||
+      reinterpret_cast<uintptr_t>(residues) % 16)
+    return fail(EVO2_ERR_UNSUPPORTED,
+                "iir_verify_gated: poles and residues need 16 contiguous, 16-byte aligned fp32 per "
+                "channel");
+  if (nreq == 0) return EVO2_OK;
+  VerifyArgs a{zf, zs, 1, 0, nullptr, 0, 0, log_poles, p0, p1, residues, r0, r1,
+               state, ss0, ss1, ss2, ins, is0, is1, outs, os0, os1,
+               starts, ends, accepted, g, gs, Q, static_cast<int>(H), null_block, num_blocks, T,
+               static_cast<const bf16_t *>(D), 1};
+  return launch_iir<true>(a, nreq, static_cast<hipStream_t>(stream));
 }

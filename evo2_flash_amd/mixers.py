@@ -29,10 +29,10 @@ Speculative decode (`num_spec` > 0 draft tokens, mixers.py:17-35, 952-1074):
 a step whose metadata is speculative by the reference's predicate
 (mixers.py:930-937) runs its decode rows as
 
-  decode rows   in_proj -> causal_conv1d_update (speculative form: the
-                widened window in column 0 of each request's slot row) ->
-                u = x1*v -> fir_snapshots | iir_snapshots (one snapshot per
-                verifier position) -> [+ D*u] -> x2*y -> out_proj
+  decode rows   in_proj -> the speculative short conv (the widened window in
+                column 0 of each request's slot row) -> fir_verify_gated |
+                iir_verify_gated (u = x1*v, one snapshot per verifier
+                position, [+ D*u], x2*y) -> out_proj
 
 with the live snapshot of each request resolved from the position stamps in
 slice 2 before any state is written, and every snapshot written in the step
@@ -55,11 +55,11 @@ from .hcl import hcl_block_t, hyena_hcl_prefill
 from .linear import linear
 from .metadata import decode_state_indices, longest_prefill_segment, prefill_tables
 from .prefill import fir_prefill_block_t, hyena_fir_prefill
-from .short_conv import PAD_SLOT_ID, causal_conv1d_update
+from .short_conv import PAD_SLOT_ID, _update_spec as conv_update_spec
 from .speculative import (packed_rows, pool_holds, record_stamps, repair_prefill_states,
                           slot_matrix, spec_accepted, verify_plan)
 from .state import unified_state_dtype, unified_state_shape
-from .verify import fir_snapshots, iir_snapshots
+from .verify import fir_verify_gated, iir_verify_gated
 
 # Test-only cross-check (mixers.py:77, 989-998): where the engine does send
 # acceptance counts, they must agree with the stamps.
@@ -330,8 +330,9 @@ class HyenaMixerBase(nn.Module):
                       m.seq_lens[nd:nd + npf] if npf else None)
 
     def _spec_short_conv(self, z_d, m, accepted):
-        """(x2, x1, v) of the decode rows of a speculative step through the
-        widened short window (mixers.py:1153-1193)."""
+        """The (x2, x1, v) triples of a speculative step's decode rows through
+        the widened short window (mixers.py:1153-1193); rows outside every
+        request are unset."""
         window = self._conv_state(0)
         n = int(m.num_decodes)
         engine_rows = m.state_indices_tensor_d
@@ -342,16 +343,13 @@ class HyenaMixerBase(nn.Module):
         comp = getattr(m, "block_idx_last_computed_token", None)
         if accepted is None:
             accepted = self._verify_plan(m).engine_accepted
-        zf = causal_conv1d_update(
-            z_d, window, self._short_w(), None, activation=None,
-            conv_state_indices=rows[:n],
-            block_idx_last_scheduled_token=None if sched is None else sched[:n],
-            initial_state_idx=None if comp is None else comp[:n],
-            num_accepted_tokens=accepted, query_start_loc=packed_rows(m, n, z_d.device),
-            max_query_len=rows.shape[1], pad_slot_id=PAD_SLOT_ID)
-        return zf[:, 0::3], zf[:, 1::3], zf[:, 2::3]
+        return conv_update_spec(
+            z_d, window, self._short_w(), None, 0, rows[:n], accepted,
+            packed_rows(m, n, z_d.device), rows.shape[1], PAD_SLOT_ID,
+            None if sched is None else sched[:n], None if comp is None else comp[:n],
+            zero_rows=False)
 
-    def _spec_tensors(self, m, num_tokens, state, accepted):
+    def _spec_tensors(self, m, state, accepted):
         """(ins, outs, starts, ends, accepted) for the inner operator's
         snapshots (mixers.py:578-598); `accepted` is the stamp-derived count,
         or the engine's when there is none."""
@@ -435,14 +433,9 @@ class HyenaFIRMixer(HyenaMixerBase):
     def _spec_decode(self, z_d, m, accepted, inner_state):
         """g = x2 * (FIR(u) [+ D*u]) for the decode rows of a speculative step,
         one inner snapshot per verifier position (mixers.py:1264-1275, 1286-1298)."""
-        x2, x1, v = self._spec_short_conv(z_d, m, accepted)
-        u = x1 * v
-        w = self.conv.view(self.hidden, self.k_inner)
-        y = fir_snapshots(u, w, inner_state,
-                          self._spec_tensors(m, u.shape[0], inner_state, accepted))
-        if self.has_D:
-            y = y + self.D.to(y.dtype) * u
-        return x2 * y
+        zf = self._spec_short_conv(z_d, m, accepted)
+        return fir_verify_gated(zf, self.conv.view(self.hidden, self.k_inner), self.D, inner_state,
+                                self._spec_tensors(m, inner_state, accepted))
 
     def _forward_impl(self, hidden_states, token_ids=None, output=None):
         m = self._meta()
@@ -505,11 +498,8 @@ class HyenaIIRMixer(HyenaMixerBase):
     def _spec_decode(self, z_d, m, accepted, ssm, lp, res):
         """g = x2 * (LI(u) + u*D) for the decode rows of a speculative step, one
         state snapshot per verifier position (mixers.py:1366-1378, 1396)."""
-        x2, x1, v = self._spec_short_conv(z_d, m, accepted)
-        x1v = x1 * v
-        y = iir_snapshots(x1v, torch.exp(lp), res, ssm,
-                          self._spec_tensors(m, x1v.shape[0], ssm, accepted))
-        return (y + x1v * self.D.to(y.dtype)) * x2
+        zf = self._spec_short_conv(z_d, m, accepted)
+        return iir_verify_gated(zf, lp, res, self.D, ssm, self._spec_tensors(m, ssm, accepted))
 
     def _forward_impl(self, hidden_states, token_ids=None, output=None):
         m = self._meta()

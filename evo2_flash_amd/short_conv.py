@@ -73,8 +73,9 @@ def _index_table(idx, n, fn, name):
 
 
 def _update_spec(x, conv_state, weight, bias, act, conv_state_indices, num_accepted_tokens,
-                 query_start_loc, max_query_len, pad_slot_id, out_col, in_col):
-    """The speculative varlen form (see `causal_conv1d_update`)."""
+                 query_start_loc, max_query_len, pad_slot_id, out_col, in_col, zero_rows=True):
+    """The speculative varlen form (see `causal_conv1d_update`); zero_rows:
+    rows outside every request are zero, else they are left unset."""
     fn = "causal_conv1d_update"
     if query_start_loc is None or x.dim() != 2:
         raise NotImplementedError(f"{fn}: the speculative form takes packed rows x (T, dim) "
@@ -109,7 +110,8 @@ def _update_spec(x, conv_state, weight, bias, act, conv_state_indices, num_accep
             c = c[:nreq].to(torch.int32).contiguous()
         cols.append(c)
     T = x.shape[0]
-    out = torch.zeros(T, dim, dtype=torch.bfloat16, device=x.device)
+    out = (torch.zeros if zero_rows else torch.empty)(T, dim, dtype=torch.bfloat16,
+                                                      device=x.device)
     _lib.call("evo2_causal_conv1d_update_spec",
               _lib.ptr(x), x.stride(0), x.stride(1),
               _lib.ptr(conv_state), *conv_state.stride(), state_len,

@@ -141,6 +141,46 @@ def iir_snapshots(x, poles, residues, state, metadata, null_block=0):
                 null_block)
 
 
+def _gated_args(zf, state, D, metadata):
+    """Checks of the gated calls; (D, g, the arguments both share)."""
+    ins, outs, starts, ends, accepted = meta = _meta(metadata)
+    _lib.require_device(zf, state, D, *meta)
+    H = state.shape[1]
+    if zf.dim() != 2 or zf.shape[1] != 3 * H or zf.dtype != torch.bfloat16 or zf.stride(1) != 1:
+        raise ValueError(f"zf must be (T, {3 * H}) bf16 rows, got {tuple(zf.shape)} {zf.dtype}")
+    if D is not None:
+        D = D.to(torch.bfloat16).contiguous()
+    g = torch.zeros(zf.shape[0], H, dtype=zf.dtype, device=zf.device)
+    return D, g, meta, (_lib.ptr(state), *state.stride(), _lib.ptr(ins), *ins.stride(),
+                        _lib.ptr(outs), *outs.stride(), outs.shape[1], _lib.ptr(starts),
+                        _lib.ptr(ends), _lib.ptr(accepted), _lib.ptr(g), g.stride(0),
+                        ins.shape[0], zf.shape[0], H)
+
+
+def fir_verify_gated(zf, weight, D, state, metadata, null_block=0):
+    """x2 * (FIR(x1 v) [+ D x1 v]) over each request's rows of the short filter's
+    output zf (T, 3H), one window snapshot per token, in one launch:
+    fir_snapshots with the gate around it, each step rounded to bf16; (T, H),
+    zero on rows no request covers."""
+    _lib.require_device(weight)
+    D, g, _keep, args = _gated_args(zf, state, D, metadata)
+    _lib.call("evo2_fir_verify_gated", _lib.ptr(zf), zf.stride(0), _lib.ptr(weight),
+              *weight.stride(), weight.shape[1], _lib.ptr(D), *args, int(null_block),
+              _blocks(state), _lib.stream_of(zf))
+    return g
+
+
+def iir_verify_gated(zf, log_poles, residues, D, state, metadata, null_block=0):
+    """(LI(x1 v) + D x1 v) * x2 in one launch (fir_verify_gated's form of
+    iir_snapshots; poles exp(log_poles) taken in the kernel)."""
+    _lib.require_device(log_poles, residues)
+    D, g, _keep, args = _gated_args(zf, state, D, metadata)
+    _lib.call("evo2_iir_verify_gated", _lib.ptr(zf), zf.stride(0),
+              _lib.ptr(log_poles), *log_poles.stride(), _lib.ptr(residues), *residues.stride(),
+              _lib.ptr(D), *args, int(null_block), _blocks(state), _lib.stream_of(zf))
+    return g
+
+
 def fir_one(x, weight, state, slots, null_block=0):
     """One token per request: row r reads and rewrites block slots[r]
     (triton_verifier.py:157-167)."""

@@ -383,6 +383,33 @@ int evo2_prefill_attention_rows(const void *q, const void *k, const void *vt, vo
                                 int64_t head_dim, float scale, void *stream);
 
 /*
+ * evo2_fir_verify / evo2_iir_verify with the rest of a mixer's verify step
+ * around them, one launch:
+ *   zf (T, 3H) bf16 rows of (x2, x1, v) triples, row stride zs;
+ *   u = bf16(x1 v) is the operator's input, and
+ *   g[t] = bf16(x2 * bf16(y [+ bf16(D u)])) its output, bf16 (T, H), row stride
+ *   gs (rows no request covers are not written);
+ * D (H,) bf16 or null; the LI form takes log_poles.
+ *
+ * Replace the speculative decode branch of the mixers after the short filter
+ * (evo2_flash/mixers.py:1264-1298, 1366-1398).
+ */
+int evo2_fir_verify_gated(const void *zf, int64_t zs, const void *w, int64_t w0, int64_t w1, int32_t K,
+                          const void *D, float *state, int64_t ss0, int64_t ss1, int64_t ss2,
+                          const int32_t *ins, int64_t is0, int64_t is1, const int32_t *outs,
+                          int64_t os0, int64_t os1, int32_t Q, const int64_t *starts,
+                          const int64_t *ends, const int64_t *accepted, void *g, int64_t gs,
+                          int64_t nreq, int64_t T, int64_t H, int32_t null_block,
+                          int64_t num_blocks, void *stream);
+int evo2_iir_verify_gated(const void *zf, int64_t zs, const float *log_poles, int64_t p0, int64_t p1,
+                          const float *residues, int64_t r0, int64_t r1, const void *D, float *state,
+                          int64_t ss0, int64_t ss1, int64_t ss2, const int32_t *ins, int64_t is0,
+                          int64_t is1, const int32_t *outs, int64_t os0, int64_t os1, int32_t Q,
+                          const int64_t *starts, const int64_t *ends, const int64_t *accepted, void *g,
+                          int64_t gs, int64_t nreq, int64_t T, int64_t H, int32_t null_block, int64_t num_blocks,
+                          void *stream);
+
+/*
  * bf16 projections of at most 16 rows (decode steps), fp32 sums:
  *   _linear  out[m, n] = bf16(sum_k x[m, k] w[n, k] [+ bias[n]]), then with
  *            residual (row stride sr) bf16(that + residual[m, n])

@@ -142,3 +142,47 @@ def test_long_requests_bitwise(kind):
         ref = oracle.fir_verify_emulated(x, w, st, *meta)
         assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
     assert torch.equal(gst.cpu(), st)
+
+
+@pytest.mark.parametrize("kind", ["hcs", "hcm", "hcl"])
+@pytest.mark.parametrize("H,Q", [(256, 4), (193, 4), (192, 19)])
+def test_gated_forms_bitwise(kind, H, Q):
+    """The one-launch verify step (gate and D around the snapshots) against the
+    separate operators: outputs and states bit for bit,
+    with rows outside every request (before, between and after), a request of
+    no rows, part-filled channel blocks and requests longer than the kernels
+    stage at once.  H = 193: FIR kinds' one-channel-per-lane form."""
+    from evo2_flash_amd.verify import fir_verify_gated, iir_verify_gated
+    nreq = 6
+    nblk = 2 * nreq * Q + 2
+    prm, x, state, meta = verify_case(kind, H, nreq, Q, nblk, seed=H + Q)
+    ins, outs, starts, ends, accepted = (t.clone() for t in meta)
+    starts, ends = starts + 2, ends + 2                  # two rows before the first request
+    ends[2] = starts[2]                                  # a request of no rows: its rows uncovered
+    T = int(ends[-1]) + 3
+    meta = (ins, outs, starts, ends, accepted)
+    g = torch.Generator().manual_seed(H)
+    zf = torch.randn(T, 3 * H + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :3 * H]
+    x2, u = zf[:, 0::3], (zf[:, 1::3] * zf[:, 2::3]).contiguous()
+    md = _meta_dev(meta, False)
+    D = prm["D"].to(DEV) if "D" in prm else None
+    print(f"gated verify {kind} H={H} Q={Q}", flush=True)
+    if kind == "hcl":
+        lp, res = prm["log_poles"][..., 0].contiguous().to(DEV), prm["residues"].to(DEV)
+        a, b = state.to(DEV), state.to(DEV)
+        y = iir_snapshots(u, torch.exp(lp), res, a, md)
+        got = iir_verify_gated(zf, lp, res, D, b, md)
+    else:
+        w = prm["conv"].view(H, -1).to(DEV)
+        a, b = _fir_state_dev(state), _fir_state_dev(state)
+        y = fir_snapshots(u, w, a, md)
+        got = fir_verify_gated(zf, w, D, b, md)
+    if D is not None:
+        y = y + D * u
+    ref = x2 * y
+    covered = torch.zeros(T, dtype=torch.bool)
+    for r in range(nreq):
+        covered[int(starts[r]):min(int(ends[r]), int(starts[r]) + Q)] = True
+    ref[~covered.to(DEV)] = 0
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+    assert torch.equal(a, b)
