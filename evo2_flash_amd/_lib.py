@@ -208,6 +208,11 @@ SIGNATURES = {
         _c_p, _c_i64, _c_i64, _c_i64, _c_i64,     # out, so, M, N, K
         _c_p,                                     # stream
     ],
+    "evo2_fp8_quant_gemv": [
+        _c_p, _c_p, _c_i64, _c_i32,               # x, w, sw, packed
+        _c_p, _c_p, _c_p,                         # x_scale, w_scale, bias
+        _c_p, _c_i64, _c_i64, _c_p,               # out, N, K, stream
+    ],
     "evo2_fp8_gemm_persist_order": [_c_i64, _c_i64, ctypes.c_int, _c_p, _c_p],
     "evo2_fp8_fast_accum_gemm": [
         _c_p, _c_i64, _c_p, _c_i64,               # a8, sa, b_t, sb

@@ -860,6 +860,116 @@ static void launch_small(const GemmArgs &a, hipStream_t stream) {
   hipLaunchKernelGGL((fp8_gemm_small_kernel<WPG, PACKED>), grid, dim3(64 * WPG), 0, stream, a);
 }
 
+// e4m3fn(clamp(x / s, -448, 448)) of 16 bf16 values (two 16-byte loads).
+__device__ __forceinline__ int4 quantize16(const bf16_t *x, float s) {
+  const uint4 *xp = reinterpret_cast<const uint4 *>(x);
+  const uint4 a = xp[0], b = xp[1];
+  const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  int out[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float v[4] = {lo_bf(w[2 * j]), hi_bf(w[2 * j]), lo_bf(w[2 * j + 1]), hi_bf(w[2 * j + 1])};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = fminf(fmaxf(v[i] / s, -448.0f), 448.0f);
+    int packed = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+    out[j] = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], packed, true);
+  }
+  return make_int4(out[0], out[1], out[2], out[3]);
+}
+
+// ---------------------------------------------------------------------------
+// A few rows (M <= 16): the same weight stream without the activation ring.  A
+// workgroup owns 16 W rows and its eight waves split K (the partial sums meet in
+// LDS), two K steps of weight in flight per wave in few registers, so that
+// several workgroups share a CU and one's start and end pass under the others'
+// streams.  QUANT: x is one bf16 row that each workgroup quantises into LDS
+// itself, one launch for the quantisation and the product (two rows gain
+// nothing: every workgroup repeats the work).  Quantisation and product, the
+// packed weight streaming from HBM, us before (the ring kernel behind a
+// quantisation launch) / here: 12288 x 4096 at M = 1 15.2 / 11.0 (two launches
+// 11.6), 2 14.6 / 11.7, 8 15.0 / 12.2, 16 15.2 / 14.3; 4096 x 4096 at 1 11.5 / 5.9,
+// 16 12.1 / 7.9; 5760 x 1920 at 1 8.7 / 4.7; 24576 x 8192 at 1 37.5 / 32.7, 8 37.9 /
+// 34.0, 16 36.7 / 40.8: hence 16 rows up to N K = 2^26, 8 above.  The same bits.
+constexpr int F_ROWS = 16;    // X rows
+constexpr int F_WAVES = 8;    // waves per workgroup: parts of K
+constexpr int F_QMAXK = 16384;
+
+template <bool PACKED, bool QUANT>
+__global__ __launch_bounds__(64 * F_WAVES) void fp8_few_kernel(GemmArgs p) {
+  __shared__ float part[F_WAVES][256];
+  extern __shared__ __align__(16) uint8_t xq[];  // QUANT: the row, e4m3
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;  // operand row, 32-byte part of a K step
+  const int n0 = blockIdx.x * 16;
+  const float s_x = p.sx_scale[0], s_w = p.sw_scale[0];
+  const int KT = p.K / S_BK, per = (KT + F_WAVES - 1) / F_WAVES;
+  const int k0 = wave * per, k1 = min(k0 + per, KT);  // this wave's K steps
+  const uint8_t *wr = PACKED ? p.w + (int64_t)blockIdx.x * KT * 2048 + 16 * lane
+                             : p.w + (int64_t)min(n0 + r, p.N - 1) * p.sw + 32 * g;
+  const int xrow = min(r, p.M - 1);
+  const uint8_t *xr = p.x + (int64_t)xrow * p.sx + 32 * g;
+  i32x4 wf[2][2], xf[2][2];
+  auto load = [&](auto buf, int k) __attribute__((always_inline)) {
+    constexpr int B = decltype(buf)::value;
+    k = min(k, KT - 1);  // (past the part: loaded, not used)
+    if constexpr (PACKED) {
+      wf[B][0] = ld_nt(reinterpret_cast<const i32x4 *>(wr + (int64_t)k * 2048));
+      wf[B][1] = ld_nt(reinterpret_cast<const i32x4 *>(wr + (int64_t)k * 2048 + 1024));
+    } else {
+      wf[B][0] = *reinterpret_cast<const i32x4 *>(wr + k * S_BK);
+      wf[B][1] = *reinterpret_cast<const i32x4 *>(wr + k * S_BK + 16);
+    }
+    if constexpr (!QUANT) {
+      xf[B][0] = *reinterpret_cast<const i32x4 *>(xr + k * S_BK);
+      xf[B][1] = *reinterpret_cast<const i32x4 *>(xr + k * S_BK + 16);
+    }
+  };
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  auto use = [&](auto buf, int k) __attribute__((always_inline)) {
+    constexpr int B = decltype(buf)::value;
+    if (k >= k1) return;  // uniform
+    i32x4 x0 = xf[B][0], x1 = xf[B][1];
+    if constexpr (QUANT) {
+      const uint8_t *q = xq + k * S_BK + 32 * g;  // (all operand rows: the one)
+      x0 = *reinterpret_cast<const i32x4 *>(q);
+      x1 = *reinterpret_cast<const i32x4 *>(q + 16);
+    }
+    const i32x8 a = {wf[B][0].x, wf[B][0].y, wf[B][0].z, wf[B][0].w,
+                     wf[B][1].x, wf[B][1].y, wf[B][1].z, wf[B][1].w};
+    const i32x8 b = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc, 0, 0, 0, 0, 0, 0);
+  };
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  load(B0{}, k0);
+  load(B1{}, k0 + 1);
+  if constexpr (QUANT) {
+    const bf16_t *xb = reinterpret_cast<const bf16_t *>(p.x);
+    for (int k = 16 * tid; k < p.K; k += 16 * 64 * F_WAVES)
+      *reinterpret_cast<int4 *>(xq + k) = quantize16(xb + k, s_x);
+    __syncthreads();
+  }
+  for (int k = k0; k < k1; k += 2) {
+    use(B0{}, k);
+    if (k + 2 < k1) load(B0{}, k + 2);
+    use(B1{}, k + 1);
+    if (k + 3 < k1) load(B1{}, k + 3);
+  }
+  // lane (r, g) holds X row r, W rows n0 + 4 g + i
+  *reinterpret_cast<f32x4 *>(&part[wave][4 * lane]) = acc;
+  __syncthreads();
+  if (tid >= 256) return;
+  const int m = (tid >> 2) & 15, n = n0 + 4 * (tid >> 6) + (tid & 3);
+  if (m >= p.M || n >= p.N) return;
+  float v = 0.0f;
+#pragma unroll
+  for (int w = 0; w < F_WAVES; ++w) v += part[w][tid];
+  v *= s_x * s_w;
+  if (p.bias) v += bf2f(p.bias[n]);
+  p.out[(int64_t)m * p.so + n] = f2bf(v);
+}
+
 // Decode weight layout: 16-row group G, K step k (128 bytes), half h, lane
 // l = r + 16 q holds W[16 G + r][128 k + 32 q + 16 h .. + 16) at byte
 // ((G * K / 128 + k) * 2 + h) * 1024 + 16 l.  One thread per 16 bytes.
@@ -932,19 +1042,7 @@ __global__ __launch_bounds__(256) void fp8_quantize16_kernel(const bf16_t *x, in
        c += (int64_t)gridDim.x * 256) {
     const int64_t r = c / cpr;
     const int k = static_cast<int>(c - r * cpr) * 16;
-    const uint4 *xp = reinterpret_cast<const uint4 *>(x + r * sx + k);
-    const uint4 a = xp[0], b = xp[1];
-    const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    int out[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float v[4] = {lo_bf(w[2 * j]), hi_bf(w[2 * j]), lo_bf(w[2 * j + 1]), hi_bf(w[2 * j + 1])};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = fminf(fmaxf(v[i] / s, -448.0f), 448.0f);
-      int packed = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
-      out[j] = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], packed, true);
-    }
-    *reinterpret_cast<int4 *>(q + r * sq + k) = make_int4(out[0], out[1], out[2], out[3]);
+    *reinterpret_cast<int4 *>(q + r * sq + k) = quantize16(x + r * sx + k, s);
   }
 }
 
@@ -1010,6 +1108,11 @@ static int persist_rows(int64_t tiles_n, int64_t M, int ncu) {
 
 template <bool PACKED>
 static void launch_stream(const GemmArgs &a, hipStream_t st) {
+  if (a.N <= (1 << 26) && (a.M <= 8 || (a.M <= F_ROWS && (int64_t)a.N * a.K <= (1 << 26)))) {
+    hipLaunchKernelGGL((fp8_few_kernel<PACKED, false>), dim3(static_cast<unsigned>(cdiv(a.N, 16))),
+                       dim3(64 * F_WAVES), 0, st, a);
+    return;
+  }
   const int ncu = cu_count() > 0 ? cu_count() : 256;
   const int64_t yblocks = cdiv(a.M, S_ROWS);
   int best_w = 4;
@@ -1154,6 +1257,30 @@ extern "C" int evo2_fp8_gemm_packed(const void *x8, int64_t sx, const void *wp,
              static_cast<int>(M), static_cast<int>(N), static_cast<int>(K)};
   launch_stream<true>(a, static_cast<hipStream_t>(stream));
   return check_launch("fp8_gemm_packed");
+}
+
+extern "C" int evo2_fp8_quant_gemv(const void *x, const void *w, int64_t sw, int32_t packed,
+                                   const float *x_scale, const float *w_scale, const void *bias,
+                                   void *out, int64_t N, int64_t K, void *stream) {
+  if (N <= 0 || K <= 0)
+    return fail(EVO2_ERR_INVALID, "fp8_quant_gemv: bad sizes N=%lld K=%lld", (long long)N, (long long)K);
+  if (!x || !w || !x_scale || !w_scale || !out)
+    return fail(EVO2_ERR_INVALID, "fp8_quant_gemv: null pointer argument");
+  if (K % S_BK || K > F_QMAXK || N > (1 << 26) || (packed && N % 16))
+    return fail(EVO2_ERR_UNSUPPORTED, "fp8_quant_gemv: N=%lld, K=%lld: K must be a multiple of %d up to %d",
+                (long long)N, (long long)K, S_BK, F_QMAXK);
+  if ((!packed && sw % 16) || reinterpret_cast<uintptr_t>(x) % 16 ||
+      reinterpret_cast<uintptr_t>(w) % 16)
+    return fail(EVO2_ERR_UNSUPPORTED, "fp8_quant_gemv: operands must be 16-byte aligned rows");
+  GemmArgs a{static_cast<const uint8_t *>(x), K, static_cast<const uint8_t *>(w), sw, x_scale, w_scale,
+             static_cast<const bf16_t *>(bias), static_cast<bf16_t *>(out), N, 1,
+             static_cast<int>(N), static_cast<int>(K)};
+  const dim3 grid(static_cast<unsigned>(cdiv(N, 16)));
+  const size_t lds = static_cast<size_t>(K);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (packed) hipLaunchKernelGGL((fp8_few_kernel<true, true>), grid, dim3(64 * F_WAVES), lds, st, a);
+  else hipLaunchKernelGGL((fp8_few_kernel<false, true>), grid, dim3(64 * F_WAVES), lds, st, a);
+  return check_launch("fp8_quant_gemv");
 }
 
 extern "C" int64_t evo2_fp8_gemm_persist_order(int64_t tiles_n, int64_t tiles_m, int ncu, int32_t *bn,

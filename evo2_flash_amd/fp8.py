@@ -127,6 +127,21 @@ def fp8_gemm_packed(x8, wp, x_scale, w_scale, bias=None, out=None):
     return out
 
 
+def _one_row(x, w, packed, input_scale, weight_scale, bias, out):
+    """static_fp8_linear of one row in one launch (the same result bits)."""
+    _lib.require_device(x, w, input_scale, weight_scale, bias)
+    N, K = w.shape
+    xs = input_scale.to(torch.float32).reshape(1)
+    ws = weight_scale.to(torch.float32).reshape(1)
+    if bias is not None:
+        bias = bias.to(torch.bfloat16).contiguous()
+    if out is None:
+        out = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
+    _lib.call("evo2_fp8_quant_gemv", _lib.ptr(x), _lib.ptr(w), w.stride(0), int(packed),
+              _lib.ptr(xs), _lib.ptr(ws), _lib.ptr(bias), _lib.ptr(out), N, K, _lib.stream_of(x))
+    return out
+
+
 def static_fp8_linear(x, weight, input_scale, weight_scale, bias=None, out=None, packed=None):
     """vLLM's static W8A8 linear: (..., K) bf16 -> (..., N) bf16; a 2-D x may
     write its result into `out` (M, N) bf16 with unit column stride.  With
@@ -134,6 +149,16 @@ def static_fp8_linear(x, weight, input_scale, weight_scale, bias=None, out=None,
     stream take the decode GEMM on it (the same result bits): at most 64
     rows, or ceil(M / 64) * N <= TILE_MIN_WORK."""
     K = x.shape[-1]
+    N = weight.shape[0]
+    if (x.numel() == K and x.dtype == torch.bfloat16 and x.stride(-1) == 1 and K % 128 == 0
+            and 0 < K <= 16384 and (bias is None or bias.shape == (N,))
+            and (out is None or (x.dim() == 2 and out.shape == (1, N) and out.stride(1) == 1
+                                 and out.dtype == torch.bfloat16 and out.device == x.device))):
+        w = weight if packed is None else packed
+        if (w.dtype == E4M3 and w.shape == (N, K) and w.stride(1) == 1 and w.stride(0) % 16 == 0
+                and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+                and (packed is None or packed.is_contiguous())):
+            return _one_row(x, w, packed is not None, input_scale, weight_scale, bias, out)
     x8 = quantize_input(x.reshape(-1, K), input_scale)
     gemm = fp8_gemm
     w = weight

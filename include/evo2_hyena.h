@@ -521,6 +521,19 @@ int evo2_fp8_gemm_packed(const void *x8, int64_t sx, const void *wp,
                          void *out, int64_t so, int64_t M, int64_t N, int64_t K, void *stream);
 
 /*
+ * evo2_fp8_quantize and evo2_fp8_gemm (packed = 0, row stride sw) or
+ * evo2_fp8_gemm_packed (packed = 1) of one bf16 row x (K,) in one launch, the
+ * same bits: out (N,) bf16.  K a multiple of 128 up to 16384, 16-byte aligned
+ * operands.
+ *
+ * Replaces vLLM's static fp8 linear of the in_proj at one decode token
+ * (evo2_flash/mixers.py:741-757, 1076-1092).
+ */
+int evo2_fp8_quant_gemv(const void *x, const void *w, int64_t sw, int32_t packed, const float *x_scale,
+                        const float *w_scale, const void *bias, void *out, int64_t N, int64_t K,
+                        void *stream);
+
+/*
  * The order in which evo2_fp8_gemm's persistent kernel (one workgroup per
  * compute unit; 256 W rows x 64 to 256 X rows a tile) walks a grid of tiles_n x
  * tiles_m tiles with ncu workgroups: tile t, run by workgroup

@@ -125,6 +125,37 @@ def test_gemm_known_answer_ragged_tiles(M, N, K, bias):
     assert (wide[M] == 99).all() and (wide[:, N:] == 99).all()
 
 
+@pytest.mark.parametrize("N,K", [(16, 128), (37, 1920), (96, 384), (12288, 4096), (48, 16384)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_one_row_linear_same_bits(N, K, bias, monkeypatch):
+    """One row quantised inside the product's launch: the bits of the
+    quantisation and the GEMM apart, on the row-major and the packed weight, with
+    saturated, zero and tiny inputs."""
+    from evo2_flash_amd import _lib
+    from evo2_flash_amd.fp8 import fp8_pack_weight, packable
+    g = torch.Generator().manual_seed(N + K)
+    x = torch.randn(1, K, generator=g) * 3
+    x[0, :4] = torch.tensor([1e4, -1e4, 0.0, 1e-9])
+    x = x.to(torch.bfloat16).to(DEV)
+    w = (torch.randn(N, K, generator=g) * 0.5).to(E4M3).to(DEV)
+    b = torch.randn(N, generator=g).to(torch.bfloat16).to(DEV) if bias else None
+    xs, ws = torch.tensor([0.013], device=DEV), torch.tensor([0.3], device=DEV)
+    ref = fp8_gemm(quantize_input(x, xs), w, xs, ws, b)
+    calls = []
+    call = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda n, *a: (calls.append(n), call(n, *a)))
+    print(f"one-row fp8 linear N={N} K={K} bias={bias}", flush=True)
+    wide = torch.full((2, N), 9.0, dtype=torch.bfloat16, device=DEV)
+    got = [static_fp8_linear(x, w, xs, ws, b), static_fp8_linear(x[0], w, xs, ws, b)[None],
+           static_fp8_linear(x, w, xs, ws, b, out=wide[:1])]
+    assert calls == ["evo2_fp8_quant_gemv"] * 3
+    if packable(N, K):
+        got.append(static_fp8_linear(x, w, xs, ws, b, packed=fp8_pack_weight(w)))
+    for y in got:
+        assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+    assert (wide[1] == 9).all()
+
+
 def test_static_linear_persistent_with_bias():
     M, N, K = 4096, 4096, 1024   # 16 x 16 tiles
     g = torch.Generator().manual_seed(11)
