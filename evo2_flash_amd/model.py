@@ -19,8 +19,10 @@ split-context paged decode attention kernel (attention.py), which reads each
 page once and masks positions past each sequence's; a decode step has fixed
 shapes and captures into one HIP graph.  Prefill runs prompts through the
 same layers (the Hyena mixers on their prefill kernels, writing the states
-the decode steps continue from) with causal attention in torch.  The
-projections and MLPs are plain torch on ROCm (outside the mixer hot path).
+the decode steps continue from) with causal attention on this build's prefill
+kernel at head_dim 128 and in torch otherwise; rotary and the page writes are
+one launch (attention.py).  The projections and MLPs run on the weight-streaming
+kernel at decode batch sizes and in torch otherwise (linear.py).
 
 Weights are random, seeded, in the benchmark's distributions.
 """
