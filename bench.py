@@ -317,8 +317,9 @@ def bench_model(steps, dev, B=B_DECODE, seed=21):
             "bytes_per_step": {"weights": wbytes, "kv_cache": kvbytes},
             "achieved_GBs": round((wbytes + kvbytes) / (ms * 1e-3) / 1e9, 1),
             "kv": "16-position pages, seeded random block table",
-            "note": "states and KV pages from prefilling the prompts; Hyena mixers and decode "
-                    "attention on this build's kernels; projections and MLP in torch"}
+            "note": "states and KV pages from prefilling the prompts; Hyena mixers, rotary and "
+                    "decode attention on the package's kernels, and bf16 projections and MLP "
+                    "too at batch 8; those in torch at batch 64"}
 
 
 def _layer_timers(model):
@@ -370,8 +371,8 @@ def bench_model_prefill(dev, L=L_PREFILL, reps=3, seed=31):
             "layer_us": {k: round(v, 1) for k, v in per.items()},
             "instrumented_ms": round(t_inst * 1e3, 2),
             "note": "whole 7B-shaped model, batch 1; Hyena layers = in_proj + mixer core + "
-                    "out_proj and the causal attention on this build's kernels; attention "
-                    "projections, MLP and norms' GEMMs in torch"}
+                    "out_proj, rotary and the causal attention on the package's kernels; "
+                    "attention projections and the MLP's GEMMs in torch"}
 
 
 def bench_attn_prefill(dev, shapes=((32, L_PREFILL),), reps=3, seed=51):
