@@ -6,11 +6,14 @@
 //   angle(t, i) = (t / factor) * inv_freq[i],  i < head_dim / 2
 //   (x[i], x[i + hd/2]) -> (x[i] cos - x[i + hd/2] sin, x[i + hd/2] cos + x[i] sin)
 //
-// in fp32, rounded to bf16 once.  As separate elementwise operators this was
-// some 35 launches and ~14 passes over q, k and v: 2.3 ms of a 6.0 ms
+// in fp32, each product and sum rounded by itself (no FMA: the bits of the
+// separate fp32 operators, rotary_neox in model.py), then to bf16 once.  As
+// separate elementwise operators this was some 35 launches and ~14 passes over q, k and v: 2.3 ms of a 6.0 ms
 // attention layer over a 16384-token prompt (32 heads of 128), 100 us of a
 // 299 us decode layer at batch 8.
 #include "common.h"
+
+#pragma clang fp contract(off)
 
 namespace evo2 {
 

@@ -327,3 +327,29 @@ def test_rotary_decode_vs_fp64(B, nh, hd):
             assert torch.equal(vc[pg, :, off], vr[b])
             kc[pg, :, :, off] = vc[pg, :, off] = 0
     assert (kc == 0).all() and (vc == 0).all()      # and nowhere else
+
+
+@pytest.mark.parametrize("factor", [1.0, 4.0])
+def test_rotary_bits_of_the_separate_operators(factor):
+    """Both rotary launches round as the fp32 operators of rotary_neox do, one
+    rounding per product and sum: the same bits, positions up to 2^20."""
+    from evo2_flash_amd.attention import rotary_decode, rotary_prefill
+    from evo2_flash_amd.model import rotary_neox
+    hd, nh, L, B = 128, 4, 1000, 33
+    g, wide, inv_freq = _qkv_case(L, nh, hd, 11)
+    wd, fd = wide.to(DEV)[:, :3 * nh * hd], inv_freq.to(DEV)
+    q0, k0 = (wd.reshape(L, 3, nh, hd)[:, i] for i in (0, 1))
+    table = (torch.randperm(B * 64, generator=g)[:B * 64] + 1).int().view(B, 64).to(DEV)
+    cache = PagedKVCache(B * 64 + 1, nh, hd, DEV)
+    print(f"rotary bits factor={factor}", flush=True)
+    q, k, _ = rotary_prefill(wd, cache, table, fd, factor, 1, L)
+    pos = torch.arange(L, device=DEV)
+    for got, x in ((q, q0), (k, k0)):
+        assert torch.equal(got[0].transpose(0, 1), rotary_neox(x, pos, fd, factor))
+    pos = torch.randint(0, 1 << 20, (B,), generator=g).to(DEV)
+    q = rotary_decode(wd[:B], cache, table, pos, fd, factor)
+    assert torch.equal(q, rotary_neox(q0[:B], pos, fd, factor))
+    pos = torch.randint(0, 1024, (B,), generator=g).to(DEV)
+    rotary_decode(wd[:B], cache, table, pos, fd, factor)
+    page = table[torch.arange(B, device=DEV), pos // PAGE].long()
+    assert torch.equal(cache.k[page, :, :, pos % PAGE], rotary_neox(k0[:B], pos, fd, factor))
