@@ -541,9 +541,13 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
   //   sub-step 1: MFMAs of (k, 1) while reading (k + 1, 0) from the other
   //     stage.
   // The first step after an epilogue also has the epilogue's EPI_STORES
-  // stores outstanding (and, in wave 0, the next bias load after them), all
-  // issued after the loads of slice k + 1: loads and stores retire in order,
-  // so waiting until at most EPI_STORES remain covers the loads.
+  // stores outstanding, issued after the loads of slice k + 1: loads and
+  // stores retire in order, so waiting until at most EPI_STORES remain covers
+  // the loads.
+  // The first step of tile j issues the bias of tile j + 1 (wave 0, `bias`)
+  // behind its barrier: the buffer held tile j - 1's, and only there has every
+  // wave left that tile's epilogue.  The load precedes the refill of its step,
+  // so the next step's wait covers it, a barrier before epilogue j + 1.
   i32x8 fa[2][4], fb[2][TM];
   // every MFMA of a sub-step is followed by its share of the fragment reads
   // and of the refill loads
@@ -564,7 +568,8 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
   // first: slice 0 of a tile, whose sub-step 0 starts the accumulators.  With
   // three stages slice k + 2 may still be in flight when slice k + 1 is
   // waited for, and the freed stage takes slice k + 3.
-  auto step = [&](auto stage, int k, bool after_epilogue, auto first) __attribute__((always_inline)) {
+  auto step = [&](auto stage, int k, bool after_epilogue, auto first, auto &&bias)
+      __attribute__((always_inline)) {
     constexpr int S = decltype(stage)::value;
     constexpr int FLY = (NST - 2) * (DB + DX);
     read_frags(stage, I1{}, fa[1], fb[1]);
@@ -573,6 +578,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
     if (after_epilogue) vmcnt_wait<FLY + EPI_STORES>();
     else vmcnt_wait<FLY>();
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    bias();
     issue(stage, k + NST);
     read_frags(integral_constant<int, (S + 1) % NST>{}, I0{}, fa[0], fb[0]);
     mma(fa[1], fb[1], F0{});
@@ -581,6 +587,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
 
   using P0 = integral_constant<int, 0>;
   using P1 = integral_constant<int, 1>;
+  auto no_bias = [] {};
   load_bias(P0{}, 0);
   dma_tile(0);
   issue(I0{}, 0);
@@ -594,17 +601,18 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
     int kk = 0, j = 0;  // slice within the tile, tile
     bool after = false;
     auto one = [&](auto stage, int k) __attribute__((always_inline)) {
-      if (kk == 0) {  // uniform: a tile begins (its accumulators at zero)
-        if (j + 1 < ntile) {
-          if (j & 1) load_bias(P0{}, j + 1);
-          else load_bias(P1{}, j + 1);
-        }
+      const bool begins = kk == 0;  // uniform: a tile begins (its accumulators at zero)
+      if (begins) {
 #pragma unroll
         for (int tn = 0; tn < 4; ++tn)
 #pragma unroll
           for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = zero16;
       }
-      step(stage, k, after, F0{});
+      step(stage, k, after, F0{}, [&]() __attribute__((always_inline)) {
+        if (!begins || j + 1 >= ntile) return;
+        if (j & 1) load_bias(P0{}, j + 1);
+        else load_bias(P1{}, j + 1);
+      });
       after = ++kk == KT;
       if (after) {
         epilogue(j);
@@ -619,21 +627,21 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
     }
   } else {
     int s = 0;
-    // Tile j of parity P: first the bias of tile j + 1 into the other buffer
-    // (its previous contents, tile j - 1's, were added before this tile
-    // began), then the slices, the first starting the accumulators (an even
-    // count in pairs from stage 0; an odd one from stage P), then the epilogue
-    // with this buffer.
+    // Tile j of parity P: the slices, the first starting the accumulators and
+    // loading the bias of tile j + 1 into the other buffer (an even count in
+    // pairs from stage 0; an odd one from stage P), then the epilogue with this
+    // buffer.
     auto tile = [&](auto par, int j) __attribute__((always_inline)) {
       constexpr int P = decltype(par)::value, S = ODD ? P : 0;
       using A = integral_constant<int, S>;
       using B = integral_constant<int, S ^ 1>;
-      if (j + 1 < ntile) load_bias(integral_constant<int, P ^ 1>{}, j + 1);
-      step(A{}, s++, j > 0, F1{});
-      if (!ODD) step(B{}, s++, false, F0{});
+      step(A{}, s++, j > 0, F1{}, [&]() __attribute__((always_inline)) {
+        if (j + 1 < ntile) load_bias(integral_constant<int, P ^ 1>{}, j + 1);
+      });
+      if (!ODD) step(B{}, s++, false, F0{}, no_bias);
       for (int k = ODD ? 1 : 2; k < KT; k += 2, s += 2) {
-        step(integral_constant<int, ODD ? S ^ 1 : 0>{}, s, false, F0{});
-        step(integral_constant<int, ODD ? S : 1>{}, s + 1, false, F0{});
+        step(integral_constant<int, ODD ? S ^ 1 : 0>{}, s, false, F0{}, no_bias);
+        step(integral_constant<int, ODD ? S : 1>{}, s + 1, false, F0{}, no_bias);
       }
       epilogue(j);
     };

@@ -125,6 +125,25 @@ def test_gemm_known_answer_ragged_tiles(M, N, K, bias):
     assert (wide[M] == 99).all() and (wide[:, N:] == 99).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(8100, 8192, 128), (8100, 8192, 256),       # 256 rows a tile, 4 rounds
+                                   (3001, 12288, 640), (3001, 12288, 256),    # 192 rows, 3 rounds
+                                   (1999, 12288, 128), (1999, 12288, 640)])   # 128 rows, 3 rounds
+def test_gemm_known_answer_bias_of_every_tile(M, N, K):
+    """Three and more tiles a workgroup, the bias another in each 256-column
+    tile: a tile adds its own, whichever buffer it came through (both forms of
+    the slice ring, odd and even counts of slices, one among them)."""
+    g = torch.Generator().manual_seed(M + K)
+    x8 = _small_int_e4m3((M, K), g).to(DEV)
+    w8 = _small_int_e4m3((N, K), g).to(DEV)
+    n = torch.arange(N)
+    b = (512 * (n // 256 * 7 % 61 - 30) + n % 4).to(torch.bfloat16).to(DEV)
+    one = torch.ones(1, device=DEV)
+    print(f"bias of every tile M={M} N={N} K={K}", flush=True)
+    out = fp8_gemm(x8, w8, one, one, b)
+    ref = (x8.float() @ w8.float().t() + b.float()).to(torch.bfloat16)  # exact in fp32
+    assert torch.equal(out, ref)
+
+
 @pytest.mark.parametrize("N,K", [(16, 128), (37, 1920), (96, 384), (12288, 4096), (48, 16384)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_one_row_linear_same_bits(N, K, bias, monkeypatch):
