@@ -187,6 +187,27 @@ class PagedKVCache:
         return kd[..., :L], vd[:, :, :L]
 
 
+def _rotary_operands(qkv, cache, inv_freq):
+    """Checks of what both rotary launches read by address: the pages and the
+    frequencies, returned as contiguous fp32 (a module cast to bf16 casts its
+    buffer with it)."""
+    nh, hd = cache.k.shape[1], cache.k.shape[2]
+    if (cache.k.dtype != torch.bfloat16 or cache.v.dtype != torch.bfloat16
+            or cache.k.shape[3:] != (PAGE,) or cache.v.shape != (cache.k.shape[0], nh, PAGE, hd)
+            or cache.k.stride(3) != 1 or cache.v.stride(3) != 1):
+        raise ValueError(f"KV pages must be bf16 (pages, heads, head_dim, {PAGE}) and (pages, "
+                         f"heads, {PAGE}, head_dim) with unit last strides, got "
+                         f"{tuple(cache.k.shape)} {cache.k.dtype}, {tuple(cache.v.shape)} "
+                         f"{cache.v.dtype}")
+    if inv_freq.shape != (hd // 2,):
+        raise ValueError(f"inv_freq must be ({hd // 2},), got {tuple(inv_freq.shape)}")
+    if qkv.dim() != 2 or qkv.shape[1] != 3 * nh * hd or qkv.dtype != torch.bfloat16 \
+            or qkv.stride(1) != 1:
+        raise ValueError(f"qkv must be bf16 rows of {3 * nh * hd}, got {tuple(qkv.shape)} "
+                         f"{qkv.dtype}")
+    return nh, hd, inv_freq.to(torch.float32).contiguous()
+
+
 def rotary_prefill(qkv, cache, block_table, inv_freq, factor, nseq, L):
     """Rotary and cache write of nseq prompts of L tokens in one launch: qkv
     (nseq * L, 3 * heads * 128) bf16 rows (q | k | v).  Writes k and v into
@@ -194,10 +215,9 @@ def rotary_prefill(qkv, cache, block_table, inv_freq, factor, nseq, L):
     operands of prefill attention: q, k (nseq, heads, L, 128) rotated, and the
     values transposed, (nseq, heads, 128, L rounded up to 8), zeros from L on."""
     _lib.require_device(qkv, cache.k, cache.v, block_table, inv_freq)
-    nh, hd = cache.k.shape[1], cache.k.shape[2]
-    if qkv.shape != (nseq * L, 3 * nh * hd) or qkv.dtype != torch.bfloat16 or qkv.stride(1) != 1:
-        raise ValueError(f"qkv must be ({nseq * L}, {3 * nh * hd}) bf16 rows, got "
-                         f"{tuple(qkv.shape)} {qkv.dtype}")
+    nh, hd, inv_freq = _rotary_operands(qkv, cache, inv_freq)
+    if qkv.shape[0] != nseq * L:
+        raise ValueError(f"qkv must have {nseq * L} rows, got {qkv.shape[0]}")
     if (block_table.dtype != torch.int32 or block_table.stride(1) != 1
             or block_table.shape[0] < nseq):
         raise ValueError("block_table must be (>= nseq, pages) int32 with unit column stride")
@@ -218,11 +238,8 @@ def rotary_decode(qkv, cache, block_table, positions, inv_freq, factor):
     (B, 3 * heads * head_dim) bf16 rows (q | k | v) at positions (B,) int64.
     Writes k and v into `cache`'s pages and returns q (B, heads, head_dim)."""
     _lib.require_device(qkv, cache.k, cache.v, block_table, positions, inv_freq)
-    nh, hd = cache.k.shape[1], cache.k.shape[2]
+    nh, hd, inv_freq = _rotary_operands(qkv, cache, inv_freq)
     B = qkv.shape[0]
-    if qkv.shape[1] != 3 * nh * hd or qkv.dtype != torch.bfloat16 or qkv.stride(1) != 1:
-        raise ValueError(f"qkv must be (B, {3 * nh * hd}) bf16 rows, got {tuple(qkv.shape)} "
-                         f"{qkv.dtype}")
     if block_table.dtype != torch.int32 or block_table.stride(1) != 1 or block_table.shape[0] < B:
         raise ValueError("block_table must be (>= B, pages) int32 with unit column stride")
     if positions.shape != (B,):

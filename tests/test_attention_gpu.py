@@ -353,3 +353,32 @@ def test_rotary_bits_of_the_separate_operators(factor):
     rotary_decode(wd[:B], cache, table, pos, fd, factor)
     page = table[torch.arange(B, device=DEV), pos // PAGE].long()
     assert torch.equal(cache.k[page, :, :, pos % PAGE], rotary_neox(k0[:B], pos, fd, factor))
+
+
+@pytest.mark.parametrize("L", [40, 41])
+def test_attention_layer_cast_to_bf16(L):
+    """A layer after .to(torch.bfloat16), its inv_freq buffer with it: the
+    prompt's and the next token's keys rotate by the cast frequencies."""
+    from evo2_flash_amd.config import HyenaConfig
+    from evo2_flash_amd.model import Evo2Attention, rotary_neox
+    cfg = HyenaConfig(hidden_size=256, num_attention_heads=2, num_hidden_layers=1,
+                      attn_layer_idxs=[0])
+    layer = Evo2Attention(cfg, 9, 4, 1, rope_factor=4.0, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(L)
+    for p in layer.parameters():
+        p.data.copy_(torch.randn(p.shape, generator=g, device=DEV) * 0.05)
+    layer = layer.to(bf)
+    assert layer.inv_freq.dtype == bf
+    table = torch.tensor([[5, 2, 7, 1]], dtype=torch.int32, device=DEV)
+    x = torch.randn(L + 1, 256, generator=g, device=DEV).to(bf)
+    print(f"attention layer cast to bf16 L={L}", flush=True)
+    with torch.no_grad():
+        layer.forward_prefill(x[:L], 1, L, table)
+        layer.forward_decode(x[L:], torch.tensor([L], device=DEV), table)
+        # the keys of either call, projected by the call's own GEMM
+        for rows, pos in ((x[:L], torch.arange(L, device=DEV)),
+                          (x[L:], torch.tensor([L], device=DEV))):
+            k = layer.qkv_proj(rows)[0].view(-1, 3, 2, 128)[:, 1]
+            want = rotary_neox(k, pos, layer.inv_freq, 4.0)
+            page = table[0, pos // PAGE].long()
+            assert torch.equal(layer.cache.k[page, :, :, pos % PAGE], want)

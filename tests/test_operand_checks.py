@@ -1,0 +1,86 @@
+"""What the wrappers hand to the kernels by address, checked without a GPU: the
+native call is replaced by one that reads its arguments on the host."""
+
+import ctypes
+
+import pytest
+import torch
+
+from evo2_flash_amd import _lib
+
+bf = torch.bfloat16
+
+
+@pytest.fixture
+def native(monkeypatch):
+    """CPU tensors pass the device check; calls are recorded, not made.  A
+    recorded call is (name, arguments, what `native.look` returned inside it)."""
+    class Native(list):
+        look = staticmethod(lambda name, args: None)
+
+    calls = Native()
+    monkeypatch.setattr(_lib, "require_device", lambda *t: None)
+    monkeypatch.setattr(_lib, "stream_of", lambda t=None: None)
+    monkeypatch.setattr(_lib, "call", lambda name, *a: calls.append((name, a, calls.look(name, a))))
+    return calls
+
+
+def _floats(address, n):
+    return torch.tensor((ctypes.c_float * n).from_address(address))
+
+
+def _rotary_case(hd=128, nh=2, rows=4):
+    from evo2_flash_amd.attention import PagedKVCache
+    cache = PagedKVCache(5, nh, hd, "cpu")
+    qkv = torch.randn(rows, 3 * nh * hd).to(bf)
+    table = torch.arange(1, 5, dtype=torch.int32).view(4, 1)
+    inv_freq = 1.0 / 10000.0 ** (torch.arange(0, hd, 2, dtype=torch.float32) / hd)
+    return qkv, cache, table, inv_freq
+
+
+def _rotate(which, qkv, cache, table, inv_freq):
+    from evo2_flash_amd.attention import rotary_decode, rotary_prefill
+    if which == "prefill":
+        return rotary_prefill(qkv, cache, table, inv_freq, 1.0, 1, qkv.shape[0])
+    return rotary_decode(qkv, cache, table, torch.zeros(qkv.shape[0], dtype=torch.int64), inv_freq,
+                         1.0)
+
+
+@pytest.mark.parametrize("which", ["prefill", "decode"])
+@pytest.mark.parametrize("form", ["bf16", "fp64", "strided"])
+def test_rotary_frequencies_reach_the_kernel_as_fp32(which, form, native):
+    """inv_freq of another type (a module cast with .to(torch.bfloat16)) or
+    stride: the kernel reads head_dim / 2 contiguous fp32 of the same values."""
+    qkv, cache, table, inv_freq = _rotary_case()
+    f = {"bf16": inv_freq.to(bf), "fp64": inv_freq.double(),
+         "strided": inv_freq.repeat_interleave(2)[::2]}[form]
+    native.look = lambda name, a: _floats(a[2], 64)
+    _rotate(which, qkv, cache, table, f)
+    assert [c[0] for c in native] == ["evo2_rotary_" + which]
+    assert torch.equal(native[0][2], f.float())
+
+
+@pytest.mark.parametrize("which", ["prefill", "decode"])
+@pytest.mark.parametrize("what", ["inv_freq", "qkv_dtype", "qkv_columns", "k_dtype", "v_dtype",
+                                  "k_page", "v_pages", "v_strides"])
+def test_rotary_refuses_what_the_kernel_cannot_address(which, what, native):
+    qkv, cache, table, inv_freq = _rotary_case()
+    if what == "inv_freq":
+        inv_freq = inv_freq[:63]
+    elif what == "qkv_dtype":
+        qkv = qkv.float()
+    elif what == "qkv_columns":
+        qkv = qkv[:, :-8]
+    elif what == "k_dtype":
+        cache.k = cache.k.float()
+    elif what == "v_dtype":
+        cache.v = cache.v.to(torch.float16)
+    elif what == "k_page":
+        cache.k = cache.k[..., :8]
+    elif what == "v_pages":
+        cache.v = cache.v[:4]
+    else:
+        cache.v = cache.v.transpose(2, 3).contiguous().transpose(2, 3)
+    with pytest.raises(ValueError):
+        _rotate(which, qkv, cache, table, inv_freq)
+    assert not native
