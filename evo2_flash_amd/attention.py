@@ -300,7 +300,16 @@ def prefill_attention_rows(q, k, vt, scale, out):
     and finite from L on; the result goes to `out` (N, heads, L, 128), a view
     of any strides with unit last one."""
     _lib.require_device(q, k, vt, out)
+    if any(t.dim() != 4 or t.dtype != torch.bfloat16 for t in (q, k, vt, out)):
+        raise ValueError("prefill_attention_rows takes 4-D bf16 q, k, vt, out")
     N, nh, L, hd = q.shape
+    if (k.shape != q.shape or out.shape != q.shape or vt.shape[:3] != (N, nh, hd)
+            or vt.shape[3] < L or vt.shape[3] % 8):
+        raise ValueError(f"prefill_attention_rows: shapes q {tuple(q.shape)}, k {tuple(k.shape)}, "
+                         f"vt {tuple(vt.shape)}, out {tuple(out.shape)} do not match")
+    if not (q.is_contiguous() and k.is_contiguous() and vt.is_contiguous() and out.stride(3) == 1):
+        raise ValueError("prefill_attention_rows takes contiguous q, k, vt and out rows of unit "
+                         "stride")
     _lib.call("evo2_prefill_attention_rows", _lib.ptr(q), _lib.ptr(k), _lib.ptr(vt), _lib.ptr(out),
               out.stride(0), out.stride(1), out.stride(2), N, nh, L, vt.shape[3], hd, float(scale),
               _lib.stream_of(q))

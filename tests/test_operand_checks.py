@@ -84,3 +84,49 @@ def test_rotary_refuses_what_the_kernel_cannot_address(which, what, native):
     with pytest.raises(ValueError):
         _rotate(which, qkv, cache, table, inv_freq)
     assert not native
+
+
+def _rows_case(L=5, Lv=8, N=2, nh=3):
+    z = lambda *s: torch.zeros(*s, dtype=bf)
+    return z(N, nh, L, 128), z(N, nh, L, 128), z(N, nh, 128, Lv), z(N, nh, L, 128)
+
+
+def test_prefill_attention_rows_takes_padded_values_and_any_rows(native):
+    from evo2_flash_amd.attention import prefill_attention_rows
+    q, k, vt, _ = _rows_case()
+    out = torch.zeros(2, 5, 3, 128, dtype=bf).transpose(1, 2)
+    prefill_attention_rows(q, k, vt, 1.0, out)
+    assert [c[0] for c in native] == ["evo2_prefill_attention_rows"]
+
+
+@pytest.mark.parametrize("what", ["dtype", "dims", "k_length", "k_heads", "out_length", "out_rows",
+                                  "vt_planes", "vt_short", "vt_multiple", "q_strides",
+                                  "vt_strides"])
+def test_prefill_attention_rows_refuses_what_the_kernel_cannot_address(what, native):
+    from evo2_flash_amd.attention import prefill_attention_rows
+    q, k, vt, out = _rows_case()
+    if what == "dtype":
+        q = q.to(torch.float16)
+    elif what == "dims":
+        q = q[0]
+    elif what == "k_length":
+        k = k[:, :, :4].contiguous()
+    elif what == "k_heads":
+        k = k[:, :2].contiguous()
+    elif what == "out_length":
+        out = out[:, :, :4]
+    elif what == "out_rows":
+        out = torch.zeros(2, 3, 128, 5, dtype=bf).transpose(2, 3)
+    elif what == "vt_planes":
+        vt = vt[:1]
+    elif what == "vt_short":
+        q, k, _, out = _rows_case(L=9)
+    elif what == "vt_multiple":
+        vt = _rows_case(Lv=12)[2]
+    elif what == "q_strides":
+        q = torch.zeros(2, 5, 3, 128, dtype=bf).transpose(1, 2)
+    else:
+        vt = torch.zeros(2, 3, 8, 128, dtype=bf).transpose(2, 3)
+    with pytest.raises(ValueError):
+        prefill_attention_rows(q, k, vt, 1.0, out)
+    assert not native
