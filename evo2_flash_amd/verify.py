@@ -145,10 +145,15 @@ def _gated_args(zf, state, D, metadata):
     """Checks of the gated calls; (D, g, the arguments both share)."""
     ins, outs, starts, ends, accepted = meta = _meta(metadata)
     _lib.require_device(zf, state, D, *meta)
+    if state.dim() != 3 or state.dtype != torch.float32:
+        raise ValueError(f"state must be a (blocks, H, columns) fp32 view, got "
+                         f"{tuple(state.shape)} {state.dtype}")
     H = state.shape[1]
     if zf.dim() != 2 or zf.shape[1] != 3 * H or zf.dtype != torch.bfloat16 or zf.stride(1) != 1:
         raise ValueError(f"zf must be (T, {3 * H}) bf16 rows, got {tuple(zf.shape)} {zf.dtype}")
     if D is not None:
+        if D.shape != (H,):
+            raise ValueError(f"D must be ({H},), got {tuple(D.shape)}")
         D = D.to(torch.bfloat16).contiguous()
     g = torch.zeros(zf.shape[0], H, dtype=zf.dtype, device=zf.device)
     return D, g, meta, (_lib.ptr(state), *state.stride(), _lib.ptr(ins), *ins.stride(),
@@ -163,6 +168,12 @@ def fir_verify_gated(zf, weight, D, state, metadata, null_block=0):
     fir_snapshots with the gate around it, each step rounded to bf16; (T, H),
     zero on rows no request covers."""
     _lib.require_device(weight)
+    K = weight.shape[1] if weight.dim() == 2 else 0
+    if (K not in (7, 128) or weight.dtype != torch.bfloat16 or weight.shape[0] != state.shape[1]
+            or state.shape[2] < K - 1):
+        raise ValueError(f"fir_verify_gated takes (H, 7 | 128) bf16 taps over a window of K - 1 "
+                         f"columns, got {tuple(weight.shape)} {weight.dtype} on a state "
+                         f"{tuple(state.shape)}")
     D, g, _keep, args = _gated_args(zf, state, D, metadata)
     _lib.call("evo2_fir_verify_gated", _lib.ptr(zf), zf.stride(0), _lib.ptr(weight),
               *weight.stride(), weight.shape[1], _lib.ptr(D), *args, int(null_block),
@@ -174,6 +185,14 @@ def iir_verify_gated(zf, log_poles, residues, D, state, metadata, null_block=0):
     """(LI(x1 v) + D x1 v) * x2 in one launch (fir_verify_gated's form of
     iir_snapshots; poles exp(log_poles) taken in the kernel)."""
     _lib.require_device(log_poles, residues)
+    H = state.shape[1]
+    if (any(t.shape != (H, 16) or t.dtype != torch.float32 for t in (log_poles, residues))
+            or state.shape[2] < 16):
+        raise ValueError(f"iir_verify_gated takes ({H}, 16) fp32 log_poles and residues over a "
+                         f"state of 16 columns, got {tuple(log_poles.shape)} {log_poles.dtype}, "
+                         f"{tuple(residues.shape)} {residues.dtype}, state {tuple(state.shape)}")
+    if log_poles.stride(1) != 1 or log_poles.stride(0) % 4 or log_poles.data_ptr() % 16:
+        log_poles = log_poles.clone(memory_format=torch.contiguous_format)  # rows of float4
     D, g, _keep, args = _gated_args(zf, state, D, metadata)
     _lib.call("evo2_iir_verify_gated", _lib.ptr(zf), zf.stride(0),
               _lib.ptr(log_poles), *log_poles.stride(), _lib.ptr(residues), *residues.stride(),

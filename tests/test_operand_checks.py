@@ -130,3 +130,71 @@ def test_prefill_attention_rows_refuses_what_the_kernel_cannot_address(what, nat
     with pytest.raises(ValueError):
         prefill_attention_rows(q, k, vt, 1.0, out)
     assert not native
+
+
+def _verify_case(columns, H=8, Q=3, n=2):
+    state = torch.zeros(7, H, columns)
+    t = torch.ones(n, Q, dtype=torch.int32)
+    rows = torch.arange(n) * Q
+    meta = (t, t + 1, rows, rows + Q, torch.ones(n, dtype=torch.int64))
+    return torch.zeros(n * Q, 3 * H, dtype=bf), state, torch.zeros(H, dtype=bf), meta
+
+
+@pytest.mark.parametrize("K", [7, 128])
+@pytest.mark.parametrize("what", [None, "taps", "taps_dtype", "taps_rows", "columns", "state_dtype",
+                                  "D"])
+def test_gated_fir_operands(K, what, native):
+    from evo2_flash_amd.verify import fir_verify_gated
+    zf, state, D, meta = _verify_case(K - 1)
+    w = torch.zeros(8, K, dtype=bf)
+    if what == "taps":
+        w = torch.zeros(8, 16, dtype=bf)
+    elif what == "taps_dtype":
+        w = w.float()
+    elif what == "taps_rows":
+        w = w[:7]
+    elif what == "columns":
+        state = state[..., :K - 2]
+    elif what == "state_dtype":
+        state = state.to(bf)
+    elif what == "D":
+        D = D[:7]
+    if what is None:
+        fir_verify_gated(zf, w, D, state, meta)
+        fir_verify_gated(zf, w, None, state, meta)
+        assert [c[0] for c in native] == ["evo2_fir_verify_gated"] * 2
+    else:
+        with pytest.raises(ValueError):
+            fir_verify_gated(zf, w, D, state, meta)
+        assert not native
+
+
+@pytest.mark.parametrize("what", [None, "poles", "poles_dtype", "residues_dtype", "columns", "D"])
+def test_gated_iir_operands(what, native):
+    from evo2_flash_amd.verify import iir_verify_gated
+    zf, state, D, meta = _verify_case(17)
+    lp, res = torch.randn(8, 16), torch.zeros(8, 16)
+    if what == "poles":
+        lp = lp[:, :15]
+    elif what == "poles_dtype":
+        lp = lp.to(bf)
+    elif what == "residues_dtype":
+        res = res.double()
+    elif what == "columns":
+        state = state[..., :15]
+    elif what == "D":
+        D = D.repeat(2)
+    if what is not None:
+        with pytest.raises(ValueError):
+            iir_verify_gated(zf, lp, res, D, state, meta)
+        assert not native
+        return
+    # poles off 16-byte alignment or row-strided arrive as rows of float4
+    wide = torch.zeros(8, 33)
+    wide[:, 1::2] = lp
+    native.look = lambda name, a: (a[2] % 16, a[3:5], _floats(a[2], 128).view(8, 16))
+    for poles in (lp, wide[:, 1::2]):
+        iir_verify_gated(zf, poles, res, D, state, meta)
+    for name, _, (align, strides, seen) in native:
+        assert name == "evo2_iir_verify_gated" and align == 0 and strides == (16, 1)
+        assert torch.equal(seen, lp)
