@@ -359,6 +359,18 @@ def stream_of(t=None):
         torch.cuda.current_device() if t is None else t.get_device())
 
 
+def overlap(a, b):
+    """Whether two tensors' address ranges (first to last element) overlap."""
+    def span(t):
+        last = sum((n - 1) * s for n, s in zip(t.shape, t.stride()))
+        return t.data_ptr(), t.data_ptr() + (last + 1) * t.element_size()
+
+    if a.numel() == 0 or b.numel() == 0:
+        return False
+    (a0, a1), (b0, b1) = span(a), span(b)
+    return a0 < b1 and b0 < a1
+
+
 def require_device(*tensors):
     """The HIP path runs on ROCm devices only: raise for CPU tensors."""
     for t in tensors:

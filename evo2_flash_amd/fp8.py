@@ -152,6 +152,8 @@ def static_fp8_linear(x, weight, input_scale, weight_scale, bias=None, out=None,
     N = weight.shape[0]
     if (x.numel() == K and x.dtype == torch.bfloat16 and x.stride(-1) == 1 and K % 128 == 0
             and 0 < K <= 16384 and (bias is None or bias.shape == (N,))
+            # (in place: each workgroup would quantise x while others store to it)
+            and (out is None or not _lib.overlap(x, out))
             and (out is None or (x.dim() == 2 and out.shape == (1, N) and out.stride(1) == 1
                                  and out.dtype == torch.bfloat16 and out.device == x.device))):
         w = weight if packed is None else packed

@@ -355,3 +355,17 @@ def test_linear_decode_copy_after_loading():
             assert made[1].shape == (N, K) and lin.decode_weight() is made[1]
         outs.append(lin(x)[0])
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("rows", [1, 2])
+def test_static_linear_in_place(rows):
+    """out = x (N = K): the result of a call with an output of its own."""
+    K = 4096
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(K, K, generator=g) * 0.5).to(E4M3).to(DEV)
+    xs, ws = torch.tensor([0.013], device=DEV), torch.tensor([0.3], device=DEV)
+    print(f"fp8 linear in place rows={rows}", flush=True)
+    ref = static_fp8_linear(x, w, xs, ws)
+    assert static_fp8_linear(x, w, xs, ws, out=x).data_ptr() == x.data_ptr()
+    assert torch.equal(x.view(torch.int16), ref.view(torch.int16))

@@ -198,3 +198,20 @@ def test_gated_iir_operands(what, native):
     for name, _, (align, strides, seen) in native:
         assert name == "evo2_iir_verify_gated" and align == 0 and strides == (16, 1)
         assert torch.equal(seen, lp)
+
+
+def test_one_row_fp8_linear_in_place_quantises_apart(native):
+    """static_fp8_linear(x, out=x): x is read whole before any of it is
+    overwritten, so the one-launch form is for outputs beside x only."""
+    from evo2_flash_amd.fp8 import E4M3, static_fp8_linear
+    K = 256
+    buf = torch.zeros(4 * K, dtype=bf)
+    x, one = buf[K:2 * K].view(1, K), torch.ones(1)
+    w = torch.zeros(K, K).to(E4M3)
+    apart, joint = ["evo2_fp8_quantize", "evo2_fp8_gemm"], ["evo2_fp8_quant_gemv"]
+    for out, want in ((x, apart), (buf[K // 2:K // 2 + K].view(1, K), apart),
+                      (buf[2 * K - 1:3 * K - 1].view(1, K), apart), (buf[:K].view(1, K), joint),
+                      (buf[2 * K:3 * K].view(1, K), joint), (None, joint)):
+        static_fp8_linear(x, w, one, one, out=out)
+        assert [c[0] for c in native] == want
+        native.clear()
