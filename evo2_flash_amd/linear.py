@@ -32,12 +32,14 @@ def _plain(*tensors):
 
 def _streams(x, *weights):
     """Whether the weight-streaming kernel takes x (M, K) against weights (N, K)."""
+    # (x on the current device: a launch goes there, and the default stream's
+    # handle is the same on every device; the library's product switches over)
     return (x.dim() == 2 and 0 < x.shape[0] <= STREAM_ROWS and x.shape[1] % 32 == 0
             and x.shape[1] > 0 and all(w.shape == weights[0].shape and w.shape[0] > 0
                                        and w.shape[1] == x.shape[1]
                                        and w.stride() == weights[0].stride()
                                        and w.device == x.device for w in weights)
-            and _plain(x, *weights))
+            and _plain(x, *weights) and x.get_device() == torch.cuda.current_device())
 
 
 def linear(x, weight, bias=None, out=None, residual=None):
@@ -50,10 +52,12 @@ def linear(x, weight, bias=None, out=None, residual=None):
     24.7 / 29.7 against 26.4; 1920 x 5120 11.0 / 14.3 against 18.3 / 10.5."""
     M, (N, K) = x.shape[0], weight.shape
     if (_streams(x, weight) and (M <= 8 or (N * K <= 1 << 24 and K <= 4096))
-            and (bias is None or (bias.is_cuda and bias.dtype == x.dtype and bias.shape == (N,)
+            and (bias is None or (bias.device == x.device and bias.dtype == x.dtype
+                                  and bias.shape == (N,)
                                   and bias.is_contiguous()
                                   and not (torch.is_grad_enabled() and bias.requires_grad)))
-            and (residual is None or (residual.shape == (M, N) and _plain(residual)))
+            and (residual is None or (residual.shape == (M, N) and residual.device == x.device
+                                      and _plain(residual)))
             and (out is None or (out.shape == (M, N) and out.dtype == x.dtype
                                  and out.stride(1) == 1 and out.device == x.device))):
         y = torch.empty(M, N, dtype=x.dtype, device=x.device) if out is None else out

@@ -87,3 +87,21 @@ def test_calls_that_stay_on_the_library(monkeypatch):
     assert torch.equal(linear(odd, w), F(odd, w))
     assert linear(x.float(), w.float()).dtype == torch.float32
     assert calls == []
+
+
+def test_operands_off_the_current_device_stay_on_the_library(monkeypatch):
+    """x on a device that is not the current one (here by the current device's
+    number): no launch of the package's own."""
+    x, w = _rand(4, 64, seed=12), _rand(64, 64, seed=13)
+    calls = []
+    monkeypatch.setattr(_lib, "call", lambda n, *a: calls.append(n))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert torch.equal(linear(x, w), torch.nn.functional.linear(x, w))
+    z = torch.nn.functional.linear(x, w)
+    assert torch.equal(gated(x, w, w, False), z * z)
+    assert calls == []
+    monkeypatch.undo()
+    with pytest.raises(RuntimeError):                  # the library's own refusal
+        linear(x, w, bias=torch.zeros(64, dtype=bf))
+    with pytest.raises(RuntimeError):
+        linear(x, w, residual=torch.zeros(4, 64, dtype=bf))
