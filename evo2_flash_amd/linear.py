@@ -14,8 +14,10 @@ STREAM_ROWS = 16  # the kernel's most rows
 
 def _plain(*tensors):
     """Whether these are ordinary CUDA bf16 tensors outside every transform (no
-    tracing, autocast, vmap, gradients of either mode), 16-byte aligned rows."""
-    if torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda"):
+    tracing or dispatch mode, autocast, vmap, gradients of either mode), 16-byte
+    aligned rows."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._len_torch_dispatch_stack() > 0 or torch.is_autocast_enabled("cuda")):
         return False
     if forward_ad._current_level >= 0:
         return False
@@ -32,6 +34,8 @@ def _plain(*tensors):
 
 def _streams(x, *weights):
     """Whether the weight-streaming kernel takes x (M, K) against weights (N, K)."""
+    if torch.jit.is_tracing():  # (_plain's, before a shape is compared in the trace)
+        return False
     # (x on the current device: a launch goes there, and the default stream's
     # handle is the same on every device; the library's product switches over)
     return (x.dim() == 2 and 0 < x.shape[0] <= STREAM_ROWS and x.shape[1] % 32 == 0

@@ -105,3 +105,16 @@ def test_operands_off_the_current_device_stay_on_the_library(monkeypatch):
         linear(x, w, bias=torch.zeros(64, dtype=bf))
     with pytest.raises(RuntimeError):
         linear(x, w, residual=torch.zeros(4, 64, dtype=bf))
+
+
+def test_traced_calls_stay_in_the_graph():
+    """torch.jit.trace and make_fx see a product, not a constant: the traced
+    call follows new inputs."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    w, w2 = _rand(64, 64, seed=14), _rand(64, 64, seed=15)
+    x, y = _rand(4, 64, seed=16), _rand(4, 64, seed=17)
+    F = torch.nn.functional.linear
+    for fn, want in ((lambda t: linear(t, w), F(y, w)),
+                     (lambda t: gated(t, w, w2, False), F(y, w) * F(y, w2))):
+        assert torch.equal(torch.jit.trace(fn, x, check_trace=False)(y), want)
+        assert torch.equal(make_fx(fn)(x)(y), want)
