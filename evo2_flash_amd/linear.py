@@ -63,7 +63,10 @@ def linear(x, weight, bias=None, out=None, residual=None):
             and (residual is None or (residual.shape == (M, N) and residual.device == x.device
                                       and _plain(residual)))
             and (out is None or (out.shape == (M, N) and out.dtype == x.dtype
-                                 and out.stride(1) == 1 and out.device == x.device))):
+                                 and out.stride(1) == 1 and out.device == x.device
+                                 # (the kernel stores while others still read)
+                                 and not _lib.overlap(x, out)
+                                 and (residual is None or not _lib.overlap(residual, out))))):
         y = torch.empty(M, N, dtype=x.dtype, device=x.device) if out is None else out
         _lib.call("evo2_bf16_stream_linear", _lib.ptr(x), x.stride(0), _lib.ptr(weight),
                   weight.stride(0), _lib.ptr(bias), _lib.ptr(residual),
@@ -73,11 +76,13 @@ def linear(x, weight, bias=None, out=None, residual=None):
     if out is None:
         y = torch.nn.functional.linear(x, weight, bias)
         return y if residual is None else y + residual
+    if residual is not None:  # (which may be `out`: the product goes beside it)
+        return torch.add(torch.nn.functional.linear(x, weight, bias), residual, out=out)
     if bias is not None:
         torch.addmm(bias, x, weight.t(), out=out)
     else:
         torch.mm(x, weight.t(), out=out)
-    return out if residual is None else out.add_(residual)
+    return out
 
 
 def gated(x, w1, w2, gelu):

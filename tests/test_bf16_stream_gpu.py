@@ -118,3 +118,20 @@ def test_traced_calls_stay_in_the_graph():
                      (lambda t: gated(t, w, w2, False), F(y, w) * F(y, w2))):
         assert torch.equal(torch.jit.trace(fn, x, check_trace=False)(y), want)
         assert torch.equal(make_fx(fn)(x)(y), want)
+
+
+def test_outputs_over_inputs(monkeypatch):
+    """out over the residual: the library's product, which refuses a part of it;
+    beside it: the kernel."""
+    x, w, r = _rand(8, 64, seed=18), _rand(64, 64, seed=19), _rand(9, 64, seed=20)
+    calls = []
+    call = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda n, *a: (calls.append(n), call(n, *a)))
+    want = torch.nn.functional.linear(x, w) + r[:8]
+    buf = r.clone()
+    assert torch.equal(linear(x, w, residual=buf[:8], out=buf[:8]), want)
+    with pytest.raises(RuntimeError):
+        linear(x, w, residual=buf[:8], out=buf[1:])
+    assert calls == []
+    linear(x, w, residual=r[:8], out=torch.empty_like(want))
+    assert calls == ["evo2_bf16_stream_linear"]

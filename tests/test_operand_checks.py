@@ -215,3 +215,22 @@ def test_one_row_fp8_linear_in_place_quantises_apart(native):
         static_fp8_linear(x, w, one, one, out=out)
         assert [c[0] for c in native] == want
         native.clear()
+
+
+@pytest.mark.parametrize("M", [4, 33])
+@pytest.mark.parametrize("bias", [False, True])
+def test_linear_adds_a_residual_that_is_its_output(M, bias):
+    """out = residual: product plus residual, not twice the product."""
+    from evo2_flash_amd.linear import linear
+    x, w, r = torch.randn(M, 64), torch.randn(32, 64), torch.randn(M, 32)
+    b = torch.randn(32) if bias else None
+    want = torch.nn.functional.linear(x, w, b) + r
+    assert linear(x, w, b, out=r, residual=r).data_ptr() == r.data_ptr()
+    assert torch.equal(r, want)
+
+
+def test_overlap():
+    t = torch.zeros(6, 8, dtype=bf)
+    assert _lib.overlap(t, t[5:]) and _lib.overlap(t[:, :4], t[:, 4:])    # the ranges, not the elements
+    assert not _lib.overlap(t[:3], t[3:]) and not _lib.overlap(t, t[:0])
+    assert _lib.overlap(t[0], t.view(-1)[7:9]) and not _lib.overlap(t[0], t.view(-1)[8:9])
