@@ -41,6 +41,15 @@ from .state import HyenaStatePool, get_mamba_state_copy_func
 from .synthetic import mixer_params
 
 
+def _bare(module, cls):
+    """Whether calling `module` runs cls.forward and nothing else: no subclass or
+    replacement, no hooks (its own or global ones), no forward of the instance."""
+    hooks = torch.nn.modules.module
+    return (type(module) is cls and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                     or module._backward_pre_hooks or hooks._has_any_global_hook()))
+
+
 class Evo2MLP(nn.Module):
     """l3(act(l1 x) * l2 x), act = GELU on layer 0 only (model.py:77-101)."""
 
@@ -52,10 +61,19 @@ class Evo2MLP(nn.Module):
         self.use_act = use_act
 
     def forward(self, x, residual=None):
-        """The MLP's output, plus `residual` (the layer's input) when given."""
-        z = gated(x, self.l1.weight, self.l2.weight, self.use_act)
-        out, _ = self.l3(z, residual=residual)
-        return out
+        """The MLP's output, plus `residual` (the layer's input) when given.
+        Projections of another type, with a bias or with hooks are called as
+        modules, and l3's hooks see its output without the residual."""
+        if all(_bare(m, Linear) and m.bias is None for m in (self.l1, self.l2)):
+            z = gated(x, self.l1.weight, self.l2.weight, self.use_act)
+        else:
+            z1, _ = self.l1(x)
+            z2, _ = self.l2(x)
+            z = (nn.functional.gelu(z1) if self.use_act else z1) * z2
+        if residual is not None and _bare(self.l3, Linear):
+            return self.l3(z, residual=residual)[0]
+        out, _ = self.l3(z)
+        return out if residual is None else out + residual
 
 
 def rotary_neox(x, positions, inv_freq, factor):
@@ -143,6 +161,11 @@ class Evo2DecoderLayer(nn.Module):
         self.mixer = mixer
         self.mlp = Evo2MLP(h, config.intermediate_size, use_act=(i == 0), device=device)
 
+    def _mlp(self, post, x):
+        """The MLP's output plus x (an MLP of another type or with hooks gives
+        its own output)."""
+        return self.mlp(post, residual=x) if _bare(self.mlp, Evo2MLP) else self.mlp(post) + x
+
     def forward(self, positions, x, token_ids, block_table):
         """One decode token per sequence."""
         pre = self.pre_norm(x)
@@ -151,7 +174,7 @@ class Evo2DecoderLayer(nn.Module):
         else:
             m = self.mixer(pre, token_ids=token_ids)
         post, x = self.post_norm(m, x)
-        return self.mlp(post, residual=x)
+        return self._mlp(post, x)
 
     def forward_prefill(self, x, token_ids, nseq, L, block_table):
         """Prompts of L tokens of nseq sequences, packed (nseq * L, H); the
@@ -163,7 +186,7 @@ class Evo2DecoderLayer(nn.Module):
         else:
             m = self.mixer(pre, token_ids=token_ids)
         post, x = self.post_norm(m, x)
-        return self.mlp(post, residual=x)
+        return self._mlp(post, x)
 
 
 class Evo2DecodeModel(nn.Module):

@@ -234,3 +234,90 @@ def test_overlap():
     assert _lib.overlap(t, t[5:]) and _lib.overlap(t[:, :4], t[:, 4:])    # the ranges, not the elements
     assert not _lib.overlap(t[:3], t[3:]) and not _lib.overlap(t, t[:0])
     assert _lib.overlap(t[0], t.view(-1)[7:9]) and not _lib.overlap(t[0], t.view(-1)[8:9])
+
+
+def _layer(H=8, inter=12):
+    """A decoder layer whose norms and mixer are stand-ins that run on the CPU."""
+    from evo2_flash_amd.config import HyenaConfig
+    from evo2_flash_amd.model import Evo2DecoderLayer
+    cfg = HyenaConfig(hidden_size=H, intermediate_size=inter, num_hidden_layers=1,
+                      hcs_layer_idxs=[0])
+    layer = Evo2DecoderLayer(cfg, 0, lambda x, token_ids: x)
+    layer.pre_norm = torch.nn.Identity()
+    layer.post_norm = type("Norm", (torch.nn.Module,), {"forward": lambda self, m, x: (m, x)})()
+    for p in layer.mlp.parameters():
+        p.data.copy_(torch.randn(p.shape))
+    return layer
+
+
+def _mlp_ref(mlp, x, gelu=True):
+    F = torch.nn.functional
+    z1 = F.linear(x, mlp.l1.weight)
+    return F.linear((F.gelu(z1) if gelu else z1) * F.linear(x, mlp.l2.weight), mlp.l3.weight)
+
+
+def test_mlp_hooks_see_the_module_outputs():
+    """Hooks on l1, l2, l3 and the MLP run and see each module's own output, the
+    layer's input not in it; the layer's result does not change."""
+    layer = _layer()
+    x = torch.randn(3, 8).to(bf)
+    plain = layer(None, x, None, None)
+    seen = {}
+    for name in ("l1", "l2", "l3"):
+        getattr(layer.mlp, name).register_forward_hook(
+            lambda m, a, out, name=name: seen.__setitem__(name, out[0]))
+    layer.mlp.register_forward_hook(lambda m, a, out: seen.__setitem__("mlp", out))
+    assert torch.equal(layer(None, x, None, None), plain)
+    mlp, F = layer.mlp, torch.nn.functional
+    ref = _mlp_ref(mlp, x)
+    assert torch.equal(seen["l1"], F.linear(x, mlp.l1.weight))
+    assert torch.equal(seen["l2"], F.linear(x, mlp.l2.weight))
+    assert torch.equal(seen["l3"], ref) and torch.equal(seen["mlp"], ref)
+    assert torch.equal(plain, ref + x)
+
+
+@pytest.mark.parametrize("what", ["module_bias", "replaced", "instance_forward", "global_hook",
+                                  "mlp"])
+def test_mlp_calls_what_stands_in_its_place(what):
+    from evo2_flash_amd.mixers import Linear
+    layer = _layer()
+    mlp = layer.mlp
+    x = torch.randn(3, 8).to(bf)
+    ref = _mlp_ref(mlp, x)
+    called = []
+    if what == "module_bias":
+        w = mlp.l2.weight
+        mlp.l2 = Linear(8, 12, bias=True)
+        mlp.l2.weight.data.copy_(w)
+        mlp.l2.bias.data.fill_(2.0)
+        F = torch.nn.functional
+        z1 = F.gelu(F.linear(x, mlp.l1.weight))
+        ref = F.linear(z1 * F.linear(x, w, mlp.l2.bias), mlp.l3.weight)
+    elif what == "replaced":
+        class Twice(torch.nn.Module):
+            def forward(self, t):
+                called.append("l")
+                return torch.nn.functional.linear(t, self.inner.weight), None
+        twice = Twice()
+        twice.inner, mlp.l1 = mlp.l1, twice
+        plain, mlp.l3 = mlp.l3, Twice()
+        mlp.l3.inner = plain
+    elif what == "instance_forward":
+        inner = mlp.l2.forward
+        mlp.l2.forward = lambda t: (called.append("l2"), inner(t))[1]
+    elif what == "global_hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(
+            lambda m, a, out: called.append(type(m).__name__))
+    else:
+        class Own(torch.nn.Module):
+            def forward(self, t):
+                return -t
+        layer.mlp, ref = Own(), -x
+    try:
+        got = layer(None, x, None, None)
+    finally:
+        if what == "global_hook":
+            handle.remove()
+    assert torch.equal(got, ref + x)
+    assert {"replaced": called == ["l", "l"], "instance_forward": called == ["l2"],
+            "global_hook": called.count("Linear") == 3}.get(what, not called)
