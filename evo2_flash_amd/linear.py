@@ -12,7 +12,7 @@ from . import _lib
 STREAM_ROWS = 16  # the kernel's most rows
 
 
-def _plain(*tensors):
+def plain(*tensors):
     """Whether these are ordinary CUDA bf16 tensors outside every transform (no
     tracing or dispatch mode, autocast, vmap, gradients of either mode), 16-byte
     aligned rows."""
@@ -34,7 +34,7 @@ def _plain(*tensors):
 
 def _streams(x, *weights):
     """Whether the weight-streaming kernel takes x (M, K) against weights (N, K)."""
-    if torch.jit.is_tracing():  # (_plain's, before a shape is compared in the trace)
+    if torch.jit.is_tracing():  # (plain's, before a shape is compared in the trace)
         return False
     # (x on the current device: a launch goes there, and the default stream's
     # handle is the same on every device; the library's product switches over)
@@ -43,7 +43,7 @@ def _streams(x, *weights):
                                        and w.shape[1] == x.shape[1]
                                        and w.stride() == weights[0].stride()
                                        and w.device == x.device for w in weights)
-            and _plain(x, *weights) and x.get_device() == torch.cuda.current_device())
+            and plain(x, *weights) and x.get_device() == torch.cuda.current_device())
 
 
 def linear(x, weight, bias=None, out=None, residual=None):
@@ -61,7 +61,7 @@ def linear(x, weight, bias=None, out=None, residual=None):
                                   and bias.is_contiguous()
                                   and not (torch.is_grad_enabled() and bias.requires_grad)))
             and (residual is None or (residual.shape == (M, N) and residual.device == x.device
-                                      and _plain(residual)))
+                                      and plain(residual)))
             and (out is None or (out.shape == (M, N) and out.dtype == x.dtype
                                  and out.stride(1) == 1 and out.device == x.device
                                  # (the kernel stores while others still read)
@@ -99,4 +99,4 @@ def gated(x, w1, w2, gelu):
     return (torch.nn.functional.gelu(z1) if gelu else z1) * z2
 
 
-__all__ = ["linear", "gated", "STREAM_ROWS"]
+__all__ = ["linear", "gated", "plain", "STREAM_ROWS"]

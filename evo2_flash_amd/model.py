@@ -33,7 +33,7 @@ from torch import nn
 from .attention import (PAGE, PagedKVCache, causal_prefill_attention, check_block_table,
                         paged_decode_attention, prefill_attention_rows, rotary_decode,
                         rotary_prefill, shared_prefix_pages, workspace as attention_workspace)
-from .linear import gated, linear
+from .linear import gated, linear, plain
 from .metadata import build_metadata
 from .mixers import Linear, load_mixer_params, make_mixer, set_forward_context
 from .norm import Evo2RMSNorm
@@ -107,10 +107,8 @@ class Evo2Attention(nn.Module):
         self._attn_ws = attention_workspace(max_batch, self.heads, self.hd, max_pages * PAGE,
                                             device)
 
-    def _qkv(self, x, positions):
-        n = x.shape[0]
-        qkv, _ = self.qkv_proj(x)
-        q, k, v = qkv.view(n, 3, self.heads, self.hd).unbind(1)
+    def _rotated(self, qkv, positions):
+        q, k, v = qkv.view(qkv.shape[0], 3, self.heads, self.hd).unbind(1)
         return (rotary_neox(q, positions, self.inv_freq, self.rope_factor),
                 rotary_neox(k, positions, self.inv_freq, self.rope_factor), v)
 
@@ -129,17 +127,20 @@ class Evo2Attention(nn.Module):
     def forward_prefill(self, x, nseq, L, block_table):
         """x (nseq * L, H): prompts of L tokens (positions 0..L-1) of sequences
         0..nseq-1 of `block_table`, packed in order."""
-        if x.is_cuda and self.hd == 128 and not (torch.is_grad_enabled() and x.requires_grad):
-            qkv, _ = self.qkv_proj(x)
+        qkv, _ = self.qkv_proj(x)
+        # rows of a plain product (no gradient, of a weight's either, no tracing
+        # or autocast), in the kernels' type, grid and device
+        if (self.hd == 128 and nseq <= 65535 and plain(qkv)
+                and qkv.get_device() == torch.cuda.current_device()):
             q, k, vt = rotary_prefill(qkv, self.cache, block_table, self.inv_freq,
                                       self.rope_factor, nseq, L)
-            out = torch.empty(nseq, L, self.heads, self.hd, dtype=x.dtype, device=x.device)
+            out = torch.empty(nseq, L, self.heads, self.hd, dtype=qkv.dtype, device=qkv.device)
             prefill_attention_rows(q, k, vt, self.hd ** -0.5, out.transpose(1, 2))
             o, _ = self.o_proj(out.view(nseq * L, self.heads * self.hd))
             return o
-        # other head dims, the CPU, and a differentiated input
+        # other head dims, the CPU, and what needs torch's operators
         pos = torch.arange(L, device=x.device).repeat(nseq)
-        q, k, v = self._qkv(x, pos)
+        q, k, v = self._rotated(qkv, pos)
         shape = (nseq, L, self.heads, self.hd)
         q, k, v = (t.reshape(shape).transpose(1, 2).contiguous() for t in (q, k, v))
         self.cache.write_prompt(k, v, block_table)

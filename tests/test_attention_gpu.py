@@ -382,3 +382,40 @@ def test_attention_layer_cast_to_bf16(L):
             want = rotary_neox(k, pos, layer.inv_freq, 4.0)
             page = table[0, pos // PAGE].long()
             assert torch.equal(layer.cache.k[page, :, :, pos % PAGE], want)
+
+
+@pytest.mark.parametrize("trained", ["qkv_proj", "x"])
+def test_attention_layer_gradient_at_odd_lengths(trained):
+    """A prompt whose length is no multiple of 8 is differentiable, in the input
+    and in a trained qkv_proj.weight: the gradient of an fp32 layer, the output
+    of the layer without gradients."""
+    from evo2_flash_amd.config import HyenaConfig
+    from evo2_flash_amd.model import Evo2Attention, rotary_neox
+    cfg = HyenaConfig(hidden_size=256, num_attention_heads=2, num_hidden_layers=1,
+                      attn_layer_idxs=[0])
+    L = 41
+    layer = Evo2Attention(cfg, 9, 4, 1, rope_factor=4.0, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    for p in layer.parameters():
+        p.data.copy_(torch.randn(p.shape, generator=g, device=DEV) * 0.05)
+    table = torch.tensor([[5, 2, 7, 1]], dtype=torch.int32, device=DEV)
+    x = torch.randn(L, 256, generator=g, device=DEV).to(bf)
+    go = torch.randn(L, 256, generator=g, device=DEV).to(bf)
+    print(f"attention layer gradient of {trained}", flush=True)
+    plain = layer.forward_prefill(x, 1, L, table)
+    leaf = (layer.qkv_proj.weight if trained == "qkv_proj" else x).requires_grad_()
+    out = layer.forward_prefill(x, 1, L, table)
+    out.backward(go)
+    assert max_rel_err(out.detach(), plain) <= 1e-2
+    # the same in fp32 on the CPU
+    xr, wr = x.detach().cpu().float(), layer.qkv_proj.weight.detach().cpu().float()
+    ref = (wr if trained == "qkv_proj" else xr).requires_grad_()
+    q, k, v = (xr @ wr.t()).view(L, 3, 2, 128).unbind(1)
+    pos, f = torch.arange(L), layer.inv_freq.cpu()
+    q, k = rotary_neox(q, pos, f, 4.0), rotary_neox(k, pos, f, 4.0)
+    s = torch.einsum("ihd,jhd->hij", q, k) * 128 ** -0.5
+    s = s.masked_fill(torch.ones(L, L).triu(1).bool(), float("-inf"))
+    o = torch.einsum("hij,jhd->ihd", s.softmax(-1), v).reshape(L, 256)
+    o = o @ layer.o_proj.weight.detach().cpu().float().t()
+    o.backward(go.cpu().float())
+    assert max_rel_err(leaf.grad.cpu().float(), ref.grad) <= 2e-2   # some ten roundings of 2^-9
