@@ -188,9 +188,9 @@ class PagedKVCache:
 
 
 def _rotary_operands(qkv, cache, inv_freq):
-    """Checks of what both rotary launches read by address: the pages and the
-    frequencies, returned as contiguous fp32 (a module cast to bf16 casts its
-    buffer with it)."""
+    """Checks of what both rotary launches read by address; (qkv, heads,
+    head_dim, inv_freq), qkv as rows of unit stride and the frequencies as
+    contiguous fp32 (a module cast to bf16 casts its buffer with it)."""
     nh, hd = cache.k.shape[1], cache.k.shape[2]
     if (cache.k.dtype != torch.bfloat16 or cache.v.dtype != torch.bfloat16
             or cache.k.shape[3:] != (PAGE,) or cache.v.shape != (cache.k.shape[0], nh, PAGE, hd)
@@ -201,26 +201,39 @@ def _rotary_operands(qkv, cache, inv_freq):
                          f"{cache.v.dtype}")
     if inv_freq.shape != (hd // 2,):
         raise ValueError(f"inv_freq must be ({hd // 2},), got {tuple(inv_freq.shape)}")
-    if qkv.dim() != 2 or qkv.shape[1] != 3 * nh * hd or qkv.dtype != torch.bfloat16 \
-            or qkv.stride(1) != 1:
+    if qkv.dim() != 2 or qkv.shape[1] != 3 * nh * hd or qkv.dtype != torch.bfloat16:
         raise ValueError(f"qkv must be bf16 rows of {3 * nh * hd}, got {tuple(qkv.shape)} "
                          f"{qkv.dtype}")
-    return nh, hd, inv_freq.to(torch.float32).contiguous()
+    if qkv.stride(1) != 1:
+        qkv = qkv.contiguous()
+    return qkv, nh, hd, inv_freq.to(torch.float32).contiguous()
+
+
+def _page_table(block_table, rows, num_pages, device):
+    """The first `rows` rows of a block table as the kernels read it: int32 with
+    unit column stride on `device`.  Tables of other integer types, strides or
+    devices are converted (an entry outside the pages to -1, which is not
+    written through)."""
+    if block_table.dim() != 2 or block_table.shape[0] < rows:
+        raise ValueError(f"block_table {tuple(block_table.shape)} cannot serve {rows} sequences")
+    table = block_table[:rows]
+    if table.dtype != torch.int32:
+        table = table.to(torch.int64)
+        table = torch.where((table >= 0) & (table < num_pages), table, -1).to(torch.int32)
+    return table.to(device) if table.stride(1) == 1 else table.to(device).contiguous()
 
 
 def rotary_prefill(qkv, cache, block_table, inv_freq, factor, nseq, L):
     """Rotary and cache write of nseq prompts of L tokens in one launch: qkv
     (nseq * L, 3 * heads * 128) bf16 rows (q | k | v).  Writes k and v into
-    `cache`'s pages (block_table (>= nseq, pages) int32) and returns the
+    `cache`'s pages (block_table (>= nseq, pages), any integer type) and returns the
     operands of prefill attention: q, k (nseq, heads, L, 128) rotated, and the
     values transposed, (nseq, heads, 128, L rounded up to 8), zeros from L on."""
-    _lib.require_device(qkv, cache.k, cache.v, block_table, inv_freq)
-    nh, hd, inv_freq = _rotary_operands(qkv, cache, inv_freq)
+    _lib.require_device(qkv, cache.k, cache.v, inv_freq)
+    qkv, nh, hd, inv_freq = _rotary_operands(qkv, cache, inv_freq)
     if qkv.shape[0] != nseq * L:
         raise ValueError(f"qkv must have {nseq * L} rows, got {qkv.shape[0]}")
-    if (block_table.dtype != torch.int32 or block_table.stride(1) != 1
-            or block_table.shape[0] < nseq):
-        raise ValueError("block_table must be (>= nseq, pages) int32 with unit column stride")
+    block_table = _page_table(block_table, nseq, cache.k.shape[0], qkv.device)
     Lv = -(-L // 8) * 8
     q = torch.empty(nseq, nh, L, hd, dtype=qkv.dtype, device=qkv.device)
     k = torch.empty_like(q)
@@ -238,10 +251,9 @@ def rotary_decode(qkv, cache, block_table, positions, inv_freq, factor):
     (B, 3 * heads * head_dim) bf16 rows (q | k | v) at positions (B,) int64.
     Writes k and v into `cache`'s pages and returns q (B, heads, head_dim)."""
     _lib.require_device(qkv, cache.k, cache.v, block_table, positions, inv_freq)
-    nh, hd, inv_freq = _rotary_operands(qkv, cache, inv_freq)
+    qkv, nh, hd, inv_freq = _rotary_operands(qkv, cache, inv_freq)
     B = qkv.shape[0]
-    if block_table.dtype != torch.int32 or block_table.stride(1) != 1 or block_table.shape[0] < B:
-        raise ValueError("block_table must be (>= B, pages) int32 with unit column stride")
+    block_table = _page_table(block_table, B, cache.k.shape[0], qkv.device)
     if positions.shape != (B,):
         raise ValueError(f"positions must be ({B},), got {tuple(positions.shape)}")
     positions = positions.to(torch.int64).contiguous()

@@ -419,3 +419,22 @@ def test_attention_layer_gradient_at_odd_lengths(trained):
     o = o @ layer.o_proj.weight.detach().cpu().float().t()
     o.backward(go.cpu().float())
     assert max_rel_err(leaf.grad.cpu().float(), ref.grad) <= 2e-2   # some ten roundings of 2^-9
+
+
+@pytest.mark.parametrize("form", ["int64", "cpu", "strided"])
+def test_rotary_prefill_block_table_forms(form):
+    """Tables that PagedKVCache.write_prompt takes: the pages an int32 table on
+    the device gives."""
+    from evo2_flash_amd.attention import rotary_prefill
+    hd, nh, nseq, L = 128, 2, 2, 40
+    g, wide, inv_freq = _qkv_case(nseq * L, nh, hd, 5)
+    table = (torch.randperm(6, generator=g) + 1).view(nseq, 3)
+    given = {"int64": table.to(DEV), "cpu": table,
+             "strided": table.int().t().contiguous().to(DEV).t()}[form]
+    caches = []
+    print(f"rotary_prefill block table {form}", flush=True)
+    for t in (table.int().to(DEV), given):
+        caches.append(PagedKVCache(7, nh, hd, DEV))
+        rotary_prefill(wide.to(DEV)[:, :3 * nh * hd], caches[-1], t, inv_freq.to(DEV), 1.0, nseq, L)
+    assert torch.equal(caches[0].k, caches[1].k) and torch.equal(caches[0].v, caches[1].v)
+    assert (caches[0].k[1:].abs().amax((1, 2, 3)) > 0).all()

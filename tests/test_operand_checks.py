@@ -321,3 +321,47 @@ def test_mlp_calls_what_stands_in_its_place(what):
     assert torch.equal(got, ref + x)
     assert {"replaced": called == ["l", "l"], "instance_forward": called == ["l2"],
             "global_hook": called.count("Linear") == 3}.get(what, not called)
+
+
+@pytest.mark.parametrize("which", ["prefill", "decode"])
+@pytest.mark.parametrize("form", ["int64", "int16", "uint8", "columns", "transposed"])
+def test_rotary_block_tables_of_any_integer_type_and_stride(which, form, native):
+    """The kernel reads int32 entries at unit column stride; an int64 entry past
+    32 bits does not wrap onto a page."""
+    qkv, cache, _, inv_freq = _rotary_case()
+    want = torch.tensor([[3, 1], [2, 4], [4, 2], [1, 3]])
+    table = {"int64": want.clone(), "int16": want.short(), "uint8": want.byte(),
+             "columns": want.int().repeat_interleave(2, 1)[:, ::2],
+             "transposed": want.int().t().contiguous().t()}[form]
+    if form == "int64":
+        table[0, 1], table[1, 1], table[2, 1] = (1 << 32) + 1, -3, 5
+        want[0, 1] = want[1, 1] = want[2, 1] = -1                # five pages: 0 .. 4
+    n = 1 if which == "prefill" else 4
+
+    def look(name, a):
+        i = 17 if which == "prefill" else 14                     # table, row stride, columns
+        assert a[i + 2] == 2
+        flat = (ctypes.c_int32 * (a[i + 1] * (n - 1) + 2)).from_address(a[i])
+        return [[flat[a[i + 1] * r + c] for c in (0, 1)] for r in range(n)]
+
+    native.look = look
+    _rotate(which, qkv, cache, table, inv_freq)
+    assert native[0][2] == want[:n].tolist()
+
+
+@pytest.mark.parametrize("which", ["prefill", "decode"])
+def test_rotary_takes_rows_of_any_stride(which, native):
+    qkv, cache, table, inv_freq = _rotary_case()
+    wide = torch.zeros(qkv.shape[0], 2 * qkv.shape[1], dtype=bf)
+    wide[:, ::2] = qkv
+
+    def look(name, a):
+        flat = (ctypes.c_int16 * qkv.numel()).from_address(a[0])
+        return torch.tensor(flat, dtype=torch.int16).view(bf).view(qkv.shape), a[1]
+
+    native.look = look
+    _rotate(which, wide[:, ::2], cache, table, inv_freq)
+    seen, stride = native[0][2]
+    assert torch.equal(seen, qkv) and stride == qkv.shape[1]
+    with pytest.raises(ValueError):
+        _rotate(which, qkv, cache, table[:0], inv_freq)
