@@ -228,13 +228,14 @@ def rotary_prefill(qkv, cache, block_table, inv_freq, factor, nseq, L):
     (nseq * L, 3 * heads * 128) bf16 rows (q | k | v).  Writes k and v into
     `cache`'s pages (block_table (>= nseq, pages), any integer type) and returns the
     operands of prefill attention: q, k (nseq, heads, L, 128) rotated, and the
-    values transposed, (nseq, heads, 128, L rounded up to 8), zeros from L on."""
+    values transposed, (nseq, heads, 128, L rounded up to 128), zeros from L on
+    (whole key blocks: the kernel reads no row's values for another's)."""
     _lib.require_device(qkv, cache.k, cache.v, inv_freq)
     qkv, nh, hd, inv_freq = _rotary_operands(qkv, cache, inv_freq)
     if qkv.shape[0] != nseq * L:
         raise ValueError(f"qkv must have {nseq * L} rows, got {qkv.shape[0]}")
     block_table = _page_table(block_table, nseq, cache.k.shape[0], qkv.device)
-    Lv = -(-L // 8) * 8
+    Lv = -(-L // 128) * 128
     q = torch.empty(nseq, nh, L, hd, dtype=qkv.dtype, device=qkv.device)
     k = torch.empty_like(q)
     vt = torch.empty(nseq, nh, hd, Lv, dtype=qkv.dtype, device=qkv.device)
@@ -309,7 +310,8 @@ def prefill_attention(q, k, v, scale):
 def prefill_attention_rows(q, k, vt, scale, out):
     """The kernel of prefill_attention for any L: q, k (N, heads, L, 128)
     contiguous, vt (N, heads, 128, Lv) contiguous with Lv >= L a multiple of 8
-    and finite from L on; the result goes to `out` (N, heads, L, 128), a view
+    and finite from L on (a multiple of 128 where values may be infinite or NaN:
+    else a row's first ones also reach the row before); the result goes to `out` (N, heads, L, 128), a view
     of any strides with unit last one."""
     _lib.require_device(q, k, vt, out)
     if any(t.dim() != 4 or t.dtype != torch.bfloat16 for t in (q, k, vt, out)):

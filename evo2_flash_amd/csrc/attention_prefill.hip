@@ -96,7 +96,8 @@ __global__ __launch_bounds__(AP_NW * 64, 1) void attn_prefill_kernel(PrefillArgs
   // Buffer loads over the (sequence, head) plane: a lane's offset within the
   // block is fixed, the block's in an SGPR; key rows past the prompt read
   // zeros (past the plane), value chunks past it the padding, the next row's
-  // first keys or zeros, finite values whose probabilities are 0.
+  // first keys (with Lv off whole blocks) or zeros, finite values whose
+  // probabilities are 0.
   const uint32_t pbytes = static_cast<uint32_t>(p.plane * 2);
   const uint32_t vbytes = static_cast<uint32_t>(p.Lv) * (AP_HD * 2u);
   const __amdgpu_buffer_rsrc_t krs =

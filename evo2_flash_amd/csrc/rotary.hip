@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void rotary_prefill_kernel(RotaryArgs p) {
   const int t0 = blockIdx.x * RP_T;
   const int n = blockIdx.z;
   const int64_t h3 = static_cast<int64_t>(p.heads) * RP_HD;  // elements of q in a row
-  const int nt = min(RP_T, p.L - t0);                        // positions of the prompt here
+  const int nt = min(RP_T, p.L - t0);  // positions of the prompt here (none: values' padding only)
   for (int i = tid; i < RP_T * (RP_HD / 2); i += 256) {
     const int t = i / (RP_HD / 2), f = i % (RP_HD / 2);
     float s, c;
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256) void rotary_prefill_kernel(RotaryArgs p) {
     const int64_t page = p.table[n * p.st + t0 / 16 + pg];
     return page >= 0 && page < p.num_pages ? page : -1;  // no write outside the cache
   };
-  const int npg = (nt + 15) / 16;  // pages with a position of the prompt (the last one zero-padded)
+  const int npg = nt > 0 ? (nt + 15) / 16 : 0;  // pages with a position of the prompt (the last one zero-padded)
   for (int h = h0; h < h1; ++h) {
     const int64_t plane = static_cast<int64_t>(n) * p.heads + h;
     // rotated q to its plane, rotated k to its plane and the tile; item: (t,
@@ -240,9 +240,8 @@ extern "C" int evo2_rotary_prefill(const void *qkv, int64_t sqkv, const float *i
   if (cdiv(L, 16) > max_pages)
     return fail(EVO2_ERR_INVALID, "rotary_prefill: %lld positions exceed the block table's %lld pages",
                 (long long)L, (long long)max_pages);
-  // the last workgroup's positions cover Lv only if Lv ends in its 64
-  if (Lv > cdiv(L, RP_T) * RP_T || Lv % 8)
-    return fail(EVO2_ERR_INVALID, "rotary_prefill: Lv=%lld must be a multiple of 8 within the last 64 positions",
+  if (Lv > cdiv(L, 128) * 128 || Lv % 8)
+    return fail(EVO2_ERR_INVALID, "rotary_prefill: Lv=%lld must be a multiple of 8 within the last 128 positions",
                 (long long)Lv);
   const uintptr_t align = reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(q) |
                           reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(vt) |
@@ -255,7 +254,7 @@ extern "C" int evo2_rotary_prefill(const void *qkv, int64_t sqkv, const float *i
                static_cast<int>(max_pages), static_cast<int>(L), static_cast<int>(Lv),
                static_cast<int>(heads), RP_HD};
   hipLaunchKernelGGL(rotary_prefill_kernel,
-                     dim3(static_cast<unsigned>(cdiv(L, RP_T)), static_cast<unsigned>(cdiv(heads, RP_HEADS)),
+                     dim3(static_cast<unsigned>(cdiv(Lv, RP_T)), static_cast<unsigned>(cdiv(heads, RP_HEADS)),
                           static_cast<unsigned>(N)),
                      dim3(256), 0, static_cast<hipStream_t>(stream), a);
   return check_launch("rotary_prefill");

@@ -375,7 +375,9 @@ int evo2_prefill_attention(const void *q, const void *k, const void *vt, void *o
 /*
  * evo2_prefill_attention with padded values and any output strides:
  *   vt  (N, heads, head_dim, Lv) bf16, Lv >= L a multiple of 8 with
- *       256 Lv < 2^32, finite from L on;
+ *       256 Lv < 2^32, finite from L on; with Lv off a multiple of 128 an
+ *       infinite or NaN value among a row's first 128 also reaches the row
+ *       before (0 x inf);
  *   out at out + n on + h oh + i ol (elements, multiples of 8), any L.
  */
 int evo2_prefill_attention_rows(const void *q, const void *k, const void *vt, void *out, int64_t on,
@@ -441,7 +443,7 @@ int evo2_bf16_stream_gated(const void *x, int64_t sx, const void *w1, const void
  *               [0, num_pages) are not written through.
  * _prefill: rows n L + t, positions t = 0 .. L-1 of N sequences; also writes
  *   q, k (N, heads, L, head_dim) and vt (N, heads, head_dim, Lv), zeros from L
- *   on (Lv a multiple of 8, at most the next multiple of 64), the operands of
+ *   on (Lv a multiple of 8, at most the next multiple of 128), the operands of
  *   evo2_prefill_attention_rows; the last page's tail is zero.  head_dim 128,
  *   16-byte aligned rows.
  * _decode: one row a sequence at positions[b]; writes q (B, heads, head_dim).

@@ -438,3 +438,31 @@ def test_rotary_prefill_block_table_forms(form):
         rotary_prefill(wide.to(DEV)[:, :3 * nh * hd], caches[-1], t, inv_freq.to(DEV), 1.0, nseq, L)
     assert torch.equal(caches[0].k, caches[1].k) and torch.equal(caches[0].v, caches[1].v)
     assert (caches[0].k[1:].abs().amax((1, 2, 3)) > 0).all()
+
+
+@pytest.mark.parametrize("L", [1, 41, 129, 200])
+def test_prefill_attention_infinite_value_stays_in_its_dim(L):
+    """An infinite value of the first key makes that dim infinite for every
+    query; the dim before it, whose row ends where that key's begins, is as
+    without it.  The values' padding runs over whole key blocks, past the
+    prompt's last 64 positions too."""
+    from evo2_flash_amd.attention import prefill_attention_rows, rotary_prefill
+    hd, nh, nseq = 128, 2, 2
+    g, wide, inv_freq = _qkv_case(nseq * L, nh, hd, L)
+    qkv = wide[:, :3 * nh * hd].contiguous()
+    v = qkv.view(nseq, L, 3, nh, hd)[:, :, 2]
+    v[:, 0, :, 60] = float("inf")
+    npg = -(-L // PAGE)
+    table = (torch.randperm(nseq * npg, generator=g) + 1).int().view(nseq, npg).to(DEV)
+    cache = PagedKVCache(nseq * npg + 1, nh, hd, DEV)
+    out = torch.empty(nseq, nh, L, hd, dtype=bf, device=DEV)
+    print(f"prefill_attention infinite value L={L}", flush=True)
+    q, k, vt = rotary_prefill(qkv.to(DEV), cache, table, inv_freq.to(DEV), 1.0, nseq, L)
+    prefill_attention_rows(q, k, vt, 128 ** -0.5, out)
+    assert (out[..., 60] == float("inf")).all()
+    v[:, 0, :, 60] = 0
+    out[..., 60] = 0
+    ref = _causal_ref(q.cpu(), k.cpu(), v.transpose(1, 2), 128 ** -0.5)
+    ref[..., 60] = 0
+    assert max_rel_err(out.cpu(), ref) <= 1e-2
+    assert vt.shape[3] == -(-L // 128) * 128 and (vt[..., L:] == 0).all()
