@@ -12,38 +12,61 @@ from . import _lib
 STREAM_ROWS = 16  # the kernel's most rows
 
 
-def plain(*tensors):
-    """Whether these are ordinary CUDA bf16 tensors outside every transform (no
-    tracing or dispatch mode, autocast, vmap, gradients of either mode), 16-byte
-    aligned rows."""
+def _eager():
+    """Whether calls run as they are: nothing compiles, exports, traces or
+    dispatches them, no autocast or forward-mode level."""
     if (torch.compiler.is_compiling() or torch.jit.is_tracing()
             or torch._C._len_torch_dispatch_stack() > 0 or torch.is_autocast_enabled("cuda")):
         return False
-    if forward_ad._current_level >= 0:
+    return forward_ad._current_level < 0
+
+
+def _ordinary(t):
+    """Whether t is an ordinary dense CUDA bf16 tensor: no subclass or proxy, outside
+    vmap, without a gradient to record."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
+            and t.layout == torch.strided and t.dtype == torch.bfloat16
+            and not (t.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+
+
+def plain(*tensors):
+    """Whether these are ordinary CUDA bf16 matrices outside every transform (no
+    tracing or dispatch mode, autocast, vmap, gradients of either mode), 16-byte
+    aligned rows."""
+    if not _eager():
         return False
-    grad = torch.is_grad_enabled()
     for t in tensors:
-        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda
-                or t.dtype != torch.bfloat16 or t.dim() != 2 or t.stride(1) != 1
-                or (grad and t.requires_grad)
-                or torch._C._functorch.is_functorch_wrapped_tensor(t)
-                or t.stride(0) % 8 or t.data_ptr() % 16):
+        if not (_ordinary(t) and t.dim() == 2 and t.stride(1) == 1 and t.stride(0) % 8 == 0
+                and t.data_ptr() % 16 == 0):
             return False
     return True
 
 
 def _streams(x, *weights):
     """Whether the weight-streaming kernel takes x (M, K) against weights (N, K)."""
-    if torch.jit.is_tracing():  # (plain's, before a shape is compared in the trace)
-        return False
-    # (x on the current device: a launch goes there, and the default stream's
-    # handle is the same on every device; the library's product switches over)
-    return (x.dim() == 2 and 0 < x.shape[0] <= STREAM_ROWS and x.shape[1] % 32 == 0
+    # `plain` before a shape is compared: to a tracer each comparison is a
+    # condition on the rows.  (x on the current device: a launch goes there, and the
+    # default stream's handle is the same on every device; the library's product
+    # switches over)
+    return (plain(x, *weights) and 0 < x.shape[0] <= STREAM_ROWS and x.shape[1] % 32 == 0
             and x.shape[1] > 0 and all(w.shape == weights[0].shape and w.shape[0] > 0
                                        and w.shape[1] == x.shape[1]
                                        and w.stride() == weights[0].stride()
                                        and w.device == x.device for w in weights)
-            and plain(x, *weights) and x.get_device() == torch.cuda.current_device())
+            and x.get_device() == torch.cuda.current_device())
+
+
+def library_linear(x, weight, bias, out, residual):
+    """`linear` on the library's product."""
+    if out is None:
+        y = torch.nn.functional.linear(x, weight, bias)
+        return y if residual is None else y + residual
+    if residual is not None:  # (which may be `out`: the product goes beside it)
+        return torch.add(torch.nn.functional.linear(x, weight, bias), residual, out=out)
+    if bias is not None:
+        return torch.addmm(bias, x, weight.t(), out=out)
+    return torch.mm(x, weight.t(), out=out)
 
 
 def linear(x, weight, bias=None, out=None, residual=None):
@@ -54,35 +77,26 @@ def linear(x, weight, bias=None, out=None, residual=None):
     (N K <= 2^24, K <= 4096): there it is the faster one, measured in us against
     the library at 8 / 16 rows: 4096 x 4096 9.6 / 11.5 against 15.6; 11264 x 4096
     24.7 / 29.7 against 26.4; 1920 x 5120 11.0 / 14.3 against 18.3 / 10.5."""
-    M, (N, K) = x.shape[0], weight.shape
-    if (_streams(x, weight) and (M <= 8 or (N * K <= 1 << 24 and K <= 4096))
-            and (bias is None or (bias.device == x.device and bias.dtype == x.dtype
-                                  and bias.shape == (N,)
-                                  and bias.is_contiguous()
-                                  and not (torch.is_grad_enabled() and bias.requires_grad)))
-            and (residual is None or (residual.shape == (M, N) and residual.device == x.device
-                                      and plain(residual)))
-            and (out is None or (out.shape == (M, N) and out.dtype == x.dtype
-                                 and out.stride(1) == 1 and out.device == x.device
-                                 # (the kernel stores while others still read)
-                                 and not _lib.overlap(x, out)
-                                 and (residual is None or not _lib.overlap(residual, out))))):
-        y = torch.empty(M, N, dtype=x.dtype, device=x.device) if out is None else out
-        _lib.call("evo2_bf16_stream_linear", _lib.ptr(x), x.stride(0), _lib.ptr(weight),
-                  weight.stride(0), _lib.ptr(bias), _lib.ptr(residual),
-                  0 if residual is None else residual.stride(0), _lib.ptr(y), y.stride(0),
-                  M, N, K, _lib.stream_of(x))
-        return y
-    if out is None:
-        y = torch.nn.functional.linear(x, weight, bias)
-        return y if residual is None else y + residual
-    if residual is not None:  # (which may be `out`: the product goes beside it)
-        return torch.add(torch.nn.functional.linear(x, weight, bias), residual, out=out)
-    if bias is not None:
-        torch.addmm(bias, x, weight.t(), out=out)
-    else:
-        torch.mm(x, weight.t(), out=out)
-    return out
+    if _streams(x, weight):
+        M, (N, K) = x.shape[0], weight.shape
+        if ((M <= 8 or (N * K <= 1 << 24 and K <= 4096))
+                and (bias is None or (bias.device == x.device and bias.dtype == x.dtype
+                                      and bias.shape == (N,) and bias.is_contiguous()
+                                      and not (torch.is_grad_enabled() and bias.requires_grad)))
+                and (residual is None or (plain(residual) and residual.shape == (M, N)
+                                          and residual.device == x.device))
+                and (out is None or (out.shape == (M, N) and out.dtype == x.dtype and out.stride(1) == 1
+                                     and out.device == x.device
+                                     # (the kernel stores while others still read)
+                                     and not _lib.overlap(x, out)
+                                     and (residual is None or not _lib.overlap(residual, out))))):
+            y = torch.empty(M, N, dtype=x.dtype, device=x.device) if out is None else out
+            _lib.call("evo2_bf16_stream_linear", _lib.ptr(x), x.stride(0), _lib.ptr(weight),
+                      weight.stride(0), _lib.ptr(bias), _lib.ptr(residual),
+                      0 if residual is None else residual.stride(0), _lib.ptr(y), y.stride(0),
+                      M, N, K, _lib.stream_of(x))
+            return y
+    return library_linear(x, weight, bias, out, residual)
 
 
 def gated(x, w1, w2, gelu):

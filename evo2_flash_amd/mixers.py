@@ -87,10 +87,9 @@ class Linear(nn.Module):
         self.bias = (nn.Parameter(torch.zeros(out_features, device=device, dtype=dtype),
                                   requires_grad=False) if bias else None)
 
-    def forward(self, x, out=None, residual=None):
-        """x (..., in) -> ((..., out), None), plus `residual` when given; a 2-D x
-        may write its result into `out`."""
-        return linear(x, self.weight, self.bias, out, residual), None
+    def forward(self, x, out=None):
+        """x (..., in) -> ((..., out), None); a 2-D x may write its result into `out`."""
+        return linear(x, self.weight, self.bias, out), None
 
 
 class ProjectionTap(nn.Module):

@@ -60,20 +60,25 @@ class Evo2MLP(nn.Module):
         self.l3 = Linear(inter, hidden, device=device)
         self.use_act = use_act
 
-    def forward(self, x, residual=None):
-        """The MLP's output, plus `residual` (the layer's input) when given.
-        Projections of another type, with a bias or with hooks are called as
-        modules, and l3's hooks see its output without the residual."""
-        if all(_bare(m, Linear) and m.bias is None for m in (self.l1, self.l2)):
-            z = gated(x, self.l1.weight, self.l2.weight, self.use_act)
-        else:
-            z1, _ = self.l1(x)
-            z2, _ = self.l2(x)
-            z = (nn.functional.gelu(z1) if self.use_act else z1) * z2
-        if residual is not None and _bare(self.l3, Linear):
-            return self.l3(z, residual=residual)[0]
-        out, _ = self.l3(z)
-        return out if residual is None else out + residual
+    def _product(self, x):
+        """act(l1 x) * l2 x; projections of another type, with a bias or with
+        hooks, and all of them where something traces, are called as modules."""
+        if plain(x) and all(_bare(m, Linear) and m.bias is None for m in (self.l1, self.l2)):
+            return gated(x, self.l1.weight, self.l2.weight, self.use_act)
+        z1, _ = self.l1(x)
+        z2, _ = self.l2(x)
+        return (nn.functional.gelu(z1) if self.use_act else z1) * z2
+
+    def forward(self, x):
+        out, _ = self.l3(self._product(x))
+        return out
+
+    def plus(self, x, residual):
+        """forward(x) + residual; the sum is left to l3's launch where calling l3
+        is no more than its product (hooks on l3 see the product alone)."""
+        if not _bare(self.l3, Linear):
+            return self.forward(x) + residual
+        return linear(self._product(x), self.l3.weight, self.l3.bias, residual=residual)
 
 
 def rotary_neox(x, positions, inv_freq, factor):
@@ -165,7 +170,9 @@ class Evo2DecoderLayer(nn.Module):
     def _mlp(self, post, x):
         """The MLP's output plus x (an MLP of another type or with hooks gives
         its own output)."""
-        return self.mlp(post, residual=x) if _bare(self.mlp, Evo2MLP) else self.mlp(post) + x
+        if _bare(self.mlp, Evo2MLP) and plain(post):
+            return self.mlp.plus(post, x)
+        return self.mlp(post) + x
 
     def forward(self, positions, x, token_ids, block_table):
         """One decode token per sequence."""

@@ -365,3 +365,46 @@ def test_rotary_takes_rows_of_any_stride(which, native):
     assert torch.equal(seen, qkv) and stride == qkv.shape[1]
     with pytest.raises(ValueError):
         _rotate(which, qkv, cache, table[:0], inv_freq)
+
+
+def _mlp_or_linear(what):
+    from evo2_flash_amd.mixers import Linear
+    return Linear(8, 12) if what == "linear" else _layer().mlp
+
+
+@pytest.mark.parametrize("what", ["linear", "mlp"])
+def test_projections_trace_symbolically(what):
+    """torch.fx and torch.export with any number of rows: no condition on the rows
+    in front of the library's product, no argument beyond the module's own, and
+    l1 .. l3 can be a tracer's leaves."""
+    from torch import fx
+    from evo2_flash_amd.mixers import Linear
+    mod = _mlp_or_linear(what)
+    with torch.no_grad():
+        for p in mod.parameters():
+            p.copy_(torch.randn(p.shape))
+    x, y = torch.randn(3, 8).to(bf), torch.randn(40, 8).to(bf)
+    want = mod(y)
+    args = {"out": None} if what == "linear" else None
+    traced = fx.symbolic_trace(mod, concrete_args=args)
+    rows = torch.export.Dim("rows", min=2, max=4096)
+    program = torch.export.export(mod, (x,), dynamic_shapes={"x": {0: rows}}).module()
+    for form in (traced, program):
+        got = form(y)
+        assert torch.equal(*((got[0], want[0]) if what == "linear" else (got, want)))
+    if what == "mlp":
+        class Leaves(fx.Tracer):
+            def is_leaf_module(self, m, name):
+                return isinstance(m, Linear)
+        nodes = Leaves().trace(mod).nodes
+        assert [n.target for n in nodes if n.op == "call_module"] == ["l1", "l2", "l3"]
+
+
+def test_linear_of_a_sparse_weight():
+    """Sparse weights reach torch's own product."""
+    from evo2_flash_amd.mixers import Linear
+    mod = Linear(32, 12, dtype=torch.float32)
+    w, x = torch.randn(12, 32), torch.randn(3, 32)
+    for sparse in (w.to_sparse_csr(), w.to_sparse()):
+        mod.weight = torch.nn.Parameter(sparse, requires_grad=False)
+        torch.testing.assert_close(mod(x)[0], x @ w.t())
