@@ -4,6 +4,8 @@
 otherwise.
 """
 
+from typing import Optional
+
 import torch
 from torch.autograd import forward_ad
 
@@ -57,8 +59,9 @@ def _streams(x, *weights):
             and x.get_device() == torch.cuda.current_device())
 
 
-def library_linear(x, weight, bias, out, residual):
-    """`linear` on the library's product."""
+def library_linear(x, weight, bias: Optional[torch.Tensor], out: Optional[torch.Tensor],
+                   residual: Optional[torch.Tensor]):
+    """`linear` on the library's product (also what TorchScript compiles)."""
     if out is None:
         y = torch.nn.functional.linear(x, weight, bias)
         return y if residual is None else y + residual

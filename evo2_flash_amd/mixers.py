@@ -52,7 +52,7 @@ from .decode import channel_major_taps, hyena_decode
 from .fp8 import Fp8StaticLinear
 from .fp8_emul import static_fp8_linear_emulated
 from .hcl import hcl_block_t, hyena_hcl_prefill
-from .linear import linear
+from .linear import library_linear, linear
 from .metadata import decode_state_indices, longest_prefill_segment, prefill_tables
 from .prefill import fir_prefill_block_t, hyena_fir_prefill
 from .short_conv import PAD_SLOT_ID, _update_spec as conv_update_spec
@@ -87,9 +87,13 @@ class Linear(nn.Module):
         self.bias = (nn.Parameter(torch.zeros(out_features, device=device, dtype=dtype),
                                   requires_grad=False) if bias else None)
 
-    def forward(self, x, out=None):
+    def forward(self, x, out: Optional[torch.Tensor] = None):
         """x (..., in) -> ((..., out), None); a 2-D x may write its result into `out`."""
-        return linear(x, self.weight, self.bias, out), None
+        if torch.jit.is_scripting():  # (TorchScript compiles this branch alone)
+            y = library_linear(x, self.weight, self.bias, out, None)
+        else:
+            y = linear(x, self.weight, self.bias, out)
+        return y, None
 
 
 class ProjectionTap(nn.Module):

@@ -408,3 +408,16 @@ def test_linear_of_a_sparse_weight():
     for sparse in (w.to_sparse_csr(), w.to_sparse()):
         mod.weight = torch.nn.Parameter(sparse, requires_grad=False)
         torch.testing.assert_close(mod(x)[0], x @ w.t())
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_linear_compiles_to_torchscript(bias):
+    from evo2_flash_amd.mixers import Linear
+    mod = Linear(8, 12, bias=bias)
+    with torch.no_grad():
+        for p in mod.parameters():
+            p.copy_(torch.randn(p.shape))
+    x, out = torch.randn(3, 8).to(bf), torch.empty(3, 12, dtype=bf)
+    script = torch.jit.script(mod)
+    assert script(x, out)[0].data_ptr() == out.data_ptr()
+    assert torch.equal(out, mod(x)[0]) and torch.equal(script(x)[0], out)
