@@ -8,6 +8,7 @@ from typing import Optional
 
 import torch
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -16,9 +17,13 @@ STREAM_ROWS = 16  # the kernel's most rows
 
 def _eager():
     """Whether calls run as they are: nothing compiles, exports, traces or
-    dispatches them, no autocast or forward-mode level."""
+    intercepts them (a default device apart), no autocast or forward-mode level."""
     if (torch.compiler.is_compiling() or torch.jit.is_tracing()
             or torch._C._len_torch_dispatch_stack() > 0 or torch.is_autocast_enabled("cuda")):
+        return False
+    if torch._C._len_torch_function_stack() > 0 and any(
+            type(m) is not DeviceContext
+            for m in torch.overrides._get_current_function_mode_stack()):
         return False
     return forward_ad._current_level < 0
 

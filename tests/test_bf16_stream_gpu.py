@@ -135,3 +135,26 @@ def test_outputs_over_inputs(monkeypatch):
     assert calls == []
     linear(x, w, residual=r[:8], out=torch.empty_like(want))
     assert calls == ["evo2_bf16_stream_linear"]
+
+
+def test_function_modes_see_the_product():
+    """A function mode is called for the library's product; a default device,
+    which is one too, leaves the kernel in place."""
+    x, w = _rand(4, 64, seed=21), _rand(64, 64, seed=22)
+    seen = []
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        y = linear(x, w)
+        gated(x, w, w, False)
+    assert seen.count("linear") == 3
+    assert torch.equal(y, torch.nn.functional.linear(x, w))
+    with torch.device(DEV), pytest.MonkeyPatch.context() as mp:
+        calls, call = [], _lib.call
+        mp.setattr(_lib, "call", lambda n, *a: (calls.append(n), call(n, *a)))
+        linear(x, w)
+        assert calls == ["evo2_bf16_stream_linear"]
