@@ -88,12 +88,11 @@ def linear(x, weight, bias=None, out=None, residual=None):
     if _streams(x, weight):
         M, (N, K) = x.shape[0], weight.shape
         if ((M <= 8 or (N * K <= 1 << 24 and K <= 4096))
-                and (bias is None or (bias.device == x.device and bias.dtype == x.dtype
-                                      and bias.shape == (N,) and bias.is_contiguous()
-                                      and not (torch.is_grad_enabled() and bias.requires_grad)))
+                and (bias is None or (_ordinary(bias) and bias.device == x.device
+                                      and bias.shape == (N,) and bias.is_contiguous()))
                 and (residual is None or (plain(residual) and residual.shape == (M, N)
                                           and residual.device == x.device))
-                and (out is None or (out.shape == (M, N) and out.dtype == x.dtype and out.stride(1) == 1
+                and (out is None or (_ordinary(out) and out.shape == (M, N) and out.stride(1) == 1
                                      and out.device == x.device
                                      # (the kernel stores while others still read)
                                      and not _lib.overlap(x, out)

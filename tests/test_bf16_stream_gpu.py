@@ -158,3 +158,15 @@ def test_function_modes_see_the_product():
         mp.setattr(_lib, "call", lambda n, *a: (calls.append(n), call(n, *a)))
         linear(x, w)
         assert calls == ["evo2_bf16_stream_linear"]
+
+
+def test_vmapped_bias():
+    """A batch of biases or residuals over a plain product: torch's own."""
+    x, w, b = _rand(4, 64, seed=23), _rand(64, 64, seed=24), _rand(3, 64, seed=25)
+    F = torch.nn.functional.linear
+    # (vmap's own form of F.linear rounds the product before it adds the bias)
+    want = torch.vmap(lambda t: F(x, w, t))(b)
+    assert torch.equal(torch.vmap(lambda t: linear(x, w, t))(b), want)
+    r = torch.stack([_rand(4, 64, seed=s) for s in (26, 27)])
+    got = torch.vmap(lambda t: linear(x, w, residual=t))(r)
+    assert torch.equal(got, F(x, w) + r)
