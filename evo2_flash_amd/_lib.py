@@ -213,6 +213,10 @@ SIGNATURES = {
         _c_p, _c_p, _c_p,                         # x_scale, w_scale, bias
         _c_p, _c_i64, _c_i64, _c_p,               # out, N, K, stream
     ],
+    "evo2_fp8_gemm_plan": [
+        _c_i64, _c_i64, _c_i64, _c_i32,           # sx, sw, so, aligned
+        _c_i64, _c_i64, _c_i64, ctypes.c_int,     # M, N, K, ncu
+    ],
     "evo2_fp8_gemm_persist_order": [_c_i64, _c_i64, ctypes.c_int, _c_p, _c_p],
     "evo2_fp8_fast_accum_gemm": [
         _c_p, _c_i64, _c_p, _c_i64,               # a8, sa, b_t, sb

@@ -1114,6 +1114,30 @@ static int persist_rows(int64_t tiles_n, int64_t M, int ncu) {
   return best;
 }
 
+// The kernel for these operands: -1 the weight-streaming one, 1 .. 4 the
+// persistent one with tiles of so many times 64 X rows, 0 the general one.
+// The persistent kernel takes whole 128-byte slices of K, columns in eights,
+// 16-byte aligned output rows, and operands -- rounded up to whole tiles of the
+// chosen height, as its row offsets run -- and a tile's output within 32-bit
+// buffer offsets.
+static int gemm_plan(int64_t sx, int64_t sw, int64_t so, bool aligned, int64_t M, int64_t N, int64_t K,
+                     int ncu) {
+  const int64_t tiles_n = cdiv(N, G_BN), tiles_m = cdiv(M, G_BM);
+  int tm = 0;
+  if (ncu > 0 && K % Q_BK == 0 && N % 8 == 0 && so % 8 == 0 && aligned && so < (1 << 20) && sx >= K &&
+      sw >= K && so >= N && tiles_n * tiles_m < (1 << 24)) {
+    tm = persist_rows(tiles_n, M, ncu);
+    const int64_t bm = 64 * tm;
+    if (tiles_n * G_BN * sw + K >= (int64_t(1) << 31) || cdiv(M, bm) * bm * sx + K >= (int64_t(1) << 31))
+      tm = 0;
+  }
+  const int64_t work = cdiv(M, S_ROWS) * N;
+  if (K % S_BK == 0 && sx * S_ROWS < (int64_t(1) << 31) &&
+      (M <= S_ROWS || work <= (tm ? TILE_MIN_WORK : STREAM_MAX_WORK)))
+    return -1;
+  return tm;
+}
+
 template <bool PACKED>
 static void launch_stream(const GemmArgs &a, hipStream_t st) {
   if (a.N <= (1 << 26) && (a.M <= 8 || (a.M <= F_ROWS && (int64_t)a.N * a.K <= (1 << 26)))) {
@@ -1192,32 +1216,23 @@ extern "C" int evo2_fp8_gemm(const void *x8, int64_t sx, const void *w8, int64_t
              w_scale, static_cast<const bf16_t *>(bias), static_cast<bf16_t *>(out), so,
              static_cast<int>(M), static_cast<int>(N), static_cast<int>(K)};
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t tiles_n = cdiv(N, G_BN), tiles_m = cdiv(M, G_BM);
   const int ncu = cu_count();
-  // the persistent kernel: whole 128-byte slices of K, columns in eights,
-  // 16-byte aligned output rows, operands (rounded up to whole tiles) and a
-  // tile's output within 32-bit buffer offsets
-  const bool tiles = ncu > 0 && K % Q_BK == 0 && N % 8 == 0 && so % 8 == 0 &&
-                     reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-                     (!bias || reinterpret_cast<uintptr_t>(bias) % 8 == 0) && so < (1 << 20) &&
-                     sx >= K && sw >= K && so >= N && tiles_n * tiles_m < (1 << 24) &&
-                     (tiles_n * G_BN) * sw + K < (int64_t(1) << 31) &&
-                     (tiles_m * G_BM) * sx + K < (int64_t(1) << 31);
-  const int64_t work = cdiv(M, S_ROWS) * N;
-  if (K % S_BK == 0 && sx * S_ROWS < (int64_t(1) << 31) &&
-      (M <= S_ROWS || work <= (tiles ? TILE_MIN_WORK : STREAM_MAX_WORK))) {
+  const bool aligned = reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
+                       (!bias || reinterpret_cast<uintptr_t>(bias) % 8 == 0);
+  const int plan = gemm_plan(sx, sw, so, aligned, M, N, K, ncu);
+  if (plan < 0) {
     // the weight-streaming kernel over ceil(M / 64) blocks of 64 rows
     launch_stream<false>(a, st);
     return check_launch("fp8_gemm");
   }
-  if (tiles) {
-    const int tm = persist_rows(tiles_n, M, ncu);
-    if (tm == 4) launch_persist<4>(a, ncu, st);
-    else if (tm == 3) launch_persist<3>(a, ncu, st);
-    else if (tm == 2) launch_persist<2>(a, ncu, st);
+  if (plan > 0) {
+    if (plan == 4) launch_persist<4>(a, ncu, st);
+    else if (plan == 3) launch_persist<3>(a, ncu, st);
+    else if (plan == 2) launch_persist<2>(a, ncu, st);
     else launch_persist<1>(a, ncu, st);
     return check_launch("fp8_gemm");
   }
+  const int64_t tiles_n = cdiv(N, G_BN), tiles_m = cdiv(M, G_BM);
   dim3 grid(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m));
   hipLaunchKernelGGL(fp8_gemm_kernel, grid, dim3(256), 0, st, a);
   return check_launch("fp8_gemm");
@@ -1289,6 +1304,12 @@ extern "C" int evo2_fp8_quant_gemv(const void *x, const void *w, int64_t sw, int
   if (packed) hipLaunchKernelGGL((fp8_few_kernel<true, true>), grid, dim3(64 * F_WAVES), lds, st, a);
   else hipLaunchKernelGGL((fp8_few_kernel<false, true>), grid, dim3(64 * F_WAVES), lds, st, a);
   return check_launch("fp8_quant_gemv");
+}
+
+extern "C" int evo2_fp8_gemm_plan(int64_t sx, int64_t sw, int64_t so, int32_t aligned, int64_t M, int64_t N,
+                                  int64_t K, int ncu) {
+  if (M <= 0 || N <= 0 || K <= 0 || ncu < 0 || M > 0x7fffffff || N > 0x7fffffff) return -2;
+  return gemm_plan(sx, sw, so, aligned != 0, M, N, K, ncu);
 }
 
 extern "C" int64_t evo2_fp8_gemm_persist_order(int64_t tiles_n, int64_t tiles_m, int ncu, int32_t *bn,

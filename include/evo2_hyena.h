@@ -536,6 +536,16 @@ int evo2_fp8_quant_gemv(const void *x, const void *w, int64_t sw, int32_t packed
                         void *stream);
 
 /*
+ * The kernel evo2_fp8_gemm takes for operands of these sizes and strides on a
+ * device of ncu compute units (`aligned`: the output 16-byte aligned, a bias
+ * 8-byte): -1 the weight-streaming kernel, 0 the general tile kernel, 1 to 4
+ * the persistent kernel with tiles of 64 to 256 X rows, -2 for bad sizes.  Host
+ * only, no GPU needed; no counterpart in the reference.
+ */
+int evo2_fp8_gemm_plan(int64_t sx, int64_t sw, int64_t so, int32_t aligned, int64_t M, int64_t N,
+                       int64_t K, int ncu);
+
+/*
  * The order in which evo2_fp8_gemm's persistent kernel (one workgroup per
  * compute unit; 256 W rows x 64 to 256 X rows a tile) walks a grid of tiles_n x
  * tiles_m tiles with ncu workgroups: tile t, run by workgroup

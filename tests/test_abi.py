@@ -200,3 +200,26 @@ def test_fp8_persist_order_covers_every_tile():
                         assert len(np.unique(bm[:whole][sel] // 8)) == 1
     assert lib.evo2_fp8_gemm_persist_order(48, 8, 256, None, None) == 1
     assert lib.evo2_fp8_gemm_persist_order(0, 8, 256, None, None) == -1
+
+
+@needs_lib
+def test_fp8_tiles_stay_within_buffer_offsets():
+    """The persistent GEMM's row offsets are 32-bit and run to the end of the
+    last tile of the height it takes: 1000 rows are 1152 in tiles of 192.  Strides
+    past that go to the general kernel."""
+    import random
+    plan = _lib.lib().evo2_fp8_gemm_plan
+    fits = ((1 << 31) - 128) // 1152 // 16 * 16
+    assert plan(128, 128, 10240, 1, 1000, 10240, 128, 256) == 3
+    assert plan(fits - 16, 128, 10240, 1, 1000, 10240, 128, 256) == 3
+    assert plan(fits + 16, 128, 10240, 1, 1000, 10240, 128, 256) == 0
+    assert plan(2000000, 128, 10240, 1, 1000, 10240, 128, 256) == 0
+    assert plan(0, 0, 0, 1, 0, 64, 128, 256) == -2
+    rng = random.Random(1)
+    for _ in range(20000):
+        M, N, K = rng.randint(1, 9000), 8 * rng.randint(1, 3000), 128 * rng.randint(1, 64)
+        sx = max(K, int(2 ** rng.uniform(20, 31) / M) // 16 * 16)
+        tm = plan(sx, K, N, 1, M, N, K, 256)
+        if tm > 0:
+            bm = 64 * tm
+            assert -(-M // bm) * bm * sx + K < 1 << 31, (M, N, K, sx)

@@ -369,3 +369,16 @@ def test_static_linear_in_place(rows):
     ref = static_fp8_linear(x, w, xs, ws)
     assert static_fp8_linear(x, w, xs, ws, out=x).data_ptr() == x.data_ptr()
     assert torch.equal(x.view(torch.int16), ref.view(torch.int16))
+
+
+def test_gemm_rows_far_apart():
+    """1000 rows at a stride where whole tiles of 192 rows pass 2^31 bytes: the
+    product of the same rows side by side."""
+    M, N, K, sx = 1000, 10240, 128, 2000000
+    g = torch.Generator().manual_seed(1)
+    x8, w8 = _small_int_e4m3((M, K), g).to(DEV), _small_int_e4m3((N, K), g).to(DEV)
+    one = torch.ones(1, device=DEV)
+    print(f"rows far apart M={M} N={N} K={K} stride={sx}", flush=True)
+    wide = torch.empty((M - 1) * sx + K, dtype=torch.uint8, device=DEV).as_strided((M, K), (sx, 1))
+    wide.copy_(x8.view(torch.uint8))
+    assert torch.equal(fp8_gemm(wide.view(E4M3), w8, one, one), fp8_gemm(x8, w8, one, one))
