@@ -55,19 +55,20 @@ def _small_int_e4m3(shape, g):
     return (torch.randint(-6, 7, shape, generator=g).float()).to(E4M3)
 
 
-# With K a multiple of 128 the weight-streaming kernel takes M <= 64, and
-# larger M over blocks of 64 rows while ceil(M / 64) x N <= 60000 (16 W rows
-# per wave in registers, 16x16x128 MFMA, the blocks of one weight slice on
-# one XCD); the others run the 256x256-tile kernel (K = 192 here, or too much
-# work).
+# The dispatch, as evo2_fp8_gemm_plan has it for this device.  With K a multiple
+# of 128 the weight-streaming kernels take M <= 64 (fp8_few_kernel up to 8 or 16
+# rows), and larger M over blocks of 64 rows while ceil(M / 64) x N is at most
+# 50000 (60000 where the persistent tiles do not apply); above, the persistent
+# kernel, and the general tile kernel for what that does not take (K = 192 here).
 @pytest.mark.parametrize("M,N,K", [(64, 384, 256), (1, 64, 128), (5, 130, 1920),
                                    (64, 4096, 4096),                      # one row block
                                    (65, 200, 256), (130, 96, 384), (300, 512, 1920),
                                    (1000, 130, 640), (128, 12288, 256), (100, 10000, 384),
                                    (192, 12288, 256), (170, 12000, 256),
                                    (256, 12288, 512),                     # gridded over M
-                                   (256, 256, 192), (1100, 6400, 640),
-                                   (500, 12288, 256)])                    # 256x256 tiles
+                                   (256, 256, 192),                       # general, one tile
+                                   (1100, 6400, 640),
+                                   (500, 12288, 256)])                    # persistent, 128 rows a tile
 def test_gemm_known_answer(M, N, K):
     g = torch.Generator().manual_seed(M + N)
     x8 = _small_int_e4m3((M, K), g)
@@ -79,13 +80,10 @@ def test_gemm_known_answer(M, N, K):
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
 
 
-# Persistent 256x256 form: (2048, 8192) has 8 x 32 tiles (the XCD-block
-# order); (2048, 12288) has 8 x 48 = 384 tiles, twelve blocks of 4 x 8, so
-# the XCD-block order's second round is half full and its last four blocks
-# go out tile by tile; (3328, 5120) has 13 x 20 = 260 tiles over 256
-# workgroups (row-major order, four workgroups take a second tile);
-# (2048, 12288, 256) has tiles of one slice pair, the one that starts the
-# accumulators.
+# Persistent kernel on whole tiles: (2048, 8192) is one round of 32 x 8 tiles of
+# 256 rows (the XCD-block order); (2048, 12288) 48 x 16 tiles of 128 rows, three
+# whole rounds of 4 x 8 blocks on the three-stage ring, with K = 256 of two slices
+# a tile; (3328, 5120) 20 x 18 tiles of 192 rows, two rounds in panel order.
 @pytest.mark.parametrize("M,N,K", [(2048, 8192, 512), (2048, 12288, 512), (3328, 5120, 768),
                                    (2048, 12288, 256)])
 def test_gemm_known_answer_persistent(M, N, K):
@@ -105,10 +103,10 @@ def test_gemm_known_answer_persistent(M, N, K):
                                    (2047, 5760, 256), (3001, 8192, 128), (6001, 5000, 256)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_gemm_known_answer_ragged_tiles(M, N, K, bias):
-    """The persistent kernel off whole tiles, each of its four tile heights
-    (one and several rounds over the CUs, the last part-filled): rows and
-    columns past the output (columns in eights) and odd counts of 128-byte
-    slices.  Small-integer operands, exact sums: bit for bit, and nothing
+    """The persistent kernel off whole tiles, each of its four tile heights in one
+    round over the CUs, 192 and 256 rows in two as well (the last part-filled):
+    rows and columns past the output (columns in eights) and odd counts of
+    128-byte slices.  Small-integer operands, exact sums: bit for bit, and nothing
     written beside the output."""
     g = torch.Generator().manual_seed(M + K)
     x8 = _small_int_e4m3((M, K), g).to(DEV)
@@ -123,6 +121,83 @@ def test_gemm_known_answer_ragged_tiles(M, N, K, bias):
         ref += b.float()
     assert torch.equal(wide[:M, :N], ref.to(torch.bfloat16))
     assert (wide[M] == 99).all() and (wide[:, N:] == 99).all()
+
+
+def _plan(M, N, K, so=None, aligned=True):
+    """(kernel of evo2_fp8_gemm: -1 streaming, 0 general, 64-row units of a
+    persistent tile; that kernel's rounds over the CUs)."""
+    from evo2_flash_amd import _lib
+    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+    tm = _lib.lib().evo2_fp8_gemm_plan(K, K, so or N, int(aligned), M, N, K, ncu)
+    tiles = -(-N // 256) * -(-M // (64 * max(tm, 1)))
+    return tm, -(-tiles // ncu)
+
+
+def _exact_case(M, N, K, bias):
+    """Small-integer operands and their exact product (|sums| < 2^24) in bf16."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x8 = _small_int_e4m3((M, K), g).to(DEV)
+    w8 = _small_int_e4m3((N, K), g).to(DEV)
+    b = torch.randint(-8, 9, (N,), generator=g).to(torch.bfloat16).to(DEV) if bias else None
+    ref = x8.float() @ w8.float().t()
+    return x8, w8, b, (ref + b.float() if bias else ref).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 515, 832), (600, 1000, 704),  # K off 128: 13 and 11 steps
+                                   (700, 6001, 1408),                  # N off 8: 22 steps
+                                   (600, 8192, 640)])                  # output rows off 16 bytes
+@pytest.mark.parametrize("bias", [False, True])
+def test_gemm_known_answer_general(M, N, K, bias):
+    """The general tile kernel: several tiles, the last of each direction partial,
+    its unguarded ten-step loop and every kind of remainder after it."""
+    x8, w8, b, ref = _exact_case(M, N, K, bias)
+    wide = torch.full((M + 1, N + 8), 99.0, dtype=torch.bfloat16, device=DEV)
+    out = wide[:M, 1:N + 1]
+    one = torch.ones(1, device=DEV)
+    assert _plan(M, N, K, so=N + 8, aligned=False)[0] == 0
+    print(f"general tiles M={M} N={N} K={K} bias={bias}", flush=True)
+    fp8_gemm(x8, w8, one, one, b, out=out)
+    assert torch.equal(out, ref)
+    assert (wide[M] == 99).all() and (wide[:, 0] == 99).all() and (wide[:, N + 1:] == 99).all()
+    if K % 128 or N % 8:  # contiguous rows as well
+        assert _plan(M, N, K)[0] == 0
+        assert torch.equal(fp8_gemm(x8, w8, one, one, b), ref)
+
+
+@pytest.mark.parametrize("M,N,K,plan", [(1999, 12280, 384, (2, 3)), (6407, 2552, 640, (2, 2)),
+                                        (6140, 5120, 256, (4, 2)), (6140, 5120, 384, (4, 2)),
+                                        (3001, 12280, 384, (3, 3))])
+@pytest.mark.parametrize("bias", [False, True])
+def test_gemm_known_answer_tile_rounds(M, N, K, plan, bias):
+    """From one tile to the next in both slice rings, with odd and even counts of
+    slices, the last round part-filled and whole rows and columns past the output;
+    (6140, 5120) has 15 blocks of 4 x 8 tiles, the XCD-block order's part-filled
+    round.  (Tiles of 64 rows never take a second round of 256 CUs.)"""
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert _plan(M, N, K) == plan
+    x8, w8, b, ref = _exact_case(M, N, K, bias)
+    wide = torch.full((M + 1, N + 8), 99.0, dtype=torch.bfloat16, device=DEV)
+    one = torch.ones(1, device=DEV)
+    print(f"tile rounds M={M} N={N} K={K} bias={bias}", flush=True)
+    fp8_gemm(x8, w8, one, one, b, out=wide[:M, :N])
+    assert torch.equal(wide[:M, :N], ref)
+    assert (wide[M] == 99).all() and (wide[:, N:] == 99).all()
+
+
+@pytest.mark.parametrize("M", [2, 8, 9, 16, 17])
+@pytest.mark.parametrize("N,K", [(16, 128), (130, 1920), (96, 1152), (8208, 8320)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_gemm_known_answer_few_rows(M, N, K, bias):
+    """fp8_few_kernel (up to 8 rows, 16 where N K <= 2^26) and the ring kernel from
+    the next row on, row-major (N off 16 too) and packed: exact sums, whose bits
+    do not depend on how K is split."""
+    from evo2_flash_amd.fp8 import fp8_gemm_packed, fp8_pack_weight, packable
+    x8, w8, b, ref = _exact_case(M, N, K, bias)
+    one = torch.ones(1, device=DEV)
+    print(f"few rows M={M} N={N} K={K} bias={bias}", flush=True)
+    assert torch.equal(fp8_gemm(x8, w8, one, one, b), ref)
+    if packable(N, K):
+        assert torch.equal(fp8_gemm_packed(x8, fp8_pack_weight(w8), one, one, b), ref)
 
 
 @pytest.mark.parametrize("M,N,K", [(8100, 8192, 128), (8100, 8192, 256),       # 256 rows a tile, 4 rounds
