@@ -69,9 +69,15 @@ TILE_MIN_WORK = 50000    # and above this prefers its persistent tile kernel (M 
 def streams_weight(M, N):
     """Whether evo2_fp8_gemm may take its weight-streaming kernel for M rows
     (always at M <= 64; over 64-row blocks while ceil(M / 64) * N is at most
-    STREAM_MAX_WORK): the shapes a packed weight copy is kept for.  Above
-    TILE_MIN_WORK the persistent tile kernel is the faster one."""
+    STREAM_MAX_WORK, which it does above TILE_MIN_WORK only where its persistent
+    tile kernel does not take the operands)."""
     return 0 < M and (M <= 64 or -(-M // 64) * N <= STREAM_MAX_WORK)
+
+
+def reads_packed(M, N):
+    """Whether static_fp8_linear reads a packed weight copy for M rows: streamed
+    shapes below TILE_MIN_WORK."""
+    return 0 < M and (M <= 64 or -(-M // 64) * N <= TILE_MIN_WORK)
 
 
 def packable(N, K):
@@ -165,8 +171,7 @@ def static_fp8_linear(x, weight, input_scale, weight_scale, bias=None, out=None,
     gemm = fp8_gemm
     w = weight
     M, N = x8.shape[0], weight.shape[0]
-    if packed is not None and streams_weight(M, N) and (
-            M <= 64 or -(-M // 64) * N <= TILE_MIN_WORK):
+    if packed is not None and reads_packed(M, N):
         gemm, w = fp8_gemm_packed, packed
     if out is not None:
         if x.dim() != 2 or out.shape != (x.shape[0], weight.shape[0]) or out.stride(1) != 1:
@@ -261,6 +266,6 @@ class Fp8StaticLinear(nn.Module):
 
     def forward(self, x, out=None):
         rows = x.numel() // max(x.shape[-1], 1)
-        packed = self.decode_weight() if streams_weight(rows, self.out_features) else None
+        packed = self.decode_weight() if reads_packed(rows, self.out_features) else None
         return static_fp8_linear(x, self.weight, self.input_scale, self.weight_scale,
                                  self.bias, out=out, packed=packed), None

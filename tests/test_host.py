@@ -213,10 +213,9 @@ def test_conv_reload_refreshes_decode_taps():
 
 
 def test_packed_weight_rules():
-    """Where the fp8 linear reads its packed decode copy: the shapes where
-    evo2_fp8_gemm streams the weight (M <= 64, or ceil(M / 64) * N <= 60000,
-    the constant the C dispatcher uses), for weights with a decode layout
-    (N a multiple of 16, K of 128)."""
+    """The shapes where evo2_fp8_gemm may stream the weight (M <= 64, or
+    ceil(M / 64) * N <= 60000, the constant the C dispatcher uses), and the
+    weights with a decode layout (N a multiple of 16, K of 128)."""
     import re
     from evo2_flash_amd.fp8 import STREAM_MAX_WORK, packable, streams_weight
     src = open(__file__.replace("tests/test_host.py",

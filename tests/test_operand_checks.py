@@ -217,6 +217,19 @@ def test_one_row_fp8_linear_in_place_quantises_apart(native):
         native.clear()
 
 
+@pytest.mark.parametrize("rows,N,reads", [(1, 64, True), (64, 60016, True), (256, 12288, True),
+                                          (65, 25008, False), (320, 12000, False)])
+def test_packed_copy_is_asked_for_where_it_is_read(rows, N, reads, native, monkeypatch):
+    from evo2_flash_amd.fp8 import E4M3, Fp8StaticLinear
+    lin = Fp8StaticLinear(128, N, bias=False)
+    copy = torch.zeros(N, 128).to(E4M3)
+    asked = []
+    monkeypatch.setattr(lin, "decode_weight", lambda: (asked.append(1), copy)[1])
+    lin(torch.zeros(rows, 128, dtype=bf))
+    assert bool(asked) == reads
+    assert (_lib.ptr(copy) in native[-1][1]) == reads
+
+
 @pytest.mark.parametrize("M", [4, 33])
 @pytest.mark.parametrize("bias", [False, True])
 def test_linear_adds_a_residual_that_is_its_output(M, bias):
