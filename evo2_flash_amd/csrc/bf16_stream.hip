@@ -22,7 +22,8 @@
 // 24.7 / 29.7 (26.4), 4096 x 11264 18.7 / 20.0 / 26.7 (20.6 / 19.5 / 20.0), 1920 x
 // 1920 4.5 / 5.1 / 5.9 (8.0); gated 2 x 11264 x 4096 34.5 / 37.0 / 42.0 (52.4 and
 // 5 for the multiply).  The rows of X cost as L2 reads, so the plain form takes
-// M > 8 only for small weights (linear.py).  Sixteen k steps ahead 9.3 / 11.9 /
+// M > 8 only for small weights, and fewer than 8 at K > 5120 (linear.py has the
+// rule and its figures).  Sixteen k steps ahead 9.3 / 11.9 /
 // 13.5 at 4096 x 4096, two row groups a workgroup 13 / 15 / 17, sixteen waves 9.1
 // / 10.4 / 12.3, loads of X for the M rows alone 11.0 / 11.8 / 12.8.
 #include <type_traits>

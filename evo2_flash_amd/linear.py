@@ -77,17 +77,39 @@ def library_linear(x, weight, bias: Optional[torch.Tensor], out: Optional[torch.
     return torch.mm(x, weight.t(), out=out)
 
 
+def stream_rows(N, K, residual=False):
+    """The most rows for which the streaming kernel is the faster one of an
+    (N, K) weight.  The library's time hardly depends on the rows; the kernel's
+    grows with rows x K, which every 16 columns' workgroup reads from the L2.
+    Weights from HBM, us against the library's: 4096 x 4096 9.6 at 8 rows and
+    11.6 at 16 against 15.5; 11264 x 4096 24.8 and 30.1 against 26.3; 1920 x 5120
+    10.8 and 14.4 against 18.2 and 10.3; 24576 x 8192 77.2 at 4 and 85.2 at 8
+    against 80.9 and 78.8; 4096 x 11264 19.6 and 20.5 against 20.8 and 19.8, and
+    22.4 against 22.0 where the library's residual takes another launch (8192 x
+    11264 then 40.7 against 37.3); behind it at 1 to 8 rows 6144 x 6144 (20.9 - 23.4
+    against 19), 512 x 8192 from 2 rows (14.2 at 8 against 11.5), 8192 x 22528 from
+    3 (81 at 8 against 71)."""
+    if K <= 5120:
+        return 16 if N * K <= 1 << 24 and K <= 4096 else 8
+    if 8192 <= K <= 11264 and N >= 4096:
+        return 8 if residual and N * K <= 1 << 26 else 4
+    return 0
+
+
+def gated_rows(K):
+    """The most rows for which `gated` streams: 11264 x 4096 46.4 us at 16 against
+    the library's 53.2 in three launches; 22528 x 8192 146.7 at 8 against 149.4,
+    153.3 at 10 against 150.3; 4096 x 16384 behind it from one row (72.5, 61.9)."""
+    return 16 if K <= 5120 else 8 if K <= 11264 else 0
+
+
 def linear(x, weight, bias=None, out=None, residual=None):
     """x @ weight^T [+ bias] [+ residual], each step rounded to x's dtype; with
-    `out` a 2-D x's result is written there.
-
-    The streaming kernel takes at most 8 rows, and up to 16 of a small weight
-    (N K <= 2^24, K <= 4096): there it is the faster one, measured in us against
-    the library at 8 / 16 rows: 4096 x 4096 9.6 / 11.5 against 15.6; 11264 x 4096
-    24.7 / 29.7 against 26.4; 1920 x 5120 11.0 / 14.3 against 18.3 / 10.5."""
+    `out` a 2-D x's result is written there.  Up to stream_rows rows on the
+    streaming kernel."""
     if _streams(x, weight):
         M, (N, K) = x.shape[0], weight.shape
-        if ((M <= 8 or (N * K <= 1 << 24 and K <= 4096))
+        if (M <= stream_rows(N, K, residual is not None)
                 and (bias is None or (_ordinary(bias) and bias.device == x.device
                                       and bias.shape == (N,) and bias.is_contiguous()))
                 and (residual is None or (plain(residual) and residual.shape == (M, N)
@@ -108,8 +130,8 @@ def linear(x, weight, bias=None, out=None, residual=None):
 
 def gated(x, w1, w2, gelu):
     """act(x @ w1^T) * (x @ w2^T), act the exact GELU or the identity, each step
-    rounded to x's dtype (at most 16 rows: one launch)."""
-    if _streams(x, w1, w2):
+    rounded to x's dtype (up to gated_rows rows: one launch)."""
+    if _streams(x, w1, w2) and x.shape[0] <= gated_rows(x.shape[1]):
         M, (N, K) = x.shape[0], w1.shape
         y = torch.empty(M, N, dtype=x.dtype, device=x.device)
         _lib.call("evo2_bf16_stream_gated", _lib.ptr(x), x.stride(0), _lib.ptr(w1), _lib.ptr(w2),

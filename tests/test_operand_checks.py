@@ -434,3 +434,14 @@ def test_linear_compiles_to_torchscript(bias):
     script = torch.jit.script(mod)
     assert script(x, out)[0].data_ptr() == out.data_ptr()
     assert torch.equal(out, mod(x)[0]) and torch.equal(script(x)[0], out)
+
+
+def test_rows_that_stream_by_width():
+    """The widths of the 1B, 7B and 40B models, and those between."""
+    from evo2_flash_amd.linear import gated_rows, stream_rows
+    for N, K, rows, added in ((1920, 1920, 16, 16), (5760, 1920, 16, 16), (1920, 5120, 8, 8),
+                              (4096, 4096, 16, 16), (12288, 4096, 8, 8), (4096, 11264, 4, 8),
+                              (8192, 8192, 4, 8), (24576, 8192, 4, 4), (512, 8192, 0, 0),
+                              (8192, 22528, 0, 0), (6144, 6144, 0, 0)):
+        assert stream_rows(N, K) == rows and stream_rows(N, K, residual=True) == added
+    assert [gated_rows(K) for K in (1920, 4096, 5120, 8192, 11264, 16384)] == [16, 16, 16, 8, 8, 0]
