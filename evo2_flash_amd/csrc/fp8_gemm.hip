@@ -285,13 +285,14 @@ __host__ __device__ inline bool persist_grouped(int ncu, int tiles_n, int tiles_
 }
 
 // Output tile (bn, bm) of the t-th tile in the persistent order, for
-// 0 <= t < tiles_n * tiles_m, with `grid` workgroups; a bijection onto the
-// tile grid.  Where the grid does not split into whole 4 x 8 blocks, the tiles
-// are numbered down panels of four W tiles (row by row inside a panel), and
-// each round hands every XCD one contiguous run of them: 32 tiles of a panel
-// are a 4 x 8 block again.
-__host__ __device__ inline void persist_tile(int t, int tiles_n, int tiles_m, int grid, bool grouped,
-                                             int &bn, int &bm) {
+// 0 <= t < tiles_n * tiles_m; a bijection onto the tile grid.  Where the grid
+// does not split into whole 4 x 8 blocks, row by row: the first rounds stream
+// the whole weight, and a part-filled last one finds it in the caches.  (Panels
+// of four W tiles, a run of 32 for each XCD, left the last round cold weights:
+// K = 8192, N = 24576, 256-row tiles, us, panels / rows: 1024 rows 205 / 160, 1280
+// 210 / 166, 3001 487 / 469; K = 4096, N = 12288: 1000 54 / 44, 3001 154 / 140.)
+__host__ __device__ inline void persist_tile(int t, int tiles_n, int tiles_m, bool grouped, int &bn,
+                                             int &bm) {
   if (grouped) {
     const int nbn = tiles_n >> 2;
     const int whole = ((nbn * (tiles_m >> 3)) >> 3) << 8;  // tiles in whole rounds
@@ -306,14 +307,8 @@ __host__ __device__ inline void persist_tile(int t, int tiles_n, int tiles_m, in
     bn = (blk % nbn) * 4 + (i & 3);
     bm = (blk / nbn) * 8 + (i >> 2);
   } else {
-    const int r0 = t / grid * grid, pos = t - r0;
-    const int left = tiles_n * tiles_m - r0, cnt = left < grid ? left : grid;  // this round's tiles
-    const int x = pos & 7, rest = cnt & 7;
-    const int u = r0 + x * (cnt >> 3) + (x < rest ? x : rest) + (pos >> 3);
-    const int panel = u / (4 * tiles_m), v = u - panel * 4 * tiles_m;
-    const int w = tiles_n - 4 * panel < 4 ? tiles_n - 4 * panel : 4;
-    bm = v / w;
-    bn = 4 * panel + v - bm * w;
+    bn = t % tiles_n;
+    bm = t / tiles_n;
   }
 }
 
@@ -380,7 +375,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
   int tw = 0, tx = 0;  // byte offsets of the wave's first DMA row in the tile being loaded
   auto dma_tile = [&](int j) __attribute__((always_inline)) {
     int bn, bm;
-    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grid, grouped != 0, bn, bm);
+    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grouped != 0, bn, bm);
     tw = (bn * G_BN + DB * 8 * wave) * static_cast<int>(p.sw);
     tx = (bm * BM + DX * 8 * wave) * static_cast<int>(p.sx);
   };
@@ -463,7 +458,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
   auto load_bias = [&](auto par, int j) __attribute__((always_inline)) {
     if (!p.bias || wave != 0) return;  // uniform
     int bn, bm;
-    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grid, grouped != 0, bn, bm);
+    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grouped != 0, bn, bm);
     bf16_t *lb = decltype(par)::value ? bias1 : bias0;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(brs, (lds_void *)lb, 16, 16 * lane_now(), 2 * bn * G_BN,
                                              0, 0);
@@ -476,7 +471,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_persist_kernel(GemmArgs p, int t
   constexpr int EPI_STORES = TM * 4 * 2;
   auto epilogue = [&](int j) __attribute__((always_inline)) {
     int bn, bm;
-    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grid, grouped != 0, bn, bm);
+    persist_tile(static_cast<int>(blockIdx.x) + j * grid, tiles_n, tiles_m, grouped != 0, bn, bm);
     // The order is a bijection onto the grid (checked on the host for every
     // grid up to 64 x 40 tiles); a tile outside it stores nothing rather than
     // past the output (the operand loads are bounded by their descriptors).
@@ -1321,7 +1316,7 @@ extern "C" int64_t evo2_fp8_gemm_persist_order(int64_t tiles_n, int64_t tiles_m,
   if (bn && bm) {
     for (int t = 0; t < total; ++t) {
       int n, m;
-      persist_tile(t, tn, tm, ncu, grouped, n, m);
+      persist_tile(t, tn, tm, grouped, n, m);
       bn[t] = n;
       bm[t] = m;
     }

@@ -551,7 +551,7 @@ int evo2_fp8_gemm_plan(int64_t sx, int64_t sw, int64_t so, int32_t aligned, int6
  * tiles_m tiles with ncu workgroups: tile t, run by workgroup
  * t mod ncu, is output tile (bn[t], bm[t]).  Fills bn / bm (tiles_n * tiles_m
  * entries each, both may be NULL) and returns 1 for the XCD-grouped order,
- * 0 for the panel order, -1 for bad sizes.  Host only, no GPU needed.
+ * 0 for row by row, -1 for bad sizes.  Host only, no GPU needed.
  *
  * No counterpart in the reference (its GEMM is a library call): a planning
  * query for callers and tests that check the tile order covers every tile.

@@ -203,6 +203,19 @@ def test_fp8_persist_order_covers_every_tile():
 
 
 @needs_lib
+def test_fp8_persist_order_row_by_row():
+    """Off whole 4 x 8 blocks the tiles go out row by row, so that every W tile is
+    read in the first rounds."""
+    import numpy as np
+    for tn, tm, ncu in ((96, 4, 256), (48, 3, 144), (23, 24, 256), (48, 13, 256)):
+        bn, bm = (np.empty(tn * tm, dtype=np.int32) for _ in range(2))
+        assert _lib.lib().evo2_fp8_gemm_persist_order(tn, tm, ncu, bn.ctypes.data,
+                                                      bm.ctypes.data) == 0
+        t = np.arange(tn * tm)
+        assert (bn == t % tn).all() and (bm == t // tn).all()
+
+
+@needs_lib
 def test_fp8_tiles_stay_within_buffer_offsets():
     """The persistent GEMM's row offsets are 32-bit and run to the end of the
     last tile of the height it takes: 1000 rows are 1152 in tiles of 192.  Strides

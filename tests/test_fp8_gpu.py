@@ -83,7 +83,7 @@ def test_gemm_known_answer(M, N, K):
 # Persistent kernel on whole tiles: (2048, 8192) is one round of 32 x 8 tiles of
 # 256 rows (the XCD-block order); (2048, 12288) 48 x 16 tiles of 128 rows, three
 # whole rounds of 4 x 8 blocks on the three-stage ring, with K = 256 of two slices
-# a tile; (3328, 5120) 20 x 18 tiles of 192 rows, two rounds in panel order.
+# a tile; (3328, 5120) 20 x 18 tiles of 192 rows, two rounds row by row.
 @pytest.mark.parametrize("M,N,K", [(2048, 8192, 512), (2048, 12288, 512), (3328, 5120, 768),
                                    (2048, 12288, 256)])
 def test_gemm_known_answer_persistent(M, N, K):
