@@ -1087,20 +1087,27 @@ static void launch_persist(const GemmArgs &a, int ncu, hipStream_t st) {
     hipLaunchKernelGGL((fp8_gemm_persist_kernel<TM, false>), dim3(grid), dim3(256), 0, st, a, tiles_n, tiles_m, grouped);
 }
 
-// X rows of a tile (in units of 64) of the persistent kernel: the fewest
-// rounds of tiles over the CUs, weighted by what a round costs, TM + 1.3
-// (rounds measured over 32768 x 12288 x 4096, us: 51.5, 39.5, 31.9, 22.3 for
-// TM 4 .. 1; a single round is bound by its loads' latency and costs a little
-// less).  The larger tile on a tie.  Measured at K = 4096 (1920 for N = 5760,
-// 1920), us for TM 4 / 3 / 2 / 1: 300 x 12288 52.0 / 46.6 / 37.5 / 33.2; 777 x
-// 12288 52.8 / 47.3 / 69.8 / 87.1; 3001 x 12288 163 / 147 / 182 / 265; 6001 x
-// 12288 262 / 265 / 304 / 409; 2047 x 5760 27.7 / 25.5 / 34.7 / 38.0; 2047 x
-// 1920 24.1 / 20.7 / 18.4 / 15.3.
+// X rows of a tile (in units of 64) of the persistent kernel: the least of
+// rounds of tiles over the CUs times what a round costs, TM + 1.3 (rounds
+// measured over 32768 x 12288 x 4096, us: 51.5, 39.5, 31.9, 22.3 for TM 4 .. 1; a
+// single round is bound by its loads' latency and costs a little less).  A
+// part-filled last round counts 0.6 of a whole one and 0.4 of its share: its CUs
+// find the weight in the caches and run faster (256-row tiles of 24576 x 8192:
+// 1.5 rounds 160-180 us, 1.9 166-207, 2.3 245-272, 3 325, 4.5 469; counted whole,
+// the rule took tiles of 128 at 1024 rows, 215).  The larger tile on a tie.  Over
+// 305 sizes from 69 to 8192 rows, N 1920 to 32768, K 1920 to 11264, the choice is
+// within 4% of the best height but at 1500 and 1536 rows of 24576 x 8192 (285
+// against 245-274) and 1536 and 2048 of 16384 x 4096 (102, 127 against 95, 118).
+// Measured, us for TM 4 / 3 / 2 / 1: K = 4096, N = 12288: 777 rows 43.8 / 42.8 /
+// 64.8 / 77.7; 1000 44.2 / 74.7 / 70.0 / 81.8; 3001 140 / 137 / 161 / 211; 6001 245 /
+// 251 / 278 / 397; K = 1920, N = 5760: 2047 25.2 / 22.6 / 33.0 / 35.7.
 static int persist_rows(int64_t tiles_n, int64_t M, int ncu) {
   int best = 4;
   double least = 1e30;
   for (int tm = 4; tm >= 1; --tm) {
-    const double cost = double(cdiv(tiles_n * cdiv(M, 64 * tm), ncu)) * (tm + 1.3);
+    const int64_t tiles = tiles_n * cdiv(M, 64 * tm), last = tiles % ncu;
+    const double rounds = double(tiles / ncu) + (last ? 0.6 + 0.4 * double(last) / ncu : 0.0);
+    const double cost = rounds * (tm + 1.3);
     if (cost < least - 1e-9) {
       least = cost;
       best = tm;

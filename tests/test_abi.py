@@ -216,6 +216,19 @@ def test_fp8_persist_order_row_by_row():
 
 
 @needs_lib
+def test_fp8_tile_heights():
+    """Tile heights where counting a part-filled last round as a whole one took
+    others that measured slower (24576 x 8192, 12288 x 4096, 8192 x 8192), and
+    where one round or whole ones decide."""
+    plan = _lib.lib().evo2_fp8_gemm_plan
+    for M, N, K, tm in ((971, 24576, 8192, 4), (1024, 24576, 8192, 4), (3001, 24576, 8192, 4),
+                        (2048, 12288, 4096, 4), (777, 12288, 4096, 3), (300, 12288, 4096, 1),
+                        (6001, 12288, 4096, 4), (2047, 5760, 1920, 3), (2047, 1920, 1920, 1),
+                        (1000, 8192, 8192, 2), (8192, 12288, 4096, 4)):
+        assert plan(K, K, N, 1, M, N, K, 256) == tm, (M, N, K)
+
+
+@needs_lib
 def test_fp8_tiles_stay_within_buffer_offsets():
     """The persistent GEMM's row offsets are 32-bit and run to the end of the
     last tile of the height it takes: 1000 rows are 1152 in tiles of 192.  Strides

@@ -80,10 +80,11 @@ def test_gemm_known_answer(M, N, K):
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
 
 
-# Persistent kernel on whole tiles: (2048, 8192) is one round of 32 x 8 tiles of
-# 256 rows (the XCD-block order); (2048, 12288) 48 x 16 tiles of 128 rows, three
-# whole rounds of 4 x 8 blocks on the three-stage ring, with K = 256 of two slices
-# a tile; (3328, 5120) 20 x 18 tiles of 192 rows, two rounds row by row.
+# Persistent kernel on whole tiles of 256 rows: (2048, 8192) is one round of 32 x 8
+# (the XCD-block order); (2048, 12288) has 48 x 8, twelve blocks of 4 x 8, so the
+# order's second round is half full, and K = 256 tiles of one slice pair, the one
+# that starts the accumulators; (3328, 5120) 20 x 18 tiles of 192 rows, two rounds
+# row by row.
 @pytest.mark.parametrize("M,N,K", [(2048, 8192, 512), (2048, 12288, 512), (3328, 5120, 768),
                                    (2048, 12288, 256)])
 def test_gemm_known_answer_persistent(M, N, K):
@@ -164,7 +165,7 @@ def test_gemm_known_answer_general(M, N, K, bias):
         assert torch.equal(fp8_gemm(x8, w8, one, one, b), ref)
 
 
-@pytest.mark.parametrize("M,N,K,plan", [(1999, 12280, 384, (2, 3)), (6407, 2552, 640, (2, 2)),
+@pytest.mark.parametrize("M,N,K,plan", [(600, 33016, 384, (2, 3)), (6407, 2552, 640, (2, 2)),
                                         (6140, 5120, 256, (4, 2)), (6140, 5120, 384, (4, 2)),
                                         (3001, 12280, 384, (3, 3))])
 @pytest.mark.parametrize("bias", [False, True])
@@ -202,7 +203,8 @@ def test_gemm_known_answer_few_rows(M, N, K, bias):
 
 @pytest.mark.parametrize("M,N,K", [(8100, 8192, 128), (8100, 8192, 256),       # 256 rows a tile, 4 rounds
                                    (3001, 12288, 640), (3001, 12288, 256),    # 192 rows, 3 rounds
-                                   (1999, 12288, 128), (1999, 12288, 640)])   # 128 rows, 3 rounds
+                                   (1999, 12288, 128), (1999, 12288, 640),    # 256 rows, 2 rounds
+                                   (600, 33016, 128), (600, 33016, 640)])     # 128 rows, 3 rounds
 def test_gemm_known_answer_bias_of_every_tile(M, N, K):
     """Three and more tiles a workgroup, the bias another in each 256-column
     tile: a tile adds its own, whichever buffer it came through (both forms of
