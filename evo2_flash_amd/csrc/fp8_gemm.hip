@@ -892,7 +892,10 @@ __device__ __forceinline__ int4 quantize16(const bf16_t *x, float s) {
 // quantisation launch) / here: 12288 x 4096 at M = 1 15.2 / 11.0 (two launches
 // 11.6), 2 14.6 / 11.7, 8 15.0 / 12.2, 16 15.2 / 14.3; 4096 x 4096 at 1 11.5 / 5.9,
 // 16 12.1 / 7.9; 5760 x 1920 at 1 8.7 / 4.7; 24576 x 8192 at 1 37.5 / 32.7, 8 37.9 /
-// 34.0, 16 36.7 / 40.8: hence 16 rows up to N K = 2^26, 8 above.  The same bits.
+// 34.0, 16 36.7 / 40.8: hence 16 rows up to N K = 2^26, 8 above.  The bits are
+// those of the quantisation and this kernel apart, and the same packed and
+// row-major.  The ring kernel sums K in one chain, so a row's bits can differ across
+// the row count where the kernels change (they agree where the sums are exact).
 constexpr int F_ROWS = 16;    // X rows
 constexpr int F_WAVES = 8;    // waves per workgroup: parts of K
 constexpr int F_QMAXK = 16384;
@@ -996,12 +999,13 @@ __global__ __launch_bounds__(256) void fp8_pack_kernel(const uint8_t *w, int64_t
 // streaming from HBM (K = 4096, us, stream / tiles): M=65, N=4096 11.5 / 24.1;
 // M=300, N=4096 22.9 / 23.7; M=777, N=4096 53.7 / 24.9; N=12288: M=65 26.1 /
 // 31.6, M=128 28.2 / 33.8, M=200 44.1 / 31.7, M=300 51.3 / 32.9; K=1920,
-// N=5760: M=130 14.0 / 14.0, M=600 31.8 / 15.2.  Streaming takes
-// ceil(M / 64) x N up to TILE_MIN_WORK (the tiles are the faster from ~30000;
-// verify-sized steps, M <= 256 at N = 12288, keep the streaming kernels' sums,
-// the same bits with a packed weight and without), and up to STREAM_MAX_WORK where the
-// persistent kernel does not apply (against the 256 x 256 tile kernel: M=256,
-// N=12288 42 / 62; M=512, N=4096 25 / 41); M <= 64 always streams.
+// N=5760: M=130 14.0 / 14.0, M=600 31.8 / 15.2.  So the tiles are the faster from
+// some 17000 to 37000 of ceil(M / 64) x N, by N and K, which this product alone does
+// not tell apart.  The line is where it was drawn before the tiles took ragged
+// rows, past 4 x 12288 (64-request verify steps stream, packed or not): it leaves
+// up to twice the tiles' time below it (N = 4096 at 768 rows).  STREAM_MAX_WORK is
+// the line where the persistent kernel does not apply (against the 256 x 256 tile
+// kernel: M=256, N=12288 42 / 62; M=512, N=4096 25 / 41); M <= 64 always streams.
 #define TILE_MIN_WORK 50000
 #ifndef STREAM_MAX_WORK
 #define STREAM_MAX_WORK 60000

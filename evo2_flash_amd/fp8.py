@@ -63,7 +63,7 @@ def fp8_gemm(x8, w8, x_scale, w_scale, bias=None, out=None):
 
 
 STREAM_MAX_WORK = 60000  # evo2_fp8_gemm may stream the weight while ceil(M / 64) * N <= this
-TILE_MIN_WORK = 50000    # and above this prefers its persistent tile kernel (M > 64)
+TILE_MIN_WORK = 50000    # and above this takes its persistent tile kernel (M > 64)
 
 
 def streams_weight(M, N):
