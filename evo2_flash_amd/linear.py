@@ -13,6 +13,7 @@ from torch.utils._device import DeviceContext
 from . import _lib
 
 STREAM_ROWS = 16  # the kernel's most rows
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
 def _eager():
@@ -31,7 +32,7 @@ def _eager():
 def _ordinary(t):
     """Whether t is an ordinary dense CUDA bf16 tensor: no subclass or proxy, outside
     vmap, without a gradient to record."""
-    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
+    return (type(t) in _TENSORS and t.is_cuda
             and t.layout == torch.strided and t.dtype == torch.bfloat16
             and not (t.requires_grad and torch.is_grad_enabled())
             and not torch._C._functorch.is_functorch_wrapped_tensor(t))
@@ -52,15 +53,18 @@ def plain(*tensors):
 
 def _streams(x, *weights):
     """Whether the weight-streaming kernel takes x (M, K) against weights (N, K)."""
-    # `plain` before a shape is compared: to a tracer each comparison is a
-    # condition on the rows.  (x on the current device: a launch goes there, and the
-    # default stream's handle is the same on every device; the library's product
-    # switches over)
-    return (plain(x, *weights) and 0 < x.shape[0] <= STREAM_ROWS and x.shape[1] % 32 == 0
-            and x.shape[1] > 0 and all(w.shape == weights[0].shape and w.shape[0] > 0
-                                       and w.shape[1] == x.shape[1]
-                                       and w.stride() == weights[0].stride()
-                                       and w.device == x.device for w in weights)
+    # what traces comes before a shape is compared: to a tracer each comparison is
+    # a condition on the rows.  (Most rows go to the library: their count comes
+    # next.)
+    if (type(x) not in _TENSORS or torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or x.dim() != 2 or not 0 < x.shape[0] <= STREAM_ROWS):
+        return False
+    # (x on the current device: a launch goes there, and the default stream's
+    # handle is the same on every device; the library's product switches over)
+    return (plain(x, *weights) and x.shape[1] % 32 == 0 and x.shape[1] > 0
+            and all(w.shape == weights[0].shape and w.shape[0] > 0
+                    and w.shape[1] == x.shape[1] and w.stride() == weights[0].stride()
+                    and w.device == x.device for w in weights)
             and x.get_device() == torch.cuda.current_device())
 
 
