@@ -25,8 +25,13 @@
 //    operand is the lane's own probabilities of those keys as bf16.
 // Online softmax in fp32 with exp2 of scores kept in log2 units; a row's
 // reference max moves (and its sums are rescaled) only when a half's max
-// exceeds it by more than AP_SLACK, so the probabilities stay below
-// 2^AP_SLACK and most halves rescale nothing.  The probabilities enter the
+// exceeds it by more than the slack, so the probabilities stay below 2^slack.
+// At lengths in eights the slack is AP_SLACK and most halves rescale nothing; at
+// others it is 0, so that the largest probability is exactly 1, as in the fused
+// torch kernel that took those lengths before: relative error against 64 bits
+// at 3001 keys, scores of deviation 3, 0.00176 (torch 0.00176; with AP_SLACK
+// 0.00193), of deviation 1 0.00202 (0.00204; 0.00208); 127 us for 32 heads (torch
+// 319; with AP_SLACK 121).  The probabilities enter the
 // value product rounded to bf16, as in flash attention, and the row sums are
 // the same bf16 probabilities summed by one more product (an all-ones
 // operand), so numerator and denominator use the same values.  LDS rows are
@@ -44,7 +49,7 @@ constexpr int AP_QW = 16 * AP_NQT;         // queries per wave
 constexpr int AP_QB = AP_NW * AP_QW;       // queries per workgroup
 constexpr int AP_KB = 128;                 // keys per block
 constexpr int AP_TILE = AP_KB * AP_HD;     // bf16 per staged operand block (32 KB)
-constexpr float AP_SLACK = 8.0f;           // log2 headroom of the reference max
+constexpr float AP_SLACK = 8.0f;           // log2 headroom of the reference max, L a multiple of 8
 
 struct PrefillArgs {
   const bf16_t *q, *k, *vt;
@@ -56,6 +61,7 @@ struct PrefillArgs {
   int heads;
   int nqb;         // query blocks per plane
   float c2;        // scale * log2(e)
+  float slack;     // log2 headroom of the reference max
   int xcd_heads;   // 1-D grid, whole heads per XCD (heads a multiple of 8)
 };
 
@@ -205,7 +211,7 @@ __global__ __launch_bounds__(AP_NW * 64, 1) void attn_prefill_kernel(PrefillArgs
         bm *= p.c2;
         // the reference max moves only past the slack (from -inf: at the
         // first live score)
-        const bool move = bm > mrun[nt] + AP_SLACK;
+        const bool move = bm > mrun[nt] + p.slack;
         const float mn = move ? bm : mrun[nt];
         const float msub = mn == -INFINITY ? 0.0f : mn;  // all masked so far: every exp2 is 0
 #pragma unroll
@@ -315,7 +321,8 @@ extern "C" int evo2_prefill_attention_rows(const void *q, const void *k, const v
                 (long long)Lv);
   PrefillArgs a{static_cast<const bf16_t *>(q), static_cast<const bf16_t *>(k), static_cast<const bf16_t *>(vt),
                 static_cast<bf16_t *>(out), on, oh, ol, L * AP_HD, static_cast<int>(L), static_cast<int>(Lv),
-                static_cast<int>(heads), static_cast<int>(cdiv(L, AP_QB)), scale * 1.4426950408889634f, 0};
+                static_cast<int>(heads), static_cast<int>(cdiv(L, AP_QB)), scale * 1.4426950408889634f,
+                L % 8 ? 0.0f : AP_SLACK, 0};
   // whole heads per XCD where the heads split evenly over the eight (32
   // heads x 32768: 9.96 -> 8.34 ms, 8192: 1.05 -> 0.70 ms, the same bits)
   a.xcd_heads = heads % 8 == 0 && static_cast<int64_t>(a.nqb) * heads <= 0x7fffffff;
